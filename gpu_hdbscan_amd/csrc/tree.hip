@@ -13,10 +13,14 @@
 //    queries of edges whose index has bit b set move from the start of
 //    their segment to its middle -- the edges of the segment's first half
 //    join the components they touch (connected components over component
-//    representatives, one union-find on the GPU per level), and a query
-//    whose component is among them takes the merged component's
-//    representative, its last edge (the node that roots it) and its point
-//    count.  log2(m) levels of sorts, scans and hooking.
+//    names, one union-find on the GPU per level), and a query whose
+//    component is among them takes the merged component, its last edge (the
+//    node that roots it) and its point count.  Three launches per level down
+//    to segments of 1024 edges, which finish their levels in LDS.  Bound by
+//    the random reads of the top levels.  Replaced one radix sort of all
+//    queries by (segment, component) per level, which cost 45 launches and
+//    4-6 passes over them each; path and labels together 6.94 -> 3.71 ms at
+//    5k x 12, 12.9 -> 8.4 ms at 100k and 531 -> 491 ms at 10M.
 // 2. The condensed tree (build_Condensed_tree, tree.cu:255-442) follows from
 //    the linkage tree without a traversal: a node is processed when it is
 //    the root or holds at least mpts points; a processed node whose two
@@ -45,65 +49,15 @@ namespace {
 constexpr int kRepBits = 26;  // n < 2^26
 
 // ---------------------------------------------------------------- linkage --
-__global__ void k_lk_init(const hdb_mst_edge* __restrict__ e, int64_t m, int32_t* __restrict__ rep,
-                          int32_t* __restrict__ top, int32_t* __restrict__ sz) {
-  const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (q >= 2 * m) return;
-  const hdb_mst_edge x = e[q >> 1];
-  const int32_t v = (q & 1) ? x.to_node : x.from_node;
-  rep[q] = v;
-  top[q] = v;
-  sz[q] = 1;
-}
-
-// Key of query q at bit b: (segment, representative, second-half flag).
-__global__ void k_lk_keys(int64_t m, int b, const int32_t* __restrict__ rep, uint64_t* __restrict__ keys,
-                          uint32_t* __restrict__ vals) {
-  const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (q >= 2 * m) return;
-  const int64_t i = q >> 1;
-  const uint64_t seg = static_cast<uint64_t>(i >> (b + 1));
-  const uint64_t right = static_cast<uint64_t>((i >> b) & 1);
-  keys[q] = (seg << (kRepBits + 1)) | (static_cast<uint64_t>(static_cast<uint32_t>(rep[q])) << 1) | right;
-  vals[q] = static_cast<uint32_t>(q);
-}
-
-// fg: first of a (segment, representative) group; fl: first of a group
-// that holds a first-half query (those sort before the group's others).
-__global__ void k_lk_flags(const uint64_t* __restrict__ K, int64_t Q, int32_t* __restrict__ fg,
-                           int32_t* __restrict__ fl) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= Q) return;
-  const bool start = t == 0 || (K[t] >> 1) != (K[t - 1] >> 1);
-  fg[t] = start ? 1 : 0;
-  fl[t] = (start && !(K[t] & 1)) ? 1 : 0;
-}
-
-// Left group g (a vertex of this level's union-find): its group index and
-// sorted position.
-__global__ void k_lk_groups(const int32_t* __restrict__ fl, const int64_t* __restrict__ eg,
-                            const int64_t* __restrict__ el, int64_t Q, int64_t* __restrict__ lg_group,
-                            int64_t* __restrict__ lg_pos, int32_t* __restrict__ uf) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= Q || !fl[t]) return;
-  const int64_t g = el[t];
-  lg_group[g] = eg[t];
-  lg_pos[g] = t;
-  uf[g] = static_cast<int32_t>(g);
-}
-
-// vid[q]: the union-find vertex of query q's group, -1 when the group has no
-// first-half query (its component gets no edge at this level).
-__global__ void k_lk_vid(const uint32_t* __restrict__ V, const int32_t* __restrict__ fg,
-                         const int32_t* __restrict__ fl, const int64_t* __restrict__ eg,
-                         const int64_t* __restrict__ el, const int64_t* __restrict__ lg_group, int64_t Q,
-                         int32_t* __restrict__ vid) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= Q) return;
-  const int64_t s1 = el[t] + fl[t], s2 = eg[t] + fg[t];
-  const bool has_left = s1 > 0 && lg_group[s1 - 1] == s2 - 1;
-  vid[V[t]] = has_left ? static_cast<int32_t>(s1 - 1) : -1;
-}
+// A component of a segment is named by its lowest end: the smallest query q
+// (end q & 1 of edge q >> 1) of the segment that lies in it.  Names of a
+// segment therefore fall in its own index range, so every per-component
+// array is read near the segment's own positions once segments are small,
+// and no sort, scan or count of components is needed.  top and sz hold, at
+// a component's name, the node that roots it and its point count.
+constexpr int kLkBits = 10;             // segments of 1024 edges are finished in LDS
+constexpr int kLkEdges = 1 << kLkBits;  // one per thread of k_lk_local
+constexpr int32_t kNoName = INT_MAX;
 
 // Entries of the union-find are read and written with device-scope
 // atomics: the union kernel's blocks run on every XCD, each behind its own
@@ -129,59 +83,85 @@ __device__ __forceinline__ int32_t uf_find(int32_t* uf, int32_t x) {
   return cur;
 }
 
-// Root of x without writes: in k_lk_compress every vertex stores its own
-// root, and a halving write by another thread could land after that store
-// and leave a non-root ancestor there.
-__device__ __forceinline__ int32_t uf_root(const int32_t* uf, int32_t x) {
-  int32_t cur = x, next;
-  while ((next = uf_load(uf, cur)) != cur) cur = next;
-  return cur;
-}
-
-// First-half edges of every segment join their ends' components: the
-// larger root is hooked under the smaller with a compare-and-swap.
-__global__ void k_lk_union(int64_t m, int b, const int32_t* __restrict__ vid, int32_t* __restrict__ uf) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= m || ((i >> b) & 1)) return;
-  int32_t a = vid[2 * i], c = vid[2 * i + 1];
+// The larger root is hooked under the smaller with a compare-and-swap.
+__device__ __forceinline__ void uf_join(int32_t* uf, int32_t a, int32_t c) {
   while (true) {
     a = uf_find(uf, a);
     c = uf_find(uf, c);
-    if (a == c) break;
+    if (a == c) return;
     if (a > c) {
       const int32_t t = a;
       a = c;
       c = t;
     }
-    if (atomicCAS(&uf[c], c, a) == c) break;
+    if (atomicCAS(&uf[c], c, a) == c) return;
   }
 }
 
-__global__ void k_lk_compress(int64_t V, int32_t* __restrict__ uf, int32_t* __restrict__ cmax,
-                              int32_t* __restrict__ csize) {
-  const int64_t v = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (v >= V) return;
-  uf[v] = uf_root(uf, static_cast<int32_t>(v));
-  cmax[v] = -1;
-  csize[v] = 0;
+// *p = min(*p, v), skipping the atomic when *p (which only falls, so a stale
+// read only costs an atomic) is already there: the members of a component
+// arrive roughly in ascending order, so a large one takes few atomics.
+__device__ __forceinline__ void lower_to(int32_t* p, int32_t v) {
+  if (v < uf_load(p, 0)) atomicMin(p, v);
 }
 
-// Per component: its last (highest) first-half edge and its point count.
-// A few huge components take most of the updates at the top levels, so a
-// block first combines its updates in an LDS table keyed by component root
-// (linear probing, four slots) and sends one global atomic per root it saw;
-// a root that finds no slot goes to the global atomic directly.  Max and
-// integer sums do not depend on the order.
+// The union-find and the per-component accumulators of one level: names of
+// the two halves' components, last first-half edge, point count.
+struct LkLevel {
+  int32_t *uf, *rep_l, *rep_r, *cmax, *csize;
+};
+
+__device__ __forceinline__ void lk_reset(const LkLevel& a, int64_t q) {
+  a.uf[q] = static_cast<int32_t>(q);
+  a.rep_l[q] = kNoName;
+  a.rep_r[q] = kNoName;
+  a.cmax[q] = -1;
+  a.csize[q] = 0;
+}
+
+// first[v] = the lowest end at point v, through the level's rep_l (2m >= n
+// entries for m >= 1); an end outside [0, n) marks the input bad.
+__global__ void k_lk_first(const hdb_mst_edge* __restrict__ e, int64_t m, int64_t n, int32_t* __restrict__ first,
+                           int32_t* __restrict__ bad) {
+  const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (q >= 2 * m) return;
+  const int32_t v = (q & 1) ? e[q >> 1].to_node : e[q >> 1].from_node;
+  if (v < 0 || v >= n) *bad = 1;
+  else lower_to(first + v, static_cast<int32_t>(q));
+}
+
+__global__ void k_lk_init(const hdb_mst_edge* __restrict__ e, int64_t m, int64_t n, const int32_t* __restrict__ first,
+                          int32_t* __restrict__ vid, int32_t* __restrict__ top, int32_t* __restrict__ sz, LkLevel a) {
+  const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (q >= 2 * m) return;
+  const int32_t v = (q & 1) ? e[q >> 1].to_node : e[q >> 1].from_node;
+  vid[q] = v >= 0 && v < n ? first[v] : static_cast<int32_t>(q);
+  top[q] = v;
+  sz[q] = 1;
+  lk_reset(a, q);
+}
+
+// Level b, first kernel: the first-half edges (bit b clear) of every segment
+// join their ends' components, and the components they touch get their name
+// in the first half.
+__global__ void k_lk_union(int64_t m, int b, const int32_t* __restrict__ vid, LkLevel a) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= m || ((i >> b) & 1)) return;
+  const int32_t v0 = vid[2 * i], v1 = vid[2 * i + 1];
+  lower_to(a.rep_l + v0, static_cast<int32_t>(2 * i));
+  lower_to(a.rep_l + v1, static_cast<int32_t>(2 * i + 1));
+  uf_join(a.uf, v0, v1);
+}
+
+// Per merged component: its last (highest) first-half edge, its point count
+// (each component a first-half edge touches counts once, at its name) and
+// its name in the second half.  A few huge components take most of the
+// updates at the top levels, so a block combines maxima and sums in two LDS
+// tables keyed by component root (linear probing, four slots) and sends one
+// global atomic per root it saw; a root that finds no slot goes to the
+// global atomic directly.  Max, min and integer sums do not depend on the
+// order.
 constexpr int kAggSlots = 1024;
-constexpr int kAggItems = 16;  // entries per thread
-
-template <bool MAX>
-__device__ __forceinline__ void agg_init(int32_t* keys, int32_t* acc) {
-  for (int s = threadIdx.x; s < kAggSlots; s += blockDim.x) {
-    keys[s] = -1;
-    acc[s] = MAX ? -1 : 0;
-  }
-}
 
 template <bool MAX>
 __device__ __forceinline__ void agg_put(int32_t* keys, int32_t* acc, int32_t* glob, int32_t root, int32_t v) {
@@ -201,59 +181,144 @@ __device__ __forceinline__ void agg_put(int32_t* keys, int32_t* acc, int32_t* gl
   else atomicAdd(&glob[root], v);
 }
 
-template <bool MAX>
-__device__ __forceinline__ void agg_flush(const int32_t* keys, const int32_t* acc, int32_t* glob) {
-  for (int s = threadIdx.x; s < kAggSlots; s += blockDim.x) {
-    const int32_t k = keys[s];
-    if (k < 0) continue;
-    if (MAX) atomicMax(&glob[k], acc[s]);
-    else atomicAdd(&glob[k], acc[s]);
+// `items` edges per thread.
+__global__ __launch_bounds__(256) void k_lk_merge(int64_t m, int b, int items, int32_t* __restrict__ vid,
+                                                  const int32_t* __restrict__ sz, LkLevel a) {
+  __shared__ int32_t kmax[kAggSlots], vmax[kAggSlots], ksum[kAggSlots], vsum[kAggSlots];
+  for (int s = threadIdx.x; s < kAggSlots; s += 256) {
+    kmax[s] = ksum[s] = vmax[s] = -1;
+    vsum[s] = 0;
   }
-}
-
-__global__ __launch_bounds__(256) void k_lk_stats(int64_t m, int b, const int32_t* __restrict__ vid,
-                                                  const int32_t* __restrict__ uf, int32_t* __restrict__ cmax) {
-  __shared__ int32_t keys[kAggSlots], acc[kAggSlots];
-  agg_init<true>(keys, acc);
   __syncthreads();
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * (256 * kAggItems);
-  for (int k = 0; k < kAggItems; ++k) {
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * (256 * items);
+  for (int k = 0; k < items; ++k) {
     const int64_t i = base + k * 256 + threadIdx.x;
-    if (i < m && !((i >> b) & 1)) agg_put<true>(keys, acc, cmax, uf[vid[2 * i]], static_cast<int32_t>(i));
+    if (i >= m) break;
+    const int32_t v0 = vid[2 * i], v1 = vid[2 * i + 1];
+    const int32_t r0 = uf_find(a.uf, v0);
+    const int32_t q0 = static_cast<int32_t>(2 * i);
+    if (!((i >> b) & 1)) {
+      agg_put<true>(kmax, vmax, a.cmax, r0, static_cast<int32_t>(i));
+      const int32_t s = (a.rep_l[v0] == q0 ? sz[v0] : 0) + (a.rep_l[v1] == q0 + 1 ? sz[v1] : 0);
+      if (s) agg_put<false>(ksum, vsum, a.csize, r0, s);
+    } else {
+      const int32_t r1 = uf_find(a.uf, v1);
+      vid[2 * i] = r0;
+      vid[2 * i + 1] = r1;
+      lower_to(a.rep_r + r0, q0);
+      lower_to(a.rep_r + r1, q0 + 1);
+    }
   }
   __syncthreads();
-  agg_flush<true>(keys, acc, cmax);
-}
-
-__global__ __launch_bounds__(256) void k_lk_sizes(int64_t V, const int64_t* __restrict__ lg_pos,
-                                                  const uint32_t* __restrict__ vals, const int32_t* __restrict__ sz,
-                                                  const int32_t* __restrict__ uf, int32_t* __restrict__ csize) {
-  __shared__ int32_t keys[kAggSlots], acc[kAggSlots];
-  agg_init<false>(keys, acc);
-  __syncthreads();
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * (256 * kAggItems);
-  for (int k = 0; k < kAggItems; ++k) {
-    const int64_t g = base + k * 256 + threadIdx.x;
-    if (g < V) agg_put<false>(keys, acc, csize, uf[g], sz[vals[lg_pos[g]]]);
+  for (int s = threadIdx.x; s < kAggSlots; s += 256) {
+    if (kmax[s] >= 0) atomicMax(&a.cmax[kmax[s]], vmax[s]);
+    if (ksum[s] >= 0) atomicAdd(&a.csize[ksum[s]], vsum[s]);
   }
-  __syncthreads();
-  agg_flush<false>(keys, acc, csize);
 }
 
-// Second-half queries whose component grew take the merged component.
-__global__ void k_lk_update(int64_t m, int b, int64_t n, const int32_t* __restrict__ vid,
-                            const int32_t* __restrict__ uf, const int32_t* __restrict__ cmax,
-                            const int32_t* __restrict__ csize, const int64_t* __restrict__ lg_pos,
-                            const uint64_t* __restrict__ K, int32_t* __restrict__ rep, int32_t* __restrict__ top,
-                            int32_t* __restrict__ sz) {
+// Every end takes its component's name in its half, and the component's
+// named end its root node and point count: unchanged in the first half and
+// for a component no first-half edge touched, else the last first-half
+// edge's node and the merged count.  The next level's arrays are reset.
+__global__ void k_lk_rename(int64_t m, int b, int64_t n, int32_t* __restrict__ vid, const int32_t* __restrict__ top,
+                            const int32_t* __restrict__ sz, int32_t* __restrict__ top2, int32_t* __restrict__ sz2,
+                            LkLevel a, LkLevel next) {
   const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (q >= 2 * m || !(((q >> 1) >> b) & 1)) return;
+  if (q >= 2 * m) return;
   const int32_t v = vid[q];
-  if (v < 0) return;
-  const int32_t r = uf[v];
-  rep[q] = static_cast<int32_t>((K[lg_pos[r]] >> 1) & ((1ull << kRepBits) - 1));
-  top[q] = static_cast<int32_t>(n + cmax[r]);
-  sz[q] = csize[r];
+  const bool second = ((q >> (b + 1)) & 1) != 0;
+  const int32_t nv = second ? a.rep_r[v] : a.rep_l[v];
+  vid[q] = nv;
+  if (nv == static_cast<int32_t>(q)) {
+    const int32_t last = second ? a.cmax[v] : -1;
+    top2[q] = last >= 0 ? static_cast<int32_t>(n + last) : top[v];
+    sz2[q] = last >= 0 ? a.csize[v] : sz[v];
+  }
+  lk_reset(next, q);
+}
+
+// The remaining levels of one segment of up to 1024 edges in LDS (56 KB, two
+// blocks per CU), the same three steps per level between block barriers; one
+// edge per thread.  Doing the last ten levels here is what keeps the
+// linkage at 3 launches and one pass over the edges per remaining level: at
+// 5k points three levels are left.  Writes top and sz of each end itself.
+__global__ __launch_bounds__(kLkEdges) void k_lk_local(int64_t m, int levels, int64_t n,
+                                                       const int32_t* __restrict__ vid,
+                                                       const int32_t* __restrict__ top,
+                                                       const int32_t* __restrict__ sz, int32_t* __restrict__ top_end,
+                                                       int32_t* __restrict__ sz_end) {
+  constexpr int Q = 2 * kLkEdges;
+  __shared__ int32_t uf[Q], rep_l[Q], rep_r[Q], cmax[Q], csize[Q], s_top[Q], s_sz[Q];
+  const int t = static_cast<int>(threadIdx.x);
+  const int64_t i0 = static_cast<int64_t>(blockIdx.x) << kLkBits, q0 = 2 * i0;
+  const bool live = i0 + t < m;
+  int32_t v[2] = {0, 0};
+  for (int k = 0; k < 2; ++k) {
+    const int64_t q = q0 + 2 * t + k;
+    if (live) {
+      v[k] = static_cast<int32_t>(vid[q] - q0);
+      s_top[2 * t + k] = top[q];
+      s_sz[2 * t + k] = sz[q];
+    }
+  }
+  for (int b = levels - 1; b >= 0; --b) {
+    for (int x = t; x < Q; x += kLkEdges) {
+      uf[x] = x;
+      rep_l[x] = rep_r[x] = kNoName;
+      cmax[x] = -1;
+      csize[x] = 0;
+    }
+    __syncthreads();
+    const bool second = ((t >> b) & 1) != 0;
+    if (live && !second) {
+      atomicMin(&rep_l[v[0]], 2 * t);
+      atomicMin(&rep_l[v[1]], 2 * t + 1);
+      uf_join(uf, v[0], v[1]);
+    }
+    __syncthreads();
+    if (live) {
+      const int32_t r = uf_find(uf, v[0]);
+      if (!second) {
+        atomicMax(&cmax[r], t);
+        const int32_t s = (rep_l[v[0]] == 2 * t ? s_sz[v[0]] : 0) + (rep_l[v[1]] == 2 * t + 1 ? s_sz[v[1]] : 0);
+        if (s) atomicAdd(&csize[r], s);
+      } else {
+        v[0] = r;
+        v[1] = uf_find(uf, v[1]);
+        atomicMin(&rep_r[v[0]], 2 * t);
+        atomicMin(&rep_r[v[1]], 2 * t + 1);
+      }
+    }
+    __syncthreads();
+    int32_t nt[2] = {0, 0}, ns[2] = {0, 0};
+    bool mine[2] = {false, false};
+    if (live) {
+      for (int k = 0; k < 2; ++k) {
+        const int32_t x = v[k];
+        const int32_t nv = second ? rep_r[x] : rep_l[x];
+        mine[k] = nv == 2 * t + k;
+        if (mine[k]) {
+          const int32_t last = second ? cmax[x] : -1;
+          nt[k] = last >= 0 ? static_cast<int32_t>(n + i0 + last) : s_top[x];
+          ns[k] = last >= 0 ? csize[x] : s_sz[x];
+        }
+        v[k] = nv;
+      }
+    }
+    __syncthreads();
+    for (int k = 0; k < 2; ++k)
+      if (mine[k]) {
+        s_top[2 * t + k] = nt[k];
+        s_sz[2 * t + k] = ns[k];
+      }
+    __syncthreads();
+  }
+  __syncthreads();
+  if (live)
+    for (int k = 0; k < 2; ++k) {
+      top_end[q0 + 2 * t + k] = s_top[v[k]];
+      sz_end[q0 + 2 * t + k] = s_sz[v[k]];
+    }
 }
 
 // ------------------------------------------------------- condensed tree --
@@ -563,61 +628,46 @@ int labels_gpu(hdb_ctx* ctx, const hdb_mst_edge* edges, int64_t m, int64_t n, in
   }
   const int64_t Q = 2 * m;
   // ---- linkage
-  int32_t *rep, *top, *sz, *fg, *fl, *vid, *uf, *cmax, *csize;
-  int64_t *eg, *el, *lg_group, *lg_pos;
-  uint64_t* keys;
-  uint32_t* vals;
-  HDB_CALL(scratch_t(ctx, kSlotMisc0, 3 * Q, &rep));
-  top = rep + Q;
+  int32_t *vid, *top, *sz, *top2, *sz2, *lv, *bad0;
+  HDB_CALL(scratch_t(ctx, kSlotMisc0, 5 * Q, &vid));
+  top = vid + Q;
   sz = top + Q;
-  HDB_CALL(scratch_t(ctx, kSlotRowCnt, 3 * Q, &fg));
-  fl = fg + Q;
-  vid = fl + Q;
-  HDB_CALL(scratch_t(ctx, kSlotRowTmp, 2 * (Q + 1), &eg));
-  el = eg + (Q + 1);
-  HDB_CALL(scratch_t(ctx, kSlotRowUniq, 2 * Q, &lg_group));
-  lg_pos = lg_group + Q;
-  HDB_CALL(scratch_t(ctx, kSlotMisc1, 3 * Q, &uf));
-  cmax = uf + Q;
-  csize = cmax + Q;
-  HDB_CALL(scratch_t(ctx, kSlotRowCursor, Q, &keys));
-  HDB_CALL(scratch_t(ctx, kSlotMisc2, Q, &vals));
-  hipLaunchKernelGGL(k_lk_init, dim3(grid_for(Q, 256)), dim3(256), 0, ctx->stream, edges, m, rep, top, sz);
+  top2 = sz + Q;
+  sz2 = top2 + Q;
+  HDB_CALL(scratch_t(ctx, kSlotMisc1, 10 * Q + 1, &lv));
+  LkLevel cur{lv, lv + Q, lv + 2 * Q, lv + 3 * Q, lv + 4 * Q};
+  LkLevel alt{lv + 5 * Q, lv + 6 * Q, lv + 7 * Q, lv + 8 * Q, lv + 9 * Q};
+  bad0 = lv + 10 * Q;
+  const unsigned gq = grid_for(Q, 256), gm = grid_for(m, 256);
+  // the lowest end of every point, in an array the first level resets later
+  HDB_CALL(fill_i32(ctx, alt.rep_l, Q, kNoName));  // Q >= n for m = n - 1 >= 1
+  HDB_CALL(fill_i32(ctx, bad0, 1, 0));
+  hipLaunchKernelGGL(k_lk_first, dim3(gq), dim3(256), 0, ctx->stream, edges, m, n, alt.rep_l, bad0);
+  HDB_LAUNCHED();
+  hipLaunchKernelGGL(k_lk_init, dim3(gq), dim3(256), 0, ctx->stream, edges, m, n, alt.rep_l, vid, top, sz, cur);
   HDB_LAUNCHED();
   const int L = bits_for(m - 1);
-  for (int b = L - 1; b >= 0; --b) {
-    hipLaunchKernelGGL(k_lk_keys, dim3(grid_for(Q, 256)), dim3(256), 0, ctx->stream, m, b, rep, keys, vals);
+  // edges per thread of k_lk_merge: blocks of 4096 edges where they fill the
+  // chip, fewer where that would leave it idle
+  const int items = static_cast<int>(std::min<int64_t>(16, std::max<int64_t>(1, m / (256 * 1024))));
+  for (int b = L - 1; b >= kLkBits; --b) {
+    hipLaunchKernelGGL(k_lk_union, dim3(gm), dim3(256), 0, ctx->stream, m, b, vid, cur);
     HDB_LAUNCHED();
-    const int seg_bits = bits_for((m - 1) >> (b + 1));
-    HDB_CALL(radix_sort_u64_u32(ctx, keys, vals, Q, 0, kRepBits + 1 + seg_bits));
-    hipLaunchKernelGGL(k_lk_flags, dim3(grid_for(Q, 256)), dim3(256), 0, ctx->stream, keys, Q, fg, fl);
+    hipLaunchKernelGGL(k_lk_merge, dim3(grid_for(m, 256 * items)), dim3(256), 0, ctx->stream, m, b, items, vid, sz,
+                       cur);
     HDB_LAUNCHED();
-    HDB_CALL(scan_i32_to_i64(ctx, fg, Q, eg));
-    HDB_CALL(scan_i32_to_i64(ctx, fl, Q, el));
-    int64_t V = 0;
-    HDB_CALL(read_i64(ctx, el + Q, &V));
-    hipLaunchKernelGGL(k_lk_groups, dim3(grid_for(Q, 256)), dim3(256), 0, ctx->stream, fl, eg, el, Q, lg_group, lg_pos,
-                       uf);
+    hipLaunchKernelGGL(k_lk_rename, dim3(gq), dim3(256), 0, ctx->stream, m, b, n, vid, top, sz, top2, sz2, cur, alt);
     HDB_LAUNCHED();
-    hipLaunchKernelGGL(k_lk_vid, dim3(grid_for(Q, 256)), dim3(256), 0, ctx->stream, vals, fg, fl, eg, el, lg_group, Q,
-                       vid);
-    HDB_LAUNCHED();
-    hipLaunchKernelGGL(k_lk_union, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, m, b, vid, uf);
-    HDB_LAUNCHED();
-    hipLaunchKernelGGL(k_lk_compress, dim3(grid_for(V, 256)), dim3(256), 0, ctx->stream, V, uf, cmax, csize);
-    HDB_LAUNCHED();
-    hipLaunchKernelGGL(k_lk_stats, dim3(grid_for(m, 256 * kAggItems)), dim3(256), 0, ctx->stream, m, b, vid, uf,
-                       cmax);
-    HDB_LAUNCHED();
-    hipLaunchKernelGGL(k_lk_sizes, dim3(grid_for(V, 256 * kAggItems)), dim3(256), 0, ctx->stream, V, lg_pos, vals, sz,
-                       uf, csize);
-    HDB_LAUNCHED();
-    hipLaunchKernelGGL(k_lk_update, dim3(grid_for(Q, 256)), dim3(256), 0, ctx->stream, m, b, n, vid, uf, cmax, csize,
-                       lg_pos, keys, rep, top, sz);
-    HDB_LAUNCHED();
+    std::swap(cur, alt);
+    std::swap(top, top2);
+    std::swap(sz, sz2);
   }
-  // ---- linkage tree and node classes (reusing the linkage scratch that
-  // is dead by now: fg/fl/vid, eg/el, lg_group/lg_pos, uf/cmax/csize)
+  hipLaunchKernelGGL(k_lk_local, dim3(grid_for(m, kLkEdges)), dim3(kLkEdges), 0, ctx->stream, m, std::min(L, kLkBits),
+                     n, vid, top, sz, top2, sz2);
+  HDB_LAUNCHED();
+  std::swap(top, top2);
+  std::swap(sz, sz2);
+  // ---- linkage tree and node classes
   int32_t *left, *right, *nsize, *par, *leaf_par, *cnt, *cs, *cs2, *cid, *srank, *more;
   float* lam;
   uint8_t *proc, *split;
@@ -634,6 +684,10 @@ int labels_gpu(hdb_ctx* ctx, const hdb_mst_edge* edges, int64_t m, int64_t n, in
   lam = reinterpret_cast<float*>(srank + m);
   leaf_par = reinterpret_cast<int32_t*>(lam + m);
   more = leaf_par + n;
+  uint64_t* keys;
+  uint32_t* vals;
+  HDB_CALL(scratch_t(ctx, kSlotRowCursor, m, &keys));
+  HDB_CALL(scratch_t(ctx, kSlotMisc2, m, &vals));
   HDB_CALL(scratch_t(ctx, kSlotMstFlag, 2 * m, &proc));
   split = proc + m;
   HDB_CALL(scratch_t(ctx, kSlotMstWl1, 6 * m, &anc));
@@ -644,10 +698,9 @@ int labels_gpu(hdb_ctx* ctx, const hdb_mst_edge* edges, int64_t m, int64_t n, in
   psum2 = dsum2 + m;
   HDB_CALL(scratch_t(ctx, kSlotMstWl2, 2 * (n + m), &up));
   up2 = up + (n + m);
-  int32_t* bad = more + 1;
+  int32_t* bad = bad0;
   HDB_CALL(fill_i32(ctx, par, m, -2));
   HDB_CALL(fill_i32(ctx, leaf_par, n, -2));
-  HDB_CALL(fill_i32(ctx, bad, 1, 0));
   hipLaunchKernelGGL(k_tr_nodes, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, edges, m, n, top, sz, left, right,
                      nsize, par, leaf_par, lam, bad);
   HDB_LAUNCHED();
@@ -703,8 +756,10 @@ int labels_gpu(hdb_ctx* ctx, const hdb_mst_edge* edges, int64_t m, int64_t n, in
   }
   if (*more_h) return ctx->fail(HDB_EDEVICE, "pointer jumping did not converge");
   // ---- splits in level order -> cluster ids
-  int32_t *flag32 = fg, *pflag32 = fl;
-  int64_t *spos = eg, *ppos = el;
+  int32_t *flag32 = cur.uf, *pflag32 = cur.rep_l;  // the linkage's arrays are dead by now
+  int64_t *spos, *ppos;
+  HDB_CALL(scratch_t(ctx, kSlotRowTmp, 2 * (m + 1), &spos));
+  ppos = spos + (m + 1);
   hipLaunchKernelGGL(k_u8_to_i32, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, split, m, flag32);
   HDB_LAUNCHED();
   hipLaunchKernelGGL(k_u8_to_i32, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, proc, m, pflag32);

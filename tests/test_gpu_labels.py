@@ -40,6 +40,28 @@ def test_labels_gpu_random_trees(ctx):
         np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("m", [1, 2, 3, 1023, 1024, 1025, 2047, 2048, 2049, 4097, 40001])
+@pytest.mark.parametrize("shape", ["path", "star", "random"])
+def test_labels_gpu_segment_edges(ctx, m, shape):
+    """Edge counts around the linkage's LDS segments (1024 edges) and the
+    halving levels above them, on the deepest, the widest and random trees."""
+    print(f"case: hdb_labels_gpu {shape} tree of {m} edges", flush=True)
+    rng = np.random.default_rng(m)
+    n = m + 1
+    e = _random_tree(rng, n, m % 4)
+    if shape != "random":
+        ids = rng.permutation(n)
+        e["from_node"] = ids[:-1] if shape == "path" else ids[0]
+        e["to_node"] = ids[1:]
+        e = e[rng.permutation(m)]
+        e["weight"] = np.sort(e["weight"])
+    for mpts in (2, 5, 32):
+        want, wnc = api.get_clusters(e, n, mpts)
+        got, gnc = api.get_clusters_gpu(ctx, e, n, mpts)
+        assert gnc == wnc
+        np.testing.assert_array_equal(got, want)
+
+
 def test_labels_gpu_quirk_cases(ctx):
     from test_labels import HAND_CASES, _edges
     for name, rows, n, want, want_nc in HAND_CASES:
