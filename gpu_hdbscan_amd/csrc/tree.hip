@@ -31,8 +31,8 @@
 //    preorder numbers and cluster membership come from pointer jumping.
 // 3. Stability (compute_stability, tree.cu:444-528): per cluster, the terms
 //    (lambda - birth) * size are added in the order of the condensed list
-//    (the cluster's nodes top-down, then its two split children), one
-//    thread per cluster, so the FP32 sums are those of the host version.
+//    (the cluster's nodes top-down, then its two split children), and the
+//    FP32 sums are those of the host's sequential loop, bit for bit.
 // 4. EOM selection (get_clusters, tree.cu:627-746) runs on the host over the
 //    cluster tree (one entry per cluster); labelling (do_labelling,
 //    tree.cu:569-625) is one GPU pass over the points.
@@ -533,8 +533,7 @@ __global__ void k_tr_path_bounds(int64_t P, const uint64_t* __restrict__ keys, i
 // for each of the cluster's nodes top-down, (lambda - birth) once per point
 // that leaves there, then (lambda - birth) * size for each child of a split
 // -- are laid out flat (one count per path position, a scan, then each
-// position writes its addends), and one wave per cluster adds them in that
-// order.
+// position writes its addends), and the sums below add them in that order.
 __global__ void k_tr_addend_count(int64_t P, const uint32_t* __restrict__ path, const int32_t* __restrict__ cnt,
                                   const uint8_t* __restrict__ split, int32_t* __restrict__ na) {
   const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -564,25 +563,132 @@ __global__ void k_tr_addends(int64_t P, int64_t n, const uint64_t* __restrict__ 
   }
 }
 
-// One wave per cluster: lanes load 64 addends at a time, then the sum takes
-// them in order from the lanes (a dependent chain of adds, the rounding of
-// the host's sequential loop).
-__global__ __launch_bounds__(256) void k_tr_stability(int64_t S, const int64_t* __restrict__ cbeg,
-                                                      const int64_t* __restrict__ cend, const int64_t* __restrict__ off,
-                                                      const float* __restrict__ add, float* __restrict__ stab) {
+// s += t[0] + ... in order, one rounding per add (the host's sequential
+// loop): lanes load 64 addends at a time, the wave takes them lane by lane.
+__device__ __forceinline__ float add_in_order(float s, const float* __restrict__ add, int64_t t0, int64_t t1) {
   const unsigned lane = __lane_id();
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (c >= S) return;
-  const int64_t a0 = off[cbeg[c]], a1 = off[cend[c]];
-  float s = 0.0f;
-  for (int64_t t0 = a0; t0 < a1; t0 += 64) {
+  for (; t0 < t1; t0 += 64) {
     // past the end, +0: adding it leaves s as it is (s >= 0 throughout)
-    const float v = t0 + lane < a1 ? add[t0 + lane] : 0.0f;
+    const float v = t0 + lane < t1 ? add[t0 + lane] : 0.0f;
     const int32_t vb = __float_as_int(v);
 #pragma unroll
     for (int j = 0; j < 64; ++j) s += __int_as_float(__builtin_amdgcn_readlane(vb, j));
   }
-  if (lane == 0) stab[c] = s;
+  return s;
+}
+
+constexpr int64_t kStabShort = 1024;  // addends a wave adds one by one
+
+// Clusters of at most kStabShort addends: one wave each.
+__global__ __launch_bounds__(256) void k_tr_stability(int64_t S, const int64_t* __restrict__ cbeg,
+                                                      const int64_t* __restrict__ cend, const int64_t* __restrict__ off,
+                                                      const float* __restrict__ add, float* __restrict__ stab) {
+  const int64_t c = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (c >= S) return;
+  const int64_t a0 = off[cbeg[c]], a1 = off[cend[c]];
+  if (a1 - a0 > kStabShort) return;
+  const float s = add_in_order(0.0f, add, a0, a1);
+  if (__lane_id() == 0) stab[c] = s;
+}
+
+// Longer clusters, bit for bit the same sequential FP32 sum, in parallel.
+// While s stays in one binade [2^e, 2^(e+1)) it is an integer multiple S of
+// u = 2^(e-23), and adding t >= 0 moves it by RNE(S + t/u) - S units.  That
+// step depends on S only through its parity (which decides ties), so a run
+// of addends is a map (parity of S) -> (units added), and such maps compose
+// associatively.  The step for an even and an odd S is read off the bits of
+// 2^e + t and 2^e + u + t, which the hardware rounds the same way.  Each of
+// the block's 16 waves composes the map of 1024 addends; the maps are then
+// applied in order until one would leave the binade (or its addends are not
+// all finite and >= 0), whose 1024 addends are added one by one.  s leaves at
+// most ~log2(addends) binades, so nearly all the work is parallel: the
+// serial chain took 8 cycles per addend, 28.7 ms for the largest cluster of
+// 10M x 12; this kernel takes 0.84 ms there.
+constexpr int kStabWaves = 16;
+constexpr uint32_t kStabBig = 1u << 25;  // more units than any binade holds
+
+__global__ __launch_bounds__(kStabWaves * 64) void k_tr_stability_long(
+    int64_t S, const int64_t* __restrict__ cbeg, const int64_t* __restrict__ cend, const int64_t* __restrict__ off,
+    const float* __restrict__ add, float* __restrict__ stab) {
+  __shared__ uint32_t s_even[kStabWaves], s_odd[kStabWaves];
+  __shared__ float s_sum;
+  const unsigned lane = __lane_id();
+  const int w = static_cast<int>(threadIdx.x >> 6);
+  for (int64_t c = blockIdx.x; c < S; c += gridDim.x) {
+    const int64_t a0 = off[cbeg[c]], a1 = off[cend[c]];
+    if (a1 - a0 <= kStabShort) continue;  // uniform across the block
+    // the first addends one by one, up to a 16-byte aligned position
+    int64_t pos = a0 + 1024 - (a0 & 3);
+    if (w == 0) {
+      const float s = add_in_order(0.0f, add, a0, pos);
+      if (lane == 0) s_sum = s;
+    }
+    __syncthreads();
+    float s = s_sum;
+    while (pos < a1) {  // uniform
+      uint32_t sb = __float_as_uint(s);
+      const uint32_t base = sb & 0xFF800000u;
+      const float b0 = __uint_as_float(base), b1 = __uint_as_float(base | 1u);
+      // units added by this lane's 16 addends from an even (e) and odd (o) S
+      uint32_t e = 0, o = 0;
+      const int64_t p0 = pos + w * 1024 + lane * 16;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t p = p0 + 4 * q;
+        float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (p + 3 < a1) {
+          const float4 v = *reinterpret_cast<const float4*>(add + p);
+          t[0] = v.x, t[1] = v.y, t[2] = v.z, t[3] = v.w;
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if (p + k < a1) t[k] = add[p + k];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const bool ok = t[k] >= 0.0f && t[k] < __uint_as_float(0x7F800000u);
+          const uint32_t i0 = ok ? __float_as_uint(b0 + t[k]) - base : kStabBig;
+          const uint32_t i1 = ok ? __float_as_uint(b1 + t[k]) - (base | 1u) : kStabBig;
+          e = min(e + min((e & 1u) ? i1 : i0, kStabBig), kStabBig);
+          o = min(o + min((o & 1u) ? i0 : i1, kStabBig), kStabBig);
+        }
+      }
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {  // lane i takes lanes [i, i + 2d)
+        const uint32_t re = __shfl_down(e, d), ro = __shfl_down(o, d);
+        e = min(e + ((e & 1u) ? ro : re), kStabBig);
+        o = min(o + ((o & 1u) ? re : ro), kStabBig);
+      }
+      if (lane == 0) {
+        s_even[w] = e;
+        s_odd[w] = o;
+      }
+      __syncthreads();
+      // s must be a normal number: 0, denormals and infinities go one by one
+      const uint32_t ex = (sb >> 23) & 0x1FFu;
+      const bool normal = ex >= 1u && ex <= 254u;
+      int k = 0;
+      for (; k < kStabWaves && normal; ++k) {
+        const uint32_t inc = (sb & 1u) ? s_odd[k] : s_even[k];
+        if (inc >= 0x800000u - (sb & 0x7FFFFFu)) break;
+        sb += inc;
+      }
+      s = __uint_as_float(sb);
+      pos += static_cast<int64_t>(k) * 1024;
+      if (k < kStabWaves && pos < a1) {  // uniform
+        if (w == 0) {
+          const float r = add_in_order(s, add, pos, pos + 1024 < a1 ? pos + 1024 : a1);
+          if (lane == 0) s_sum = r;
+        }
+        pos += 1024;
+        __syncthreads();
+        s = s_sum;
+      }
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) stab[c] = s;
+    __syncthreads();
+  }
 }
 
 // Point p leaves at internal node fall = parent of its highest small
@@ -820,6 +926,11 @@ int labels_gpu(hdb_ctx* ctx, const hdb_mst_edge* edges, int64_t m, int64_t n, in
     hipLaunchKernelGGL(k_tr_stability, dim3(grid_for(S, 4)), dim3(256), 0, ctx->stream, S, cbeg, cend, aoff, add,
                        stab);
     HDB_LAUNCHED();
+    if (A > kStabShort) {
+      hipLaunchKernelGGL(k_tr_stability_long, dim3(static_cast<unsigned>(std::min<int64_t>(S, 512))),
+                         dim3(kStabWaves * 64), 0, ctx->stream, S, cbeg, cend, aoff, add, stab);
+      HDB_LAUNCHED();
+    }
   }
   // ---- EOM selection over the cluster tree (host; one entry per cluster)
   std::vector<float> h_stab(S), h_birth(S);

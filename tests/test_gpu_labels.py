@@ -62,6 +62,38 @@ def test_labels_gpu_segment_edges(ctx, m, shape):
         np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("per", [1000, 1025, 5000, 17500, 70001])
+@pytest.mark.parametrize("weights", ["tied", "distinct", "zeros"])
+def test_labels_gpu_long_clusters(ctx, per, weights):
+    """Clusters of more than 1024 stability addends (summed in parallel, bit
+    for bit as one by one): a few dense blobs joined by long edges, with
+    weights whose exact and rounded sums tie, differ, or start at infinity's
+    stand-in (zero weights)."""
+    print(f"case: hdb_labels_gpu blobs of {per} points, {weights} weights", flush=True)
+    rng = np.random.default_rng(per)
+    blobs = 3
+    n = blobs * per
+    m = n - 1
+    e = np.empty(m, api.MST_EDGE)
+    child = np.arange(1, n)
+    start = (child // per) * per
+    joint = child == start
+    prev = start + (rng.random(m) * np.maximum(child - start, 1)).astype(np.int64)
+    e["from_node"] = np.where(joint, child - per, prev)
+    e["to_node"] = child
+    if weights == "distinct":
+        w = rng.gamma(2.0, 0.1, m)
+    else:
+        w = rng.choice([0.0, 0.25, 0.5] if weights == "zeros" else [0.25, 0.3, 0.5, 0.75, 1.0], m)
+    e["weight"] = np.where(joint, 4.0 + child / n, w).astype(np.float32)
+    e = e[np.argsort(e["weight"], kind="stable")]
+    for mpts in (2, 32):
+        want, wnc = api.get_clusters(e, n, mpts)
+        got, gnc = api.get_clusters_gpu(ctx, e, n, mpts)
+        assert gnc == wnc
+        np.testing.assert_array_equal(got, want)
+
+
 def test_labels_gpu_quirk_cases(ctx):
     from test_labels import HAND_CASES, _edges
     for name, rows, n, want, want_nc in HAND_CASES:
