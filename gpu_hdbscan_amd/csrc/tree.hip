@@ -28,7 +28,9 @@
 //    clusters, numbered in the level order of the splits (depth, then
 //    preorder); every other processed node continues its cluster, and the
 //    points of its small children leave that cluster at its lambda.  Depths,
-//    preorder numbers and cluster membership come from pointer jumping.
+//    preorder numbers and cluster starts come from one pointer jumping over
+//    16-byte node records, whose log2(m) rounds are queued without a host
+//    round trip.
 // 3. Stability (compute_stability, tree.cu:444-528): per cluster, the terms
 //    (lambda - birth) * size are added in the order of the condensed list
 //    (the cluster's nodes top-down, then its two split children), and the
@@ -38,6 +40,7 @@
 //    tree.cu:569-625) is one GPU pass over the points.
 #include <algorithm>
 #include <climits>
+#include <cstring>
 #include <vector>
 
 #include "hdb_internal.hpp"
@@ -130,10 +133,14 @@ __global__ void k_lk_first(const hdb_mst_edge* __restrict__ e, int64_t m, int64_
   else lower_to(first + v, static_cast<int32_t>(q));
 }
 
+// Also clears the parents that k_tr_nodes fills in (par: m, leaf_par: n <= 2m).
 __global__ void k_lk_init(const hdb_mst_edge* __restrict__ e, int64_t m, int64_t n, const int32_t* __restrict__ first,
-                          int32_t* __restrict__ vid, int32_t* __restrict__ top, int32_t* __restrict__ sz, LkLevel a) {
+                          int32_t* __restrict__ vid, int32_t* __restrict__ top, int32_t* __restrict__ sz, LkLevel a,
+                          int32_t* __restrict__ par, int32_t* __restrict__ leaf_par) {
   const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (q >= 2 * m) return;
+  if (q < m) par[q] = -2;
+  if (q < n) leaf_par[q] = -2;
   const int32_t v = (q & 1) ? e[q >> 1].to_node : e[q >> 1].from_node;
   vid[q] = v >= 0 && v < n ? first[v] : static_cast<int32_t>(q);
   top[q] = v;
@@ -352,212 +359,220 @@ __global__ void k_tr_nodes(const hdb_mst_edge* __restrict__ e, int64_t m, int64_
   if (i == m - 1) par[i] = -1;
 }
 
-// Every node but the root has a later node as parent, every point a node:
-// the tree is whole, so the passes below stay in bounds.
-__global__ void k_tr_check(int64_t m, int64_t n, const int32_t* __restrict__ par,
-                           const int32_t* __restrict__ leaf_par, int32_t* __restrict__ bad) {
-  const int64_t x = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (x < n) {
-    const int32_t p = leaf_par[x];
-    if (p < 0 || p >= m) *bad = 1;
-  } else if (x < n + m - 1) {
-    const int64_t i = x - n;
-    const int32_t p = par[i];
-    if (p <= i || p >= m) *bad = 1;
-  }
-}
-
 __device__ __forceinline__ int32_t node_size(int32_t x, int64_t n, const int32_t* nsize) {
   return x >= n ? nsize[x - n] : 1;
 }
 
+// State of a node in the pointer jumping: anc, the ancestor reached (-1 past
+// the root); the sums of depth and preorder steps up to it; and link, the
+// node searched for on the way up (its cluster's start for a processed node,
+// the highest small ancestor-or-self for a small one) or anc while that
+// lies further up.  One 16-byte record, so a round is one gather per node.
+struct __attribute__((aligned(16))) TrRec {
+  int32_t anc, depth, pre, link;
+};
+
+constexpr uint8_t kProc = 1, kSplit = 2;
+
 // Per internal node: processed (the root, or at least mpts points), split
 // (both children hold mpts points), the points of its small children
-// (they leave its cluster at its lambda), and the preorder increment and
-// the jump pointers of the pointer-jumping passes.
+// (they leave its cluster at its lambda), and its record before any jump:
+// its parent, one step down, its preorder increment.  Split nodes are
+// appended to `splits` (in any order).  Every node but the root must have a
+// later node as parent, every point a node; otherwise *bad is set and the
+// node treated as a root, so that the passes below stay in bounds.
 __global__ void k_tr_classify(int64_t m, int64_t n, int mpts, const int32_t* __restrict__ left,
                               const int32_t* __restrict__ right, const int32_t* __restrict__ nsize,
-                              const int32_t* __restrict__ par, uint8_t* __restrict__ proc,
-                              uint8_t* __restrict__ split, int32_t* __restrict__ cnt, int64_t* __restrict__ anc,
-                              int64_t* __restrict__ dsum, int64_t* __restrict__ psum, int32_t* __restrict__ cs) {
+                              const int32_t* __restrict__ par, const int32_t* __restrict__ leaf_par,
+                              uint8_t* __restrict__ flags, int32_t* __restrict__ cnt, TrRec* __restrict__ rec,
+                              int32_t* __restrict__ splits, int32_t* __restrict__ nsplit, int32_t* __restrict__ bad) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const bool root = i == m - 1;
-  const bool pr = root || nsize[i] >= mpts;
-  const int32_t ls = node_size(left[i], n, nsize), rs = node_size(right[i], n, nsize);
-  const bool sp = pr && ls >= mpts && rs >= mpts;
-  proc[i] = pr ? 1 : 0;
-  split[i] = sp ? 1 : 0;
-  cnt[i] = pr ? (ls < mpts ? ls : 0) + (rs < mpts ? rs : 0) : 0;
-  const int32_t p = par[i];
-  anc[i] = p;
-  dsum[i] = root ? 0 : 1;
-  int64_t inc = 0;
-  if (!root) {
-    const bool is_right = right[p] == static_cast<int32_t>(n + i);
-    inc = 1 + (is_right ? 2 * static_cast<int64_t>(node_size(left[p], n, nsize)) - 1 : 0);
+  if (i < n) {
+    const int32_t lp = leaf_par[i];
+    if (lp < 0 || lp >= m) *bad = 1;
   }
-  psum[i] = inc;
-  // cluster start: the root, or a child of a split node
-  const bool start = root || (pr && (node_size(left[p], n, nsize) >= mpts && node_size(right[p], n, nsize) >= mpts));
-  cs[i] = start ? static_cast<int32_t>(i) : p;
-}
-
-// One pointer-jumping round of (ancestor, depth sum, preorder sum).
-__global__ void k_tr_jump_sums(int64_t m, const int64_t* __restrict__ anc, const int64_t* __restrict__ dsum,
-                               const int64_t* __restrict__ psum, int64_t* __restrict__ anc2,
-                               int64_t* __restrict__ dsum2, int64_t* __restrict__ psum2, int32_t* __restrict__ more) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const int64_t a = anc[i];
-  if (a < 0) {
-    anc2[i] = a;
-    dsum2[i] = dsum[i];
-    psum2[i] = psum[i];
-    return;
+  bool sp = false;
+  if (i < m) {
+    int32_t p = par[i];
+    if (i != m - 1 && (p <= i || p >= m)) {
+      *bad = 1;
+      p = -1;
+    }
+    const bool root = p < 0;
+    const bool pr = root || nsize[i] >= mpts;
+    const int32_t ls = node_size(left[i], n, nsize), rs = node_size(right[i], n, nsize);
+    sp = pr && ls >= mpts && rs >= mpts;
+    flags[i] = (pr ? kProc : 0) | (sp ? kSplit : 0);
+    cnt[i] = pr ? (ls < mpts ? ls : 0) + (rs < mpts ? rs : 0) : 0;
+    TrRec r{p, 0, 0, static_cast<int32_t>(i)};
+    if (!root) {
+      const int32_t pl = node_size(left[p], n, nsize);
+      const bool is_right = right[p] == static_cast<int32_t>(n + i);
+      r.depth = 1;
+      r.pre = 1 + (is_right ? 2 * pl - 1 : 0);
+      // a search ends here at a cluster start (a child of a split) and at a
+      // small node under a processed one
+      const bool ppr = p == m - 1 || nsize[p] >= mpts;
+      const bool psp = ppr && pl >= mpts && node_size(right[p], n, nsize) >= mpts;
+      if (pr ? !psp : !ppr) r.link = p;
+    }
+    rec[i] = r;
   }
-  anc2[i] = anc[a];
-  dsum2[i] = dsum[i] + dsum[a];
-  psum2[i] = psum[i] + psum[a];
-  if (anc[a] >= 0) *more = 1;
+  const uint64_t bal = __ballot(sp);
+  if (bal) {
+    const unsigned lane = __lane_id();
+    int32_t base = 0;
+    if (lane == static_cast<unsigned>(__builtin_ctzll(bal))) base = atomicAdd(nsplit, __popcll(bal));
+    base = __shfl(base, __builtin_ctzll(bal));
+    if (sp) splits[base + __popcll(bal & lanemask_lt())] = static_cast<int32_t>(i);
+  }
 }
 
-// One round of the cluster-start jump (processed nodes only change).
-__global__ void k_tr_jump_cs(int64_t m, const int32_t* __restrict__ cs, int32_t* __restrict__ cs2,
-                             int32_t* __restrict__ more) {
+// One round: anc doubles its reach.  link, while it equals anc, takes what
+// anc's record found (or its anc); once it differs it is final.
+__global__ void k_tr_jump(int64_t m, const TrRec* __restrict__ in, TrRec* __restrict__ out) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= m) return;
-  const int32_t a = cs[i];
-  const int32_t b = a >= 0 ? cs[a] : a;
-  cs2[i] = b;
-  if (b != a) *more = 1;
+  TrRec r = in[i];
+  if (r.anc >= 0) {
+    const TrRec a = in[r.anc];
+    if (r.link == r.anc) r.link = a.link;
+    r.anc = a.anc;
+    r.depth += a.depth;
+    r.pre += a.pre;
+  }
+  out[i] = r;
 }
 
-// Leaves and small internal nodes: up = parent until the parent is
-// processed (points of a small subtree leave at that parent).
-__global__ void k_tr_up_init(int64_t m, int64_t n, const int32_t* __restrict__ par,
-                             const int32_t* __restrict__ leaf_par, const uint8_t* __restrict__ proc,
-                             int64_t* __restrict__ up) {
-  const int64_t x = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (x >= n + m) return;
-  const int32_t p = x < n ? leaf_par[x] : par[x - n];
-  up[x] = (p < 0 || proc[p]) ? x : n + p;
+// Up to kSplitSmall splits: ranked by (depth, preorder), their level order,
+// by one block in LDS.  The left child of the split of rank k starts
+// cluster 1 + 2k, the right one 2 + 2k (the root's cluster is 0); ids
+// relative to n.  One launch where a radix sort takes over fifty.
+constexpr int kSplitSmall = 2048;
+__global__ __launch_bounds__(1024) void k_tr_split_rank_small(int S2, const int32_t* __restrict__ splits,
+                                                              const TrRec* __restrict__ rec,
+                                                              int32_t* __restrict__ srank) {
+  __shared__ uint64_t key[kSplitSmall];
+  __shared__ int32_t node[kSplitSmall];
+  int p = 1;
+  while (p < S2) p <<= 1;
+  for (int t = threadIdx.x; t < p; t += 1024) {
+    key[t] = kKeyMax;
+    node[t] = -1;
+    if (t < S2) {
+      const int32_t i = splits[t];
+      const TrRec r = rec[i];
+      key[t] = (static_cast<uint64_t>(static_cast<uint32_t>(r.depth)) << 32) | static_cast<uint32_t>(r.pre);
+      node[t] = i;
+    }
+  }
+  __syncthreads();
+  for (int k = 2; k <= p; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      for (int t = threadIdx.x; t < p; t += 1024) {
+        const int o = t ^ j;
+        if (o > t && (key[t] > key[o]) == ((t & k) == 0)) {
+          const uint64_t x = key[t];
+          key[t] = key[o];
+          key[o] = x;
+          const int32_t y = node[t];
+          node[t] = node[o];
+          node[o] = y;
+        }
+      }
+      __syncthreads();
+    }
+  for (int t = threadIdx.x; t < S2; t += 1024) srank[node[t]] = t;
 }
 
-__global__ void k_tr_up_jump(int64_t total, const int64_t* __restrict__ up, int64_t* __restrict__ up2,
-                             int32_t* __restrict__ more) {
-  const int64_t x = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (x >= total) return;
-  const int64_t a = up[x];
-  const int64_t b = up[a];
-  up2[x] = b;
-  if (b != a) *more = 1;
-}
-
-// Split nodes, keyed by (depth, preorder): their level order.
-__global__ void k_tr_split_keys(int64_t m, const uint8_t* __restrict__ split, const int64_t* __restrict__ depth,
-                                const int64_t* __restrict__ pre, const int64_t* __restrict__ spos,
+__global__ void k_tr_split_keys(int64_t S2, const int32_t* __restrict__ splits, const TrRec* __restrict__ rec,
                                 uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= m || !split[i]) return;
-  keys[spos[i]] = (static_cast<uint64_t>(depth[i]) << 32) | static_cast<uint64_t>(pre[i]);
-  vals[spos[i]] = static_cast<uint32_t>(i);
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (t >= S2) return;
+  const int32_t i = splits[t];
+  const TrRec r = rec[i];
+  keys[t] = (static_cast<uint64_t>(static_cast<uint32_t>(r.depth)) << 32) | static_cast<uint32_t>(r.pre);
+  vals[t] = static_cast<uint32_t>(i);
 }
 
-// Split of rank k (level order): its left child starts cluster 1 + 2k, its
-// right child 2 + 2k (the root's cluster is 0); ids relative to n.
 __global__ void k_tr_split_rank(int64_t S2, const uint32_t* __restrict__ vals, int32_t* __restrict__ srank) {
   const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (k < S2) srank[vals[k]] = static_cast<int32_t>(k);
 }
 
-// Cluster of every processed node (relative id), and per cluster: its
-// start node, birth lambda, parent cluster and split children.
-__global__ void k_tr_clusters(int64_t m, int64_t n, const uint8_t* __restrict__ proc, const int32_t* __restrict__ cs,
-                              const int32_t* __restrict__ par, const int32_t* __restrict__ left,
-                              const int32_t* __restrict__ srank, const float* __restrict__ lam,
-                              int32_t* __restrict__ cid, float* __restrict__ birth, int32_t* __restrict__ cparent) {
+// Relative cluster id of the cluster that starts at node s.
+__device__ __forceinline__ int32_t cluster_of(int32_t s, int64_t n, const int32_t* __restrict__ par,
+                                              const int32_t* __restrict__ left, const int32_t* __restrict__ srank) {
+  const int32_t p = par[s];
+  if (p < 0) return 0;
+  return (left[p] == static_cast<int32_t>(n + s) ? 1 : 2) + 2 * srank[p];
+}
+
+// Cluster of every processed node (relative id) and, per cluster, its birth
+// lambda, parent cluster and length.  A cluster's nodes are one path down
+// from its start (a processed node that does not split has at most one child
+// of mpts points), so a node's position on it is a difference of depths and
+// its last node gives the length.  na is cleared for k_tr_addend_count.
+__global__ void k_tr_clusters(int64_t m, int64_t n, int mpts, const uint8_t* __restrict__ flags,
+                              const TrRec* __restrict__ rec, const int32_t* __restrict__ par,
+                              const int32_t* __restrict__ left, const int32_t* __restrict__ right,
+                              const int32_t* __restrict__ nsize, const int32_t* __restrict__ srank,
+                              const float* __restrict__ lam, int32_t* __restrict__ cid, int32_t* __restrict__ pos,
+                              float* __restrict__ birth, int32_t* __restrict__ cparent, int32_t* __restrict__ clen,
+                              int32_t* __restrict__ na) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= m) return;
-  if (!proc[i]) {
+  na[i] = 0;
+  const uint8_t f = flags[i];
+  if (!(f & kProc)) {
     cid[i] = -1;
     return;
   }
-  const int32_t s = cs[i];  // the cluster's start node
-  int32_t c;
-  if (s == static_cast<int32_t>(m - 1)) {
-    c = 0;
-  } else {
-    const int32_t p = par[s];
-    c = (left[p] == static_cast<int32_t>(n + s) ? 1 : 2) + 2 * srank[p];
-  }
+  const TrRec r = rec[i];
+  const int32_t c = cluster_of(r.link, n, par, left, srank);
+  const int32_t at = r.depth - rec[r.link].depth;
   cid[i] = c;
-  if (s == static_cast<int32_t>(i)) {
-    if (c == 0) {
-      birth[0] = 0.0f;
-      cparent[0] = -1;
-    } else {
-      birth[c] = lam[par[i]];
-      cparent[c] = -2;  // filled by k_tr_cparent (needs the parent's cid)
-    }
+  pos[i] = at;
+  if (r.link == static_cast<int32_t>(i)) {
+    const int32_t p = par[i];
+    birth[c] = p < 0 ? 0.0f : lam[p];
+    cparent[c] = p < 0 ? -1 : cluster_of(rec[p].link, n, par, left, srank);
   }
-}
-
-__global__ void k_tr_cparent(int64_t m, const int32_t* __restrict__ cs, const int32_t* __restrict__ par,
-                             const int32_t* __restrict__ cid, int32_t* __restrict__ cparent) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= m || cid[i] <= 0 || cs[i] != static_cast<int32_t>(i)) return;
-  cparent[cid[i]] = cid[par[i]];
-}
-
-// Processed nodes keyed by (cluster, depth): each cluster's nodes top-down.
-__global__ void k_tr_path_keys(int64_t m, const int32_t* __restrict__ cid, const int64_t* __restrict__ depth,
-                               const int64_t* __restrict__ ppos, const uint8_t* __restrict__ proc,
-                               uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= m || !proc[i]) return;
-  keys[ppos[i]] = (static_cast<uint64_t>(cid[i]) << 32) | static_cast<uint64_t>(depth[i]);
-  vals[ppos[i]] = static_cast<uint32_t>(i);
-}
-
-__global__ void k_tr_path_bounds(int64_t P, const uint64_t* __restrict__ keys, int64_t* __restrict__ cbeg,
-                                 int64_t* __restrict__ cend) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= P) return;
-  const uint32_t c = static_cast<uint32_t>(keys[t] >> 32);
-  if (t == 0 || static_cast<uint32_t>(keys[t - 1] >> 32) != c) cbeg[c] = t;
-  if (t == P - 1 || static_cast<uint32_t>(keys[t + 1] >> 32) != c) cend[c] = t + 1;
+  if ((f & kSplit) || (node_size(left[i], n, nsize) < mpts && node_size(right[i], n, nsize) < mpts)) clen[c] = at + 1;
 }
 
 // Stability: per cluster, the addends of the host version in its order --
 // for each of the cluster's nodes top-down, (lambda - birth) once per point
 // that leaves there, then (lambda - birth) * size for each child of a split
-// -- are laid out flat (one count per path position, a scan, then each
-// position writes its addends), and the sums below add them in that order.
-__global__ void k_tr_addend_count(int64_t P, const uint32_t* __restrict__ path, const int32_t* __restrict__ cnt,
-                                  const uint8_t* __restrict__ split, int32_t* __restrict__ na) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= P) return;
-  const uint32_t i = path[t];
-  na[t] = cnt[i] + (split[i] ? 2 : 0);
+// -- are laid out flat (one count per path position, cluster after cluster, a
+// scan, then each node writes its addends), and the sums below add them in
+// that order.
+__global__ void k_tr_addend_count(int64_t m, const uint8_t* __restrict__ flags, const int32_t* __restrict__ cid,
+                                  const int32_t* __restrict__ pos, const int64_t* __restrict__ cbeg,
+                                  const int32_t* __restrict__ cnt, int32_t* __restrict__ na) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= m) return;
+  const uint8_t f = flags[i];
+  if (f & kProc) na[cbeg[cid[i]] + pos[i]] = cnt[i] + ((f & kSplit) ? 2 : 0);
 }
 
-__global__ void k_tr_addends(int64_t P, int64_t n, const uint64_t* __restrict__ keys,
-                             const uint32_t* __restrict__ path, const int32_t* __restrict__ cnt,
-                             const uint8_t* __restrict__ split, const float* __restrict__ lam,
+__global__ void k_tr_addends(int64_t m, int64_t n, const uint8_t* __restrict__ flags, const int32_t* __restrict__ cid,
+                             const int32_t* __restrict__ pos, const int64_t* __restrict__ cbeg,
+                             const int32_t* __restrict__ cnt, const float* __restrict__ lam,
                              const int32_t* __restrict__ left, const int32_t* __restrict__ right,
                              const int32_t* __restrict__ nsize, const float* __restrict__ birth,
                              const int64_t* __restrict__ off, float* __restrict__ add) {
 #pragma clang fp contract(off)  // products rounded on their own, as on the host
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= P) return;
-  const uint32_t i = path[t];
-  const uint32_t c = static_cast<uint32_t>(keys[t] >> 32);
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= m) return;
+  const uint8_t f = flags[i];
+  if (!(f & kProc)) return;
+  const int32_t c = cid[i];
   const float term = lam[i] - birth[c];
-  float* dst = add + off[t];
+  float* dst = add + off[cbeg[c] + pos[i]];
   const int k = cnt[i];
   for (int r = 0; r < k; ++r) dst[r] = term;
-  if (split[i]) {
+  if (f & kSplit) {
     dst[k] = term * static_cast<float>(node_size(left[i], n, nsize));
     dst[k + 1] = term * static_cast<float>(node_size(right[i], n, nsize));
   }
@@ -581,11 +596,11 @@ constexpr int64_t kStabShort = 1024;  // addends a wave adds one by one
 
 // Clusters of at most kStabShort addends: one wave each.
 __global__ __launch_bounds__(256) void k_tr_stability(int64_t S, const int64_t* __restrict__ cbeg,
-                                                      const int64_t* __restrict__ cend, const int64_t* __restrict__ off,
-                                                      const float* __restrict__ add, float* __restrict__ stab) {
+                                                      const int64_t* __restrict__ off, const float* __restrict__ add,
+                                                      float* __restrict__ stab) {
   const int64_t c = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (c >= S) return;
-  const int64_t a0 = off[cbeg[c]], a1 = off[cend[c]];
+  const int64_t a0 = off[cbeg[c]], a1 = off[cbeg[c + 1]];
   if (a1 - a0 > kStabShort) return;
   const float s = add_in_order(0.0f, add, a0, a1);
   if (__lane_id() == 0) stab[c] = s;
@@ -608,14 +623,14 @@ constexpr int kStabWaves = 16;
 constexpr uint32_t kStabBig = 1u << 25;  // more units than any binade holds
 
 __global__ __launch_bounds__(kStabWaves * 64) void k_tr_stability_long(
-    int64_t S, const int64_t* __restrict__ cbeg, const int64_t* __restrict__ cend, const int64_t* __restrict__ off,
-    const float* __restrict__ add, float* __restrict__ stab) {
+    int64_t S, const int64_t* __restrict__ cbeg, const int64_t* __restrict__ off, const float* __restrict__ add,
+    float* __restrict__ stab) {
   __shared__ uint32_t s_even[kStabWaves], s_odd[kStabWaves];
   __shared__ float s_sum;
   const unsigned lane = __lane_id();
   const int w = static_cast<int>(threadIdx.x >> 6);
   for (int64_t c = blockIdx.x; c < S; c += gridDim.x) {
-    const int64_t a0 = off[cbeg[c]], a1 = off[cend[c]];
+    const int64_t a0 = off[cbeg[c]], a1 = off[cbeg[c + 1]];
     if (a1 - a0 <= kStabShort) continue;  // uniform across the block
     // the first addends one by one, up to a 16-byte aligned position
     int64_t pos = a0 + 1024 - (a0 & 3);
@@ -691,25 +706,21 @@ __global__ __launch_bounds__(kStabWaves * 64) void k_tr_stability_long(
   }
 }
 
-// Point p leaves at internal node fall = parent of its highest small
-// ancestor-or-self; its label is its cluster's selected ancestor's, when
-// its lambda is strictly above that cluster's birth.
-__global__ void k_tr_label(int64_t n, const int64_t* __restrict__ up, const int32_t* __restrict__ leaf_par,
-                           const int32_t* __restrict__ par, const int32_t* __restrict__ cid,
-                           const float* __restrict__ lam, const int32_t* __restrict__ clab,
-                           const float* __restrict__ cbirth, int32_t* __restrict__ labels) {
+// Point p leaves at its lowest processed ancestor: its parent, or the parent
+// of the highest small node above it.  Its label is its cluster's selected
+// ancestor's, when its lambda is strictly above that cluster's birth.
+__global__ void k_tr_label(int64_t n, const int32_t* __restrict__ leaf_par, const uint8_t* __restrict__ flags,
+                           const TrRec* __restrict__ rec, const int32_t* __restrict__ par,
+                           const int32_t* __restrict__ cid, const float* __restrict__ lam,
+                           const int32_t* __restrict__ clab, const float* __restrict__ cbirth,
+                           int32_t* __restrict__ labels) {
   const int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (p >= n) return;
-  const int64_t t = up[p];
-  const int32_t f = t < n ? leaf_par[t] : par[t - n];
+  int32_t f = leaf_par[p];
+  if (!(flags[f] & kProc)) f = par[rec[f].link];
   const int32_t c = cid[f];
   const int32_t l = clab[c];
   labels[p] = (l >= 0 && lam[f] > cbirth[c]) ? l : -1;
-}
-
-__global__ void k_u8_to_i32(const uint8_t* __restrict__ in, int64_t n, int32_t* __restrict__ out) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = in[i];
 }
 
 __global__ void k_tr_fill_neg(int32_t* __restrict__ p, int64_t n) {
@@ -733,24 +744,40 @@ int labels_gpu(hdb_ctx* ctx, const hdb_mst_edge* edges, int64_t m, int64_t n, in
     return HDB_OK;
   }
   const int64_t Q = 2 * m;
+  // node arrays and controls {bad, number of splits}
+  int32_t *left, *right, *nsize, *par, *leaf_par, *cnt, *cid, *pos, *srank, *splits, *ctrl;
+  float* lam;
+  HDB_CALL(scratch_t(ctx, kSlotMstParent, 10 * m + n + 8, &ctrl));
+  left = ctrl + 8;
+  right = left + m;
+  nsize = right + m;
+  par = nsize + m;
+  cnt = par + m;
+  cid = cnt + m;
+  pos = cid + m;
+  srank = pos + m;
+  splits = srank + m;
+  lam = reinterpret_cast<float*>(splits + m);
+  leaf_par = reinterpret_cast<int32_t*>(lam + m);
+  int32_t *bad = ctrl, *nsplit = ctrl + 1;
+  HDB_CALL(fill_u64(ctx, reinterpret_cast<uint64_t*>(ctrl), 1, 0));
   // ---- linkage
-  int32_t *vid, *top, *sz, *top2, *sz2, *lv, *bad0;
+  int32_t *vid, *top, *sz, *top2, *sz2, *lv;
   HDB_CALL(scratch_t(ctx, kSlotMisc0, 5 * Q, &vid));
   top = vid + Q;
   sz = top + Q;
   top2 = sz + Q;
   sz2 = top2 + Q;
-  HDB_CALL(scratch_t(ctx, kSlotMisc1, 10 * Q + 1, &lv));
+  HDB_CALL(scratch_t(ctx, kSlotMisc1, 10 * Q, &lv));
   LkLevel cur{lv, lv + Q, lv + 2 * Q, lv + 3 * Q, lv + 4 * Q};
   LkLevel alt{lv + 5 * Q, lv + 6 * Q, lv + 7 * Q, lv + 8 * Q, lv + 9 * Q};
-  bad0 = lv + 10 * Q;
   const unsigned gq = grid_for(Q, 256), gm = grid_for(m, 256);
   // the lowest end of every point, in an array the first level resets later
   HDB_CALL(fill_i32(ctx, alt.rep_l, Q, kNoName));  // Q >= n for m = n - 1 >= 1
-  HDB_CALL(fill_i32(ctx, bad0, 1, 0));
-  hipLaunchKernelGGL(k_lk_first, dim3(gq), dim3(256), 0, ctx->stream, edges, m, n, alt.rep_l, bad0);
+  hipLaunchKernelGGL(k_lk_first, dim3(gq), dim3(256), 0, ctx->stream, edges, m, n, alt.rep_l, bad);
   HDB_LAUNCHED();
-  hipLaunchKernelGGL(k_lk_init, dim3(gq), dim3(256), 0, ctx->stream, edges, m, n, alt.rep_l, vid, top, sz, cur);
+  hipLaunchKernelGGL(k_lk_init, dim3(gq), dim3(256), 0, ctx->stream, edges, m, n, alt.rep_l, vid, top, sz, cur, par,
+                     leaf_par);
   HDB_LAUNCHED();
   const int L = bits_for(m - 1);
   // edges per thread of k_lk_merge: blocks of 4096 edges where they fill the
@@ -773,172 +800,91 @@ int labels_gpu(hdb_ctx* ctx, const hdb_mst_edge* edges, int64_t m, int64_t n, in
   HDB_LAUNCHED();
   std::swap(top, top2);
   std::swap(sz, sz2);
-  // ---- linkage tree and node classes
-  int32_t *left, *right, *nsize, *par, *leaf_par, *cnt, *cs, *cs2, *cid, *srank, *more;
-  float* lam;
-  uint8_t *proc, *split;
-  int64_t *anc, *dsum, *psum, *anc2, *dsum2, *psum2, *up, *up2;
-  HDB_CALL(scratch_t(ctx, kSlotMstParent, 11 * m + n + 64, &left));
-  right = left + m;
-  nsize = right + m;
-  par = nsize + m;
-  cnt = par + m;
-  cs = cnt + m;
-  cs2 = cs + m;
-  cid = cs2 + m;
-  srank = cid + m;
-  lam = reinterpret_cast<float*>(srank + m);
-  leaf_par = reinterpret_cast<int32_t*>(lam + m);
-  more = leaf_par + n;
-  uint64_t* keys;
-  uint32_t* vals;
-  HDB_CALL(scratch_t(ctx, kSlotRowCursor, m, &keys));
-  HDB_CALL(scratch_t(ctx, kSlotMisc2, m, &vals));
-  HDB_CALL(scratch_t(ctx, kSlotMstFlag, 2 * m, &proc));
-  split = proc + m;
-  HDB_CALL(scratch_t(ctx, kSlotMstWl1, 6 * m, &anc));
-  dsum = anc + m;
-  psum = dsum + m;
-  anc2 = psum + m;
-  dsum2 = anc2 + m;
-  psum2 = dsum2 + m;
-  HDB_CALL(scratch_t(ctx, kSlotMstWl2, 2 * (n + m), &up));
-  up2 = up + (n + m);
-  int32_t* bad = bad0;
-  HDB_CALL(fill_i32(ctx, par, m, -2));
-  HDB_CALL(fill_i32(ctx, leaf_par, n, -2));
-  hipLaunchKernelGGL(k_tr_nodes, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, edges, m, n, top, sz, left, right,
-                     nsize, par, leaf_par, lam, bad);
+  // ---- linkage tree, node classes, depth / preorder / cluster starts
+  uint8_t* flags;
+  TrRec *rec, *rec2;
+  HDB_CALL(scratch_t(ctx, kSlotMstFlag, m, &flags));
+  HDB_CALL(scratch_t(ctx, kSlotMstWl1, 2 * m, &rec));
+  rec2 = rec + m;
+  hipLaunchKernelGGL(k_tr_nodes, dim3(gm), dim3(256), 0, ctx->stream, edges, m, n, top, sz, left, right, nsize, par,
+                     leaf_par, lam, bad);
   HDB_LAUNCHED();
-  hipLaunchKernelGGL(k_tr_check, dim3(grid_for(n + m, 256)), dim3(256), 0, ctx->stream, m, n, par, leaf_par, bad);
+  hipLaunchKernelGGL(k_tr_classify, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, m, n, mpts, left, right, nsize,
+                     par, leaf_par, flags, cnt, rec, splits, nsplit, bad);
   HDB_LAUNCHED();
-  int32_t* more_h = reinterpret_cast<int32_t*>(ctx->pinned + 4);
-  HDB_HIP(hipMemcpyAsync(more_h, bad, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
-  HDB_HIP(hipStreamSynchronize(ctx->stream));
-  if (*more_h) return ctx->fail(HDB_EDEVICE, "inconsistent linkage tree");
-  hipLaunchKernelGGL(k_tr_classify, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, m, n, mpts, left, right, nsize,
-                     par, proc, split, cnt, anc, dsum, psum, cs);
-  HDB_LAUNCHED();
-  // depth and preorder: pointer jumping with sums
-  for (int round = 0; round < 64; ++round) {
-    HDB_CALL(fill_i32(ctx, more, 1, 0));
-    hipLaunchKernelGGL(k_tr_jump_sums, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, m, anc, dsum, psum, anc2,
-                       dsum2, psum2, more);
+  // the controls come back while the jumps run: a node is at most m - 1
+  // deep, so bits_for(m - 1) rounds reach the root from everywhere
+  static_assert(2 * sizeof(int32_t) == sizeof(int64_t), "both controls in one word");
+  HDB_CALL(read_i64_async(ctx, reinterpret_cast<const int64_t*>(ctrl), 0));
+  for (int round = 0; round < L; ++round) {
+    hipLaunchKernelGGL(k_tr_jump, dim3(gm), dim3(256), 0, ctx->stream, m, rec, rec2);
     HDB_LAUNCHED();
-    std::swap(anc, anc2);
-    std::swap(dsum, dsum2);
-    std::swap(psum, psum2);
-    HDB_HIP(hipMemcpyAsync(more_h, more, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
-    HDB_HIP(hipStreamSynchronize(ctx->stream));
-    if (!*more_h) break;
+    std::swap(rec, rec2);
   }
-  if (*more_h) return ctx->fail(HDB_EDEVICE, "pointer jumping did not converge");
-  // the jumps above leave depth in dsum and preorder in psum
-  const int64_t* depth = dsum;
-  const int64_t* pre = psum;
-  // cluster start of every node
-  for (int round = 0; round < 64; ++round) {
-    HDB_CALL(fill_i32(ctx, more, 1, 0));
-    hipLaunchKernelGGL(k_tr_jump_cs, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, m, cs, cs2, more);
-    HDB_LAUNCHED();
-    std::swap(cs, cs2);
-    HDB_HIP(hipMemcpyAsync(more_h, more, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
-    HDB_HIP(hipStreamSynchronize(ctx->stream));
-    if (!*more_h) break;
-  }
-  if (*more_h) return ctx->fail(HDB_EDEVICE, "pointer jumping did not converge");
-  // the node each point leaves at
-  hipLaunchKernelGGL(k_tr_up_init, dim3(grid_for(n + m, 256)), dim3(256), 0, ctx->stream, m, n, par, leaf_par, proc,
-                     up);
-  HDB_LAUNCHED();
-  for (int round = 0; round < 64; ++round) {
-    HDB_CALL(fill_i32(ctx, more, 1, 0));
-    hipLaunchKernelGGL(k_tr_up_jump, dim3(grid_for(n + m, 256)), dim3(256), 0, ctx->stream, n + m, up, up2, more);
-    HDB_LAUNCHED();
-    std::swap(up, up2);
-    HDB_HIP(hipMemcpyAsync(more_h, more, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
-    HDB_HIP(hipStreamSynchronize(ctx->stream));
-    if (!*more_h) break;
-  }
-  if (*more_h) return ctx->fail(HDB_EDEVICE, "pointer jumping did not converge");
+  int64_t both = 0;
+  HDB_CALL(wait_i64(ctx, 0, &both));
+  if (static_cast<int32_t>(both) != 0) return ctx->fail(HDB_EDEVICE, "inconsistent linkage tree");
+  const int64_t S2 = both >> 32;
   // ---- splits in level order -> cluster ids
-  int32_t *flag32 = cur.uf, *pflag32 = cur.rep_l;  // the linkage's arrays are dead by now
-  int64_t *spos, *ppos;
-  HDB_CALL(scratch_t(ctx, kSlotRowTmp, 2 * (m + 1), &spos));
-  ppos = spos + (m + 1);
-  hipLaunchKernelGGL(k_u8_to_i32, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, split, m, flag32);
-  HDB_LAUNCHED();
-  hipLaunchKernelGGL(k_u8_to_i32, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, proc, m, pflag32);
-  HDB_LAUNCHED();
-  HDB_CALL(scan_i32_to_i64(ctx, flag32, m, spos));
-  HDB_CALL(scan_i32_to_i64(ctx, pflag32, m, ppos));
-  int64_t S2 = 0, P = 0;
-  HDB_CALL(read_i64(ctx, spos + m, &S2));
-  HDB_CALL(read_i64(ctx, ppos + m, &P));
-  const int64_t S = 1 + 2 * S2;  // clusters
-  if (S2 > 0) {
-    hipLaunchKernelGGL(k_tr_split_keys, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, m, split, depth, pre, spos,
-                       keys, vals);
+  if (S2 > kSplitSmall) {
+    uint64_t* keys;
+    uint32_t* vals;
+    HDB_CALL(scratch_t(ctx, kSlotRowCursor, S2, &keys));
+    HDB_CALL(scratch_t(ctx, kSlotMisc2, S2, &vals));
+    const unsigned gs = grid_for(S2, 256);
+    hipLaunchKernelGGL(k_tr_split_keys, dim3(gs), dim3(256), 0, ctx->stream, S2, splits, rec, keys, vals);
     HDB_LAUNCHED();
-    HDB_CALL(radix_sort_u64_u32(ctx, keys, vals, S2, 0, 64));
-    hipLaunchKernelGGL(k_tr_split_rank, dim3(grid_for(S2, 256)), dim3(256), 0, ctx->stream, S2, vals, srank);
+    HDB_CALL(radix_sort_u64_u32(ctx, keys, vals, S2, 0, bits_for(2 * n)));
+    HDB_CALL(radix_sort_u64_u32(ctx, keys, vals, S2, 32, 32 + bits_for(m - 1)));
+    hipLaunchKernelGGL(k_tr_split_rank, dim3(gs), dim3(256), 0, ctx->stream, S2, vals, srank);
+    HDB_LAUNCHED();
+  } else if (S2 > 0) {
+    hipLaunchKernelGGL(k_tr_split_rank_small, dim3(1), dim3(1024), 0, ctx->stream, static_cast<int>(S2), splits, rec,
+                       srank);
     HDB_LAUNCHED();
   }
-  float *birth, *stab;
-  int32_t *cparent, *clab;
-  float* cbirth;
-  int64_t *cbeg, *cend;
-  HDB_CALL(scratch_t(ctx, kSlotMstCw, 6 * S + 64, &birth));
+  const int64_t S = 1 + 2 * S2;  // clusters
+  float *birth, *stab, *cbirth;
+  int32_t *cparent, *clab, *clen, *na;
+  int64_t *cbeg, *aoff;
+  float* add;
+  HDB_CALL(scratch_t(ctx, kSlotMstCw, 6 * S, &birth));
   stab = birth + S;
   cparent = reinterpret_cast<int32_t*>(stab + S);
   clab = cparent + S;
   cbirth = reinterpret_cast<float*>(clab + S);
-  HDB_CALL(scratch_t(ctx, kSlotMstCnt, 2 * S, &cbeg));
-  cend = cbeg + S;
-  hipLaunchKernelGGL(k_tr_clusters, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, m, n, proc, cs, par, left, srank,
-                     lam, cid, birth, cparent);
+  clen = reinterpret_cast<int32_t*>(cbirth + S);
+  HDB_CALL(scratch_t(ctx, kSlotMstCnt, S + 1, &cbeg));
+  HDB_CALL(scratch_t(ctx, kSlotTreeAddCnt, m, &na));
+  HDB_CALL(scratch_t(ctx, kSlotTreeAddOff, m + 1, &aoff));
+  // a point leaves one cluster, and a split adds two terms
+  HDB_CALL(scratch_t(ctx, kSlotTreeAdd, n + 2 * S2, &add));
+  hipLaunchKernelGGL(k_tr_clusters, dim3(gm), dim3(256), 0, ctx->stream, m, n, mpts, flags, rec, par, left, right, nsize,
+                     srank, lam, cid, pos, birth, cparent, clen, na);
   HDB_LAUNCHED();
-  hipLaunchKernelGGL(k_tr_cparent, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, m, cs, par, cid, cparent);
-  HDB_LAUNCHED();
+  HDB_CALL(scan_i32_to_i64(ctx, clen, S, cbeg));
   // ---- stability: each cluster's nodes top-down
-  HDB_CALL(fill_u64(ctx, reinterpret_cast<uint64_t*>(cbeg), 2 * S, 0));
-  hipLaunchKernelGGL(k_tr_path_keys, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, m, cid, depth, ppos, proc, keys,
-                     vals);
+  hipLaunchKernelGGL(k_tr_addend_count, dim3(gm), dim3(256), 0, ctx->stream, m, flags, cid, pos, cbeg, cnt, na);
   HDB_LAUNCHED();
-  HDB_CALL(radix_sort_u64_u32(ctx, keys, vals, P, 0, 32 + bits_for(S)));
-  hipLaunchKernelGGL(k_tr_path_bounds, dim3(grid_for(P, 256)), dim3(256), 0, ctx->stream, P, keys, cbeg, cend);
+  HDB_CALL(scan_i32_to_i64(ctx, na, m, aoff));
+  hipLaunchKernelGGL(k_tr_addends, dim3(gm), dim3(256), 0, ctx->stream, m, n, flags, cid, pos, cbeg, cnt, lam, left,
+                     right, nsize, birth, aoff, add);
   HDB_LAUNCHED();
-  {
-    int32_t* na;
-    int64_t* aoff;
-    float* add;
-    HDB_CALL(scratch_t(ctx, kSlotTreeAddCnt, P, &na));
-    HDB_CALL(scratch_t(ctx, kSlotTreeAddOff, P + 1, &aoff));
-    hipLaunchKernelGGL(k_tr_addend_count, dim3(grid_for(P, 256)), dim3(256), 0, ctx->stream, P, vals, cnt, split, na);
+  hipLaunchKernelGGL(k_tr_stability, dim3(grid_for(S, 4)), dim3(256), 0, ctx->stream, S, cbeg, aoff, add, stab);
+  HDB_LAUNCHED();
+  if (n + 2 * S2 > kStabShort) {
+    hipLaunchKernelGGL(k_tr_stability_long, dim3(static_cast<unsigned>(std::min<int64_t>(S, 512))),
+                       dim3(kStabWaves * 64), 0, ctx->stream, S, cbeg, aoff, add, stab);
     HDB_LAUNCHED();
-    HDB_CALL(scan_i32_to_i64(ctx, na, P, aoff));
-    int64_t A = 0;
-    HDB_CALL(read_i64(ctx, aoff + P, &A));
-    HDB_CALL(scratch_t(ctx, kSlotTreeAdd, A > 0 ? A : 1, &add));
-    hipLaunchKernelGGL(k_tr_addends, dim3(grid_for(P, 256)), dim3(256), 0, ctx->stream, P, n, keys, vals, cnt, split,
-                       lam, left, right, nsize, birth, aoff, add);
-    HDB_LAUNCHED();
-    hipLaunchKernelGGL(k_tr_stability, dim3(grid_for(S, 4)), dim3(256), 0, ctx->stream, S, cbeg, cend, aoff, add,
-                       stab);
-    HDB_LAUNCHED();
-    if (A > kStabShort) {
-      hipLaunchKernelGGL(k_tr_stability_long, dim3(static_cast<unsigned>(std::min<int64_t>(S, 512))),
-                         dim3(kStabWaves * 64), 0, ctx->stream, S, cbeg, cend, aoff, add, stab);
-      HDB_LAUNCHED();
-    }
   }
   // ---- EOM selection over the cluster tree (host; one entry per cluster)
-  std::vector<float> h_stab(S), h_birth(S);
-  std::vector<int32_t> h_par(S);
-  HDB_HIP(hipMemcpyAsync(h_stab.data(), stab, S * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-  HDB_HIP(hipMemcpyAsync(h_birth.data(), birth, S * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-  HDB_HIP(hipMemcpyAsync(h_par.data(), cparent, S * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+  std::vector<float> h_in(3 * S);  // birth, stability and parent, adjacent on the device
+  HDB_HIP(hipMemcpyAsync(h_in.data(), birth, 3 * S * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
   HDB_HIP(hipStreamSynchronize(ctx->stream));
+  const float* h_birth = h_in.data();
+  float* h_stab = h_in.data() + S;
+  std::vector<int32_t> h_par(S);
+  std::memcpy(h_par.data(), h_in.data() + 2 * S, S * sizeof(int32_t));
   // cluster c's children are the two clusters its bottom split starts: for
   // c > 0 their ids are c's split rank's 1 + 2k, 2 + 2k; descending ids put
   // children before parents (a split starts clusters after its own)
@@ -971,17 +917,16 @@ int labels_gpu(hdb_ctx* ctx, const hdb_mst_edge* edges, int64_t m, int64_t n, in
   int32_t nsel = 0;
   for (int64_t c = 1; c < S; ++c)
     if (sel[c]) cmap[c] = nsel++;
-  std::vector<int32_t> h_clab(S);
-  std::vector<float> h_cbirth(S);
+  std::vector<int32_t> h_out(2 * S);  // label and birth of the selected ancestor
   for (int64_t c = 0; c < S; ++c) {
     const int32_t a = sel_anc[c];
-    h_clab[c] = a >= 0 ? cmap[a] : -1;
-    h_cbirth[c] = a >= 0 ? h_birth[a] : 0.0f;
+    const float bl = a >= 0 ? h_birth[a] : 0.0f;
+    h_out[c] = a >= 0 ? cmap[a] : -1;
+    std::memcpy(&h_out[S + c], &bl, sizeof(bl));
   }
-  HDB_HIP(hipMemcpyAsync(clab, h_clab.data(), S * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
-  HDB_HIP(hipMemcpyAsync(cbirth, h_cbirth.data(), S * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-  hipLaunchKernelGGL(k_tr_label, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, n, up, leaf_par, par, cid, lam,
-                     clab, cbirth, labels);
+  HDB_HIP(hipMemcpyAsync(clab, h_out.data(), 2 * S * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
+  hipLaunchKernelGGL(k_tr_label, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, n, leaf_par, flags, rec, par, cid,
+                     lam, clab, cbirth, labels);
   HDB_LAUNCHED();
   HDB_HIP(hipStreamSynchronize(ctx->stream));  // the host vectors above are sources of the copies
   if (clusters_out) *clusters_out = nsel;
