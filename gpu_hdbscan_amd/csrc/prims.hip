@@ -1,5 +1,7 @@
 // Device primitives for gfx950: fills, int32->int64 exclusive scan and a
 // stable LSD radix sort (8-bit digits, wave64 match-based ranking).
+#include <utility>
+
 #include "hdb_internal.hpp"
 
 namespace hdb {
@@ -154,14 +156,11 @@ int scan_i32_to_i64(hdb_ctx* ctx, const int32_t* in, int64_t n, int64_t* out) {
 }
 
 // ----------------------------------------------------------- radix sort --
-// Tile = 4 waves x 32 chunks x 64 lanes = 8192 keys.  Within a wave, chunk c
+// A tile is WAVES waves x CH chunks x 64 lanes.  Within a wave, chunk c
 // holds keys [wave_base + 64c, wave_base + 64c + 64), one per lane, so the
 // rank order (chunk, lane) is the input order and the sort is stable.
-constexpr int kRsBlock = 256;
-constexpr int kRsChunks = 32;
-constexpr int kRsWaveKeys = 64 * kRsChunks;
-constexpr int kRsTile = kRsBlock * kRsChunks;
 constexpr int kRsBins = 256;
+constexpr int64_t kRsSmallKeys = 400000;
 
 // Input read through a segment map: logical index i lives in segment g with
 // pre[g] <= i < pre[g+1], at physical index g * seg_cap + (i - pre[g]).
@@ -227,67 +226,119 @@ __device__ __forceinline__ int64_t rs_walk_phys(const RsSegs& sg, const int64_t*
 // SEG: the input is read through a segment map (the first pass of a
 // segmented sort); otherwise logical and physical indices agree and the
 // chunk addresses are not kept in registers.
-template <typename K, bool SEG>
-__global__ __launch_bounds__(kRsBlock) void k_rs_hist(const K* __restrict__ keys, int64_t n, int shift,
-                                                      int64_t ntiles, int32_t* __restrict__ hist, RsSegs sg) {
+template <typename K, bool SEG, int WAVES, int CH>
+__global__ __launch_bounds__(WAVES * 64) void k_rs_hist(const K* __restrict__ keys, int64_t n, int shift,
+                                                        int32_t* __restrict__ hist, RsSegs sg) {
+  constexpr int kBlock = WAVES * 64;
   __shared__ int32_t h[kRsBins];
-  __shared__ int64_t s_pre[kRsMaxSegs + 1];
-  for (int i = threadIdx.x; i < kRsBins; i += kRsBlock) h[i] = 0;
-  rs_load_segs(sg, s_pre);
+  __shared__ int64_t s_pre[SEG ? kRsMaxSegs + 1 : 1];
+  for (int i = threadIdx.x; i < kRsBins; i += kBlock) h[i] = 0;
+  if (SEG) rs_load_segs(sg, s_pre);
   __syncthreads();
   const unsigned lane = __lane_id();
-  const int64_t wbase = static_cast<int64_t>(blockIdx.x) * kRsTile + static_cast<int64_t>(threadIdx.x >> 6) * kRsWaveKeys;
+  const int64_t wbase = (static_cast<int64_t>(blockIdx.x) * WAVES + (threadIdx.x >> 6)) * (64 * CH);
   // every chunk's load is issued before the first is used
-  K kv[kRsChunks];
+  K kv[CH];
   if (SEG) {
-    int64_t ph[kRsChunks];
+    int64_t ph[CH];
     RsWalk wk = rs_walk_begin(sg, s_pre, wbase < n ? wbase : 0);
 #pragma unroll
-    for (int c = 0; c < kRsChunks; ++c) {
+    for (int c = 0; c < CH; ++c) {
       const int64_t c0 = wbase + c * 64;
       ph[c] = c0 + lane < n ? rs_walk_phys(sg, s_pre, wk, c0, lane) : 0;
     }
 #pragma unroll
-    for (int c = 0; c < kRsChunks; ++c) kv[c] = keys[ph[c]];
+    for (int c = 0; c < CH; ++c) kv[c] = keys[ph[c]];
   } else {
     const K* kw = keys + wbase + lane;
 #pragma unroll
-    for (int c = 0; c < kRsChunks; ++c) kv[c] = wbase + c * 64 + lane < n ? kw[c * 64] : K(0);
+    for (int c = 0; c < CH; ++c) kv[c] = wbase + c * 64 + lane < n ? kw[c * 64] : K(0);
   }
 #pragma unroll
-  for (int c = 0; c < kRsChunks; ++c)
+  for (int c = 0; c < CH; ++c)
     if (wbase + c * 64 + lane < n) atomicAdd(&h[static_cast<unsigned>(kv[c] >> shift) & 0xFFu], 1);
   __syncthreads();
   // tile-major: the block's 256 counts are one contiguous 1 KB row
-  for (int i = threadIdx.x; i < kRsBins; i += kRsBlock) hist[static_cast<int64_t>(blockIdx.x) * kRsBins + i] = h[i];
+  for (int i = threadIdx.x; i < kRsBins; i += kBlock) hist[static_cast<int64_t>(blockIdx.x) * kRsBins + i] = h[i];
 }
 
-// Digit offsets from the tile-major counts H[t][d] (ntiles x 256):
-// O[t][d] = sum over d' < d of the digit totals + sum over t' < t of H[t'][d].
-// Tiles are taken in ranges of kRsColRows; every access to H and O is a
-// contiguous row, and only the per-range partials Q[d][b] (digit-major) are
-// read across rows.
-constexpr int kRsColRows = 16;
+// Digit offsets from the tile-major counts H[t][d] (ntiles x 256): tiles are
+// taken in ranges; H[t][d] is replaced by the sum over the earlier tiles of
+// its range (32 bits), base[b][d] is the sum over the earlier ranges, tot[d]
+// the digit's total.  The scatter adds the three (the digits' starts are a
+// scan of tot).  Every access but the transposed writes of base is a
+// contiguous row, and a tile costs 4 KB of traffic.
+//
+// Up to kRsColTiles tiles are one range and one launch: a block per 16
+// digits (a 64-byte piece of every row), thread (r, d) takes a run of tiles
+// and the runs' sums are scanned in LDS.
+constexpr int64_t kRsColTiles = 2048;
+constexpr int kRsColDigits = 16;
+
+__global__ __launch_bounds__(1024) void k_rs_col_small(int32_t* __restrict__ hist, int ntiles,
+                                                       int64_t* __restrict__ base, int64_t* __restrict__ tot) {
+  __shared__ int32_t s_sum[64][kRsColDigits + 1];
+  const int dl = static_cast<int>(threadIdx.x) & (kRsColDigits - 1);
+  const int d = static_cast<int>(blockIdx.x) * kRsColDigits + dl;
+  const int r = static_cast<int>(threadIdx.x) / kRsColDigits;  // run 0..63
+  const int per = (ntiles + 63) / 64;
+  const int t0 = r * per, t1 = t0 + per < ntiles ? t0 + per : ntiles;
+  int32_t s = 0;  // 2048 tiles of at most 5120 keys fit
+#pragma unroll 4
+  for (int t = t0; t < t1; ++t) s += hist[t * kRsBins + d];
+  s_sum[r][dl] = s;
+  __syncthreads();
+  // wave w scans digit w of the block: lane = run
+  const int lane = static_cast<int>(__lane_id()), w = static_cast<int>(threadIdx.x >> 6);
+  const int32_t v = s_sum[lane][w];
+  int32_t incl = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int32_t y = __shfl_up(incl, o);
+    if (lane >= o) incl += y;
+  }
+  s_sum[lane][w] = incl - v;
+  if (lane == 63) {
+    tot[blockIdx.x * kRsColDigits + w] = incl;
+    base[blockIdx.x * kRsColDigits + w] = 0;
+  }
+  __syncthreads();
+  int32_t run = s_sum[r][dl];
+#pragma unroll 4
+  for (int t = t0; t < t1; ++t) {
+    const int32_t h = hist[t * kRsBins + d];
+    hist[t * kRsBins + d] = run;
+    run += h;
+  }
+}
+
+// More tiles: ranges of kRsColRows.
+constexpr int kRsColRows = 32;
 static_assert(kRsBins == kScanBlock, "one thread per digit in the column scans");
 
-// Q[d][b] = sum of H[t][d] over the tiles t of range b.
-__global__ __launch_bounds__(kRsBins) void k_rs_col_sum(const int32_t* __restrict__ hist, int64_t ntiles,
-                                                        int64_t nrange, int64_t* __restrict__ q) {
+// H of range b to running sums; Q[d][b] = the range's total of digit d.
+__global__ __launch_bounds__(kRsBins) void k_rs_col_sum(int32_t* __restrict__ hist, int64_t ntiles, int64_t nrange,
+                                                        int32_t* __restrict__ q) {
   const int d = static_cast<int>(threadIdx.x);
   const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kRsColRows;
-  int64_t s = 0;
+  int32_t h[kRsColRows];
 #pragma unroll
-  for (int r = 0; r < kRsColRows; ++r)
-    if (t0 + r < ntiles) s += hist[(t0 + r) * kRsBins + d];
-  q[static_cast<int64_t>(d) * nrange + blockIdx.x] = s;
+  for (int r = 0; r < kRsColRows; ++r) h[r] = t0 + r < ntiles ? hist[(t0 + r) * kRsBins + d] : 0;
+  int32_t run = 0;
+#pragma unroll
+  for (int r = 0; r < kRsColRows; ++r) {
+    if (t0 + r < ntiles) hist[(t0 + r) * kRsBins + d] = run;
+    run += h[r];
+  }
+  q[static_cast<int64_t>(d) * nrange + blockIdx.x] = run;
 }
 
-// One block per digit: Q[d][.] becomes its exclusive prefix over ranges;
-// tot[d] receives the digit's total.
-__global__ __launch_bounds__(kScanBlock) void k_rs_col_scan(int64_t* __restrict__ q, int64_t nrange,
-                                                            int64_t* __restrict__ tot) {
+// One block per digit: base[.][d] = the exclusive prefix of Q[d][.] over
+// ranges; tot[d] receives the digit's total.
+__global__ __launch_bounds__(kScanBlock) void k_rs_col_scan(const int32_t* __restrict__ q, int64_t nrange,
+                                                            int64_t* __restrict__ base, int64_t* __restrict__ tot) {
   __shared__ int64_t carry_s;
-  int64_t* row = q + static_cast<int64_t>(blockIdx.x) * nrange;
+  const int32_t* row = q + static_cast<int64_t>(blockIdx.x) * nrange;
   if (threadIdx.x == 0) carry_s = 0;
   __syncthreads();
   for (int64_t start = 0; start < nrange; start += kScanBlock) {
@@ -296,7 +347,7 @@ __global__ __launch_bounds__(kScanBlock) void k_rs_col_scan(int64_t* __restrict_
     int64_t total;
     const int64_t ex = block_excl_scan(v, &total);
     const int64_t carry = carry_s;
-    if (idx < nrange) row[idx] = carry + ex;
+    if (idx < nrange) base[idx * kRsBins + blockIdx.x] = carry + ex;
     __syncthreads();
     if (threadIdx.x == 0) carry_s = carry + total;
     __syncthreads();
@@ -304,69 +355,150 @@ __global__ __launch_bounds__(kScanBlock) void k_rs_col_scan(int64_t* __restrict_
   if (threadIdx.x == 0) tot[blockIdx.x] = carry_s;
 }
 
-// O[t][d] for the tiles of range b: the digit's start (an exclusive scan of
-// tot over digits), the range's prefix Q[d][b], then a running sum over the
-// range's rows.
-__global__ __launch_bounds__(kRsBins) void k_rs_col_apply(const int32_t* __restrict__ hist, int64_t ntiles,
-                                                          int64_t nrange, const int64_t* __restrict__ q,
-                                                          const int64_t* __restrict__ tot, int64_t* __restrict__ off) {
-  const int d = static_cast<int>(threadIdx.x);
-  int64_t total;
-  int64_t run = block_excl_scan(tot[d], &total) + q[static_cast<int64_t>(d) * nrange + blockIdx.x];
-  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kRsColRows;
-  int32_t h[kRsColRows];
+// Lanes of the wave whose digit equals this lane's (active lanes only).
+__device__ __forceinline__ uint64_t rs_match(unsigned dg, bool act) {
+  uint64_t m = __ballot(act);
 #pragma unroll
-  for (int r = 0; r < kRsColRows; ++r) h[r] = t0 + r < ntiles ? hist[(t0 + r) * kRsBins + d] : 0;
+  for (int b = 0; b < 8; ++b) {
+    const bool bit = (dg >> b) & 1u;
+    const uint64_t bal = __ballot(bit);
+    m &= bit ? bal : ~bal;
+  }
+  return m;
+}
+
+// Stable ranks of one wave's CH chunks: rank[c] = keys of the same digit
+// before this one in the wave; wcnt (the wave's 256 counters, zero on entry)
+// ends as the wave's digit counts.
+template <typename K, int CH>
+__device__ __forceinline__ void rs_wave_ranks(const K (&key)[CH], int64_t wbase, int64_t n, int shift, uint16_t* wcnt,
+                                              uint8_t (&dig)[CH], int32_t (&rank)[CH]) {
+  const unsigned lane = __lane_id();
+  const uint64_t lt = lanemask_lt();
 #pragma unroll
-  for (int r = 0; r < kRsColRows; ++r) {
-    if (t0 + r < ntiles) off[(t0 + r) * kRsBins + d] = run;
-    run += h[r];
+  for (int c = 0; c < CH; ++c) {
+    const bool act = wbase + c * 64 + lane < n;
+    const unsigned dg = static_cast<unsigned>(key[c] >> shift) & 0xFFu;
+    dig[c] = static_cast<uint8_t>(dg);
+    const uint64_t m = rs_match(dg, act);
+    // Lanes of one digit: the lowest one advances the wave's digit counter.
+    const int leader = act ? __builtin_ctzll(m) : static_cast<int>(lane);
+    int32_t base = 0;
+    if (act && static_cast<int>(lane) == leader) {
+      base = wcnt[dg];
+      wcnt[dg] = static_cast<uint16_t>(base + __popcll(m));
+    }
+    base = __shfl(base, leader);
+    rank[c] = act ? base + __popcll(m & lt) : 0;
   }
 }
 
-template <typename K, typename V, bool HAS_V, bool SEG>
-__global__ __launch_bounds__(kRsBlock) void k_rs_scatter(const K* __restrict__ kin, const V* __restrict__ vin,
-                                                         K* __restrict__ kout, V* __restrict__ vout, int64_t n,
-                                                         int shift, int64_t ntiles,
-                                                         const int64_t* __restrict__ hoff, RsSegs sg) {
-  static_assert(kRsBlock == kRsBins, "one thread per digit");
-  // per-wave digit counts fit 16 bits (at most 64 * kRsChunks keys a wave)
-  __shared__ uint16_t wcnt[kRsBlock / 64][kRsBins];
-  __shared__ int64_t goff[kRsBins];
+// Per digit (the block's first 256 threads): the waves' counts become their
+// exclusive prefix in wave order; dstart[d] = the tile's start of digit d.
+// Every thread of the block calls it, after a barrier; wsum is LDS.
+template <int WAVES>
+__device__ __forceinline__ void rs_digit_starts(uint16_t (*wcnt)[kRsBins], int32_t* dstart, int32_t* wsum) {
+  const unsigned lane = __lane_id();
+  const unsigned w = threadIdx.x >> 6;
+  const int dgt = static_cast<int>(threadIdx.x);
+  int32_t tot = 0, incl = 0;
+  if (dgt < kRsBins) {
+#pragma unroll
+    for (int ww = 0; ww < WAVES; ++ww) {
+      const int32_t c = wcnt[ww][dgt];
+      wcnt[ww][dgt] = static_cast<uint16_t>(tot);
+      tot += c;
+    }
+    incl = tot;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int32_t y = __shfl_up(incl, o);
+      if (static_cast<int>(lane) >= o) incl += y;
+    }
+    if (lane == 63) wsum[w] = incl;
+  }
+  __syncthreads();
+  if (dgt < kRsBins) {
+    int32_t wpre = 0;
+    for (unsigned ww = 0; ww < w; ++ww) wpre += wsum[ww];
+    dstart[dgt] = wpre + incl - tot;
+  }
+  __syncthreads();
+}
+
+// Exclusive scan of tot over the 256 digits into s (first 256 threads).
+__device__ __forceinline__ void rs_digit_base(const int64_t* __restrict__ tot, int64_t* s, int64_t* wsum64) {
+  const unsigned lane = __lane_id();
+  const unsigned w = threadIdx.x >> 6;
+  int64_t v = 0, incl = 0;
+  if (threadIdx.x < kRsBins) {
+    v = tot[threadIdx.x];
+    incl = wave_incl_scan(v);
+    if (lane == 63) wsum64[w] = incl;
+  }
+  __syncthreads();
+  if (threadIdx.x < kRsBins) {
+    int64_t pre = 0;
+    for (unsigned ww = 0; ww < w; ++ww) pre += wsum64[ww];
+    s[threadIdx.x] = pre + incl - v;
+  }
+}
+
+template <typename K, typename V, bool HAS_V, bool SEG, int WAVES, int CH>
+__global__ __launch_bounds__(WAVES * 64) void k_rs_scatter(const K* __restrict__ kin, const V* __restrict__ vin,
+                                                           K* __restrict__ kout, V* __restrict__ vout, int64_t n,
+                                                           int shift, const int32_t* __restrict__ hist,
+                                                           const int64_t* __restrict__ base,
+                                                           const int64_t* __restrict__ tot, int range_shift, RsSegs sg,
+                                                           int64_t ntiles, int64_t per) {
+  constexpr int kBlock = WAVES * 64;
+  constexpr int kTile = kBlock * CH;
+  // Workgroups go to the eight XCDs in turn, so blocks b, b + 8, b + 16, ...
+  // share an L2: they take consecutive tiles (per of them for each XCD), and
+  // the runs consecutive tiles write for a digit, which continue each other
+  // in memory, fill their common cache lines in one L2.
+  const int64_t tile = (static_cast<int64_t>(blockIdx.x) & 7) * per + (blockIdx.x >> 3);
+  if (tile >= ntiles) return;  // uniform across the block
+  static_assert(kBlock >= kRsBins, "one thread per digit");
+  static_assert(kTile <= 65535, "tile counts fit 16 bits");
+  __shared__ uint16_t wcnt[WAVES][kRsBins];
+  __shared__ int64_t goff[kRsBins];  // global position of the tile's first key of a digit, less its tile start
   __shared__ int32_t dstart[kRsBins];
-  __shared__ int32_t wsum[kRsBlock / 64];
-  __shared__ int64_t s_pre[kRsMaxSegs + 1];
+  __shared__ int32_t wsum[4];
+  __shared__ int64_t wsum64[4];
+  __shared__ int64_t s_pre[SEG ? kRsMaxSegs + 1 : 1];
   // staging: keys first, then values, through one buffer
-  __shared__ uint64_t s_stage[kRsTile * (sizeof(K) > sizeof(V) || !HAS_V ? sizeof(K) : sizeof(V)) / 8];
+  __shared__ uint64_t s_stage[kTile * (sizeof(K) > sizeof(V) || !HAS_V ? sizeof(K) : sizeof(V)) / 8];
   K* skey = reinterpret_cast<K*>(s_stage);
   V* sval = reinterpret_cast<V*>(s_stage);
   const unsigned lane = __lane_id();
   const unsigned w = threadIdx.x >> 6;
-  for (int i = threadIdx.x; i < (kRsBlock / 64) * kRsBins; i += kRsBlock) (&wcnt[0][0])[i] = 0;
-  for (int i = threadIdx.x; i < kRsBins; i += kRsBlock) goff[i] = hoff[static_cast<int64_t>(blockIdx.x) * kRsBins + i];
-  rs_load_segs(sg, s_pre);
+  for (int i = threadIdx.x; i < WAVES * kRsBins / 2; i += kBlock) reinterpret_cast<uint32_t*>(&wcnt[0][0])[i] = 0;
+  if (SEG) rs_load_segs(sg, s_pre);
+  rs_digit_base(tot, goff, wsum64);
+  if (threadIdx.x < kRsBins)
+    goff[threadIdx.x] += base[(tile >> range_shift) * kRsBins + threadIdx.x] + hist[tile * kRsBins + threadIdx.x];
   __syncthreads();
-  const int64_t wbase = static_cast<int64_t>(blockIdx.x) * kRsTile + static_cast<int64_t>(w) * kRsWaveKeys;
-  K key[kRsChunks];
-  V val[kRsChunks];
-  int32_t rank[kRsChunks];
-  uint8_t dig[kRsChunks];
-  const uint64_t lt = lanemask_lt();
+  const int64_t wbase = (tile * WAVES + w) * (64 * CH);
+  K key[CH];
+  V val[CH];
+  int32_t rank[CH];
+  uint8_t dig[CH];
   // addresses first, then every chunk's loads back to back (no branch
   // between them), so their latencies overlap
   if (SEG) {
-    int64_t ph[kRsChunks];
+    int64_t ph[CH];
     RsWalk wk = rs_walk_begin(sg, s_pre, wbase < n ? wbase : 0);
 #pragma unroll
-    for (int c = 0; c < kRsChunks; ++c) {
+    for (int c = 0; c < CH; ++c) {
       const int64_t c0 = wbase + c * 64;
       ph[c] = c0 + lane < n ? rs_walk_phys(sg, s_pre, wk, c0, lane) : 0;
     }
 #pragma unroll
-    for (int c = 0; c < kRsChunks; ++c) key[c] = kin[ph[c]];
+    for (int c = 0; c < CH; ++c) key[c] = kin[ph[c]];
     if (HAS_V) {
 #pragma unroll
-      for (int c = 0; c < kRsChunks; ++c) val[c] = vin[ph[c]];
+      for (int c = 0; c < CH; ++c) val[c] = vin[ph[c]];
     }
   } else {
     // past n a lane reloads key n - 1 (never used); that also holds for a
@@ -374,105 +506,173 @@ __global__ __launch_bounds__(kRsBlock) void k_rs_scatter(const K* __restrict__ k
     // would otherwise run past the end of the input
     const int64_t last = n - 1 - wbase;
 #pragma unroll
-    for (int c = 0; c < kRsChunks; ++c) {
+    for (int c = 0; c < CH; ++c) {
       const int64_t o = c * 64 + lane;
       key[c] = kin[wbase + (o <= last ? o : last)];
     }
     if (HAS_V) {
 #pragma unroll
-      for (int c = 0; c < kRsChunks; ++c) {
+      for (int c = 0; c < CH; ++c) {
         const int64_t o = c * 64 + lane;
         val[c] = vin[wbase + (o <= last ? o : last)];
       }
     }
   }
-#pragma unroll
-  for (int c = 0; c < kRsChunks; ++c) {
-    const int64_t idx = wbase + c * 64 + lane;
-    const bool act = idx < n;
-    const unsigned dg = static_cast<unsigned>(key[c] >> shift) & 0xFFu;
-    dig[c] = static_cast<uint8_t>(dg);
-    uint64_t m = __ballot(act);
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const bool bit = (dg >> b) & 1u;
-      const uint64_t bal = __ballot(bit);
-      m &= bit ? bal : ~bal;
-    }
-    // Lanes of one digit: the lowest one advances the wave's digit counter.
-    const int leader = act ? __builtin_ctzll(m) : static_cast<int>(lane);
-    int32_t base = 0;
-    if (act && static_cast<int>(lane) == leader) {
-      base = wcnt[w][dg];
-      wcnt[w][dg] = static_cast<uint16_t>(base + __popcll(m));
-    }
-    base = __shfl(base, leader);
-    rank[c] = act ? base + __popcll(m & lt) : 0;
-  }
+  rs_wave_ranks<K, CH>(key, wbase, n, shift, wcnt[w], dig, rank);
   __syncthreads();
-  // Per digit (one thread each): exclusive prefix over waves in wave order,
-  // then the tile's digit starts, an exclusive scan over digits.
-  const int dgt = static_cast<int>(threadIdx.x);
-  int32_t tot = 0;
-#pragma unroll
-  for (int ww = 0; ww < kRsBlock / 64; ++ww) {
-    const int32_t c = wcnt[ww][dgt];
-    wcnt[ww][dgt] = static_cast<uint16_t>(tot);
-    tot += c;
-  }
-  int32_t incl = tot;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int32_t y = __shfl_up(incl, o);
-    if (static_cast<int>(lane) >= o) incl += y;
-  }
-  if (lane == 63) wsum[w] = incl;
-  __syncthreads();
-  int32_t wpre = 0;
-  for (unsigned ww = 0; ww < w; ++ww) wpre += wsum[ww];
-  dstart[dgt] = wpre + incl - tot;
-  __syncthreads();
+  rs_digit_starts<WAVES>(wcnt, dstart, wsum);
+  if (threadIdx.x < kRsBins) goff[threadIdx.x] -= dstart[threadIdx.x];
   // Stage the tile in LDS in digit order (keys, then values, through one
   // buffer) and write each digit's run to consecutive global positions.
-  int32_t lp[kRsChunks];
+  int32_t lp[CH];
 #pragma unroll
-  for (int c = 0; c < kRsChunks; ++c) {
+  for (int c = 0; c < CH; ++c) {
     const int64_t idx = wbase + c * 64 + lane;
     lp[c] = idx < n ? dstart[dig[c]] + wcnt[w][dig[c]] + rank[c] : -1;
     if (lp[c] >= 0) skey[lp[c]] = key[c];
   }
   __syncthreads();
-  const int64_t tbase = static_cast<int64_t>(blockIdx.x) * kRsTile;
-  const int32_t cnt = static_cast<int32_t>(n - tbase < kRsTile ? n - tbase : kRsTile);
+  const int64_t tbase = tile * kTile;
+  const int32_t cnt = static_cast<int32_t>(n - tbase < kTile ? n - tbase : kTile);
   // each thread keeps the digits of the staged positions it writes
-  // (threadIdx.x + 256 t), for the values' pass
-  uint8_t dpos[kRsChunks];
+  // (threadIdx.x + kBlock t), for the values' pass
+  uint8_t dpos[CH];
 #pragma unroll
-  for (int t = 0; t < kRsChunks; ++t) {
-    const int32_t i = static_cast<int32_t>(threadIdx.x) + t * kRsBlock;
+  for (int t = 0; t < CH; ++t) {
+    const int32_t i = static_cast<int32_t>(threadIdx.x) + t * kBlock;
     dpos[t] = 0;
     if (i < cnt) {
       const K k = skey[i];
       const unsigned dd = static_cast<unsigned>(k >> shift) & 0xFFu;
-      kout[goff[dd] + (i - dstart[dd])] = k;
+      kout[goff[dd] + i] = k;
       dpos[t] = static_cast<uint8_t>(dd);
     }
   }
   if (HAS_V) {
     __syncthreads();
 #pragma unroll
-    for (int c = 0; c < kRsChunks; ++c)
+    for (int c = 0; c < CH; ++c)
       if (lp[c] >= 0) sval[lp[c]] = val[c];
     __syncthreads();
 #pragma unroll
-    for (int t = 0; t < kRsChunks; ++t) {
-      const int32_t i = static_cast<int32_t>(threadIdx.x) + t * kRsBlock;
-      if (i < cnt) {
-        const unsigned dd = dpos[t];
-        vout[goff[dd] + (i - dstart[dd])] = sval[i];
-      }
+    for (int t = 0; t < CH; ++t) {
+      const int32_t i = static_cast<int32_t>(threadIdx.x) + t * kBlock;
+      if (i < cnt) vout[goff[dpos[t]] + i] = sval[i];
     }
   }
+}
+
+// Up to kRsOne keys: every pass in one block and one launch, the keys and
+// values in registers and reordered through LDS (a pass in three launches
+// costs 10 us at any such size).
+constexpr int kRsOneWaves = 16, kRsOneCh = 8;
+constexpr int64_t kRsOne = kRsOneWaves * 64 * kRsOneCh;
+
+template <typename K, typename V, bool HAS_V>
+__global__ __launch_bounds__(kRsOneWaves * 64) void k_rs_one(K* __restrict__ keys, V* __restrict__ vals, int n,
+                                                             int bit0, int bit1) {
+  constexpr int CH = kRsOneCh;
+  __shared__ uint16_t wcnt[kRsOneWaves][kRsBins];
+  __shared__ int32_t dstart[kRsBins];
+  __shared__ int32_t wsum[4];
+  __shared__ uint64_t s_stage[kRsOne * (sizeof(K) > sizeof(V) || !HAS_V ? sizeof(K) : sizeof(V)) / 8];
+  K* skey = reinterpret_cast<K*>(s_stage);
+  V* sval = reinterpret_cast<V*>(s_stage);
+  const int lane = static_cast<int>(__lane_id());
+  const unsigned w = threadIdx.x >> 6;
+  const int wbase = static_cast<int>(w) * 64 * CH;
+  K key[CH];
+  V val[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int i = wbase + c * 64 + lane;
+    key[c] = i < n ? keys[i] : K(0);
+    if (HAS_V) val[c] = i < n ? vals[i] : V(0);
+  }
+  for (int shift = bit0; shift < bit1; shift += 8) {
+    for (int i = threadIdx.x; i < kRsOneWaves * kRsBins / 2; i += kRsOneWaves * 64)
+      reinterpret_cast<uint32_t*>(&wcnt[0][0])[i] = 0;
+    __syncthreads();
+    uint8_t dig[CH];
+    int32_t rank[CH];
+    rs_wave_ranks<K, CH>(key, wbase, n, shift, wcnt[w], dig, rank);
+    __syncthreads();
+    rs_digit_starts<kRsOneWaves>(wcnt, dstart, wsum);
+    int32_t lp[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      lp[c] = wbase + c * 64 + lane < n ? dstart[dig[c]] + wcnt[w][dig[c]] + rank[c] : -1;
+      if (lp[c] >= 0) skey[lp[c]] = key[c];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+      if (wbase + c * 64 + lane < n) key[c] = skey[wbase + c * 64 + lane];
+    if (HAS_V) {
+      __syncthreads();
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+        if (lp[c] >= 0) sval[lp[c]] = val[c];
+      __syncthreads();
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+        if (wbase + c * 64 + lane < n) val[c] = sval[wbase + c * 64 + lane];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int i = wbase + c * 64 + lane;
+    if (i < n) {
+      keys[i] = key[c];
+      if (HAS_V) vals[i] = val[c];
+    }
+  }
+}
+
+// Scratch of one pass: tile counts, range bases, digit totals, range totals.
+struct RsWork {
+  int32_t* hist;
+  int64_t *base, *tot;
+  int32_t* q;
+};
+
+// One pass (digit at `shift`) from (ka, va) to (kb, vb).
+template <typename K, typename V, bool HAS_V, int WAVES, int CH>
+static int radix_pass(hdb_ctx* ctx, const K* ka, const V* va, K* kb, V* vb, int64_t n, int shift, const RsSegs& sp,
+                      const RsWork& wk) {
+  constexpr int kTile = WAVES * 64 * CH;
+  const int64_t ntiles = (n + kTile - 1) / kTile;
+  const dim3 grid(static_cast<unsigned>(ntiles)), block(WAVES * 64);
+  if (sp.pre)
+    hipLaunchKernelGGL((k_rs_hist<K, true, WAVES, CH>), grid, block, 0, ctx->stream, ka, n, shift, wk.hist, sp);
+  else
+    hipLaunchKernelGGL((k_rs_hist<K, false, WAVES, CH>), grid, block, 0, ctx->stream, ka, n, shift, wk.hist, sp);
+  HDB_LAUNCHED();
+  int range_shift = 62;  // one range
+  if (ntiles <= kRsColTiles) {
+    hipLaunchKernelGGL(k_rs_col_small, dim3(kRsBins / kRsColDigits), dim3(1024), 0, ctx->stream, wk.hist,
+                       static_cast<int>(ntiles), wk.base, wk.tot);
+    HDB_LAUNCHED();
+  } else {
+    static_assert(kRsColRows == 32, "range_shift");
+    range_shift = 5;
+    const int64_t nrange = (ntiles + kRsColRows - 1) / kRsColRows;
+    hipLaunchKernelGGL(k_rs_col_sum, dim3(nrange), dim3(kRsBins), 0, ctx->stream, wk.hist, ntiles, nrange, wk.q);
+    HDB_LAUNCHED();
+    hipLaunchKernelGGL(k_rs_col_scan, dim3(kRsBins), dim3(kScanBlock), 0, ctx->stream, wk.q, nrange, wk.base, wk.tot);
+    HDB_LAUNCHED();
+  }
+  const int64_t per = (ntiles + 7) / 8;  // tiles per XCD
+  const dim3 sgrid(static_cast<unsigned>(8 * per));
+  if (sp.pre)
+    hipLaunchKernelGGL((k_rs_scatter<K, V, HAS_V, true, WAVES, CH>), sgrid, block, 0, ctx->stream, ka, va, kb, vb, n,
+                       shift, wk.hist, wk.base, wk.tot, range_shift, sp, ntiles, per);
+  else
+    hipLaunchKernelGGL((k_rs_scatter<K, V, HAS_V, false, WAVES, CH>), sgrid, block, 0, ctx->stream, ka, va, kb, vb, n,
+                       shift, wk.hist, wk.base, wk.tot, range_shift, sp, ntiles, per);
+  HDB_LAUNCHED();
+  return HDB_OK;
 }
 
 // LSD radix sort of (keys, vals) by bits [bit0, bit1).  seg != nullptr: the
@@ -489,24 +689,37 @@ static int radix_sort_t(hdb_ctx* ctx, K* keys, V* vals, int64_t n, int bit0, int
     if (bit1 < bit0 + 8) bit1 = bit0 + 8;  // at least one pass gathers the segments
   }
   if (n <= 1 && !seg) bit1 = bit0;
-  if (n <= 0 || bit1 <= bit0) {
-    if (kout) *kout = keys;
-    if (vout) *vout = vals;
+  if (kout) *kout = keys;
+  if (vout) *vout = vals;
+  if (n <= 0 || bit1 <= bit0) return HDB_OK;
+  if (!seg && n <= kRsOne) {
+    hipLaunchKernelGGL((k_rs_one<K, V, HAS_V>), dim3(1), dim3(kRsOneWaves * 64), 0, ctx->stream, keys, vals,
+                       static_cast<int>(n), bit0, bit1);
+    HDB_LAUNCHED();
     return HDB_OK;
   }
-  const int64_t ntiles = (n + kRsTile - 1) / kRsTile;
+  // Blocks of 8 waves; tiles of 4096 keys, of 5120 with u64 values, which
+  // leave three or four blocks to a CU's LDS.  With the XCD-aware tile order
+  // runs of that length fill their cache lines: a pass over 320M u32 keys
+  // with u32 / u64 values takes 1.54 / 2.10 ms (4.2 / 4.3 TB/s; tiles of 8192
+  // from 4 waves in plain order 2.16 / 3.43, of 8192 from 16 waves 2.03 /
+  // 2.28, of 16384 1.77 / 3.04).  Up to kRsSmallKeys tiles of 2048, which
+  // spread few keys over more CUs (160k keys: 11.5 / 11.8 us against 13.5 /
+  // 14.4 with 4096; at 600k 15.0 / 15.4 against 15.0 / 16.1).
+  constexpr int kCh = sizeof(V) == 8 && HAS_V ? 10 : 8;
+  constexpr int64_t kTile = 8 * 64 * kCh;
+  const bool small = n <= kRsSmallKeys;
+  const int64_t ntiles = small ? (n + 2047) / 2048 : (n + kTile - 1) / kTile;
   K* k2;
   V* v2 = nullptr;
-  int32_t* hist;
-  int64_t* hoff;
+  RsWork wk;
   HDB_CALL(scratch_t(ctx, kSlotSortKeys, static_cast<size_t>(n), &k2));
   if (HAS_V) HDB_CALL(scratch_t(ctx, kSlotSortVals, static_cast<size_t>(n), &v2));
-  HDB_CALL(scratch_t(ctx, kSlotSortHist, static_cast<size_t>(kRsBins * ntiles), &hist));
-  // offsets, then the per-range partials and the digit totals
+  HDB_CALL(scratch_t(ctx, kSlotSortHist, static_cast<size_t>(kRsBins * ntiles), &wk.hist));
   const int64_t nrange = (ntiles + kRsColRows - 1) / kRsColRows;
-  HDB_CALL(scratch_t(ctx, kSlotSortAux, static_cast<size_t>(kRsBins * (ntiles + nrange + 1)), &hoff));
-  int64_t* colq = hoff + kRsBins * ntiles;
-  int64_t* coltot = colq + kRsBins * nrange;
+  HDB_CALL(scratch_t(ctx, kSlotSortAux, static_cast<size_t>(kRsBins * (1 + nrange + (nrange + 1) / 2)), &wk.tot));
+  wk.base = wk.tot + kRsBins;
+  wk.q = reinterpret_cast<int32_t*>(wk.base + kRsBins * nrange);
   K* ka = keys;
   K* kb = k2;
   V* va = vals;
@@ -514,29 +727,12 @@ static int radix_sort_t(hdb_ctx* ctx, K* keys, V* vals, int64_t n, int bit0, int
   int passes = 0;
   for (int shift = bit0; shift < bit1; shift += 8, ++passes) {
     const RsSegs sp = passes == 0 ? sg : RsSegs{nullptr, 0, 0};
-    if (sp.pre)
-      hipLaunchKernelGGL((k_rs_hist<K, true>), dim3(ntiles), dim3(kRsBlock), 0, ctx->stream, ka, n, shift, ntiles, hist,
-                         sp);
+    if (small)
+      HDB_CALL((radix_pass<K, V, HAS_V, 8, 4>(ctx, ka, va, kb, vb, n, shift, sp, wk)));
     else
-      hipLaunchKernelGGL((k_rs_hist<K, false>), dim3(ntiles), dim3(kRsBlock), 0, ctx->stream, ka, n, shift, ntiles, hist,
-                         sp);
-    HDB_LAUNCHED();
-    hipLaunchKernelGGL(k_rs_col_sum, dim3(nrange), dim3(kRsBins), 0, ctx->stream, hist, ntiles, nrange, colq);
-    HDB_LAUNCHED();
-    hipLaunchKernelGGL(k_rs_col_scan, dim3(kRsBins), dim3(kScanBlock), 0, ctx->stream, colq, nrange, coltot);
-    HDB_LAUNCHED();
-    hipLaunchKernelGGL(k_rs_col_apply, dim3(nrange), dim3(kRsBins), 0, ctx->stream, hist, ntiles, nrange, colq, coltot,
-                       hoff);
-    HDB_LAUNCHED();
-    if (sp.pre)
-      hipLaunchKernelGGL((k_rs_scatter<K, V, HAS_V, true>), dim3(ntiles), dim3(kRsBlock), 0, ctx->stream, ka, va, kb,
-                         vb, n, shift, ntiles, hoff, sp);
-    else
-      hipLaunchKernelGGL((k_rs_scatter<K, V, HAS_V, false>), dim3(ntiles), dim3(kRsBlock), 0, ctx->stream, ka, va, kb,
-                         vb, n, shift, ntiles, hoff, sp);
-    HDB_LAUNCHED();
-    K* tk = ka; ka = kb; kb = tk;
-    V* tv = va; va = vb; vb = tv;
+      HDB_CALL((radix_pass<K, V, HAS_V, 8, kCh>(ctx, ka, va, kb, vb, n, shift, sp, wk)));
+    std::swap(ka, kb);
+    std::swap(va, vb);
   }
   if (kout) {
     *kout = ka;

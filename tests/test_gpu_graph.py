@@ -196,3 +196,18 @@ def test_pipeline_blocked(ctx):
     ni, nl, w = O.mrd_csr(X, L, c, ah)
     ref, _ = O.kruskal(ni, nl, w)
     np.testing.assert_array_equal(res.edges, O.sort_edges(ref))
+
+
+@pytest.mark.parametrize("m", [2, 63, 8191, 8192, 8193, 399999, 400000, 400001, 5120 * 2048, 5120 * 2048 + 1])
+def test_sort_edges_forms(ctx, m):
+    """The radix sort at its changes of form: one block, tiles of 2048, tiles
+    of 5120, column scan in one launch or in two; stable on many ties."""
+    print(f"case: sort_edges m={m}", flush=True)
+    rng = np.random.default_rng(m)
+    e = np.empty(m, api.MST_EDGE)
+    e["from_node"] = np.arange(m)
+    e["to_node"] = rng.integers(0, 1 << 20, m)
+    w = rng.integers(0, 60000, m).astype(np.float32) * np.float32(0.375)
+    e["weight"] = np.where(rng.random(m) < 0.5, w, rng.random(m).astype(np.float32))
+    want = e[np.argsort(e["weight"], kind="stable")]
+    np.testing.assert_array_equal(api.sort_edges(ctx, e), want)
