@@ -171,21 +171,6 @@ __host__ __device__ inline uint64_t xorshift64star(uint64_t x) {
   return x * 0x2545F4914F6CDD1Dull;
 }
 
-// Squared L2 distance in FP32, accumulated in dimension order with fused
-// multiply-add.  Every distance of the kNN path goes through this one
-// formula, so the same pair always yields the same bits (the oracle uses the
-// identical formula with C fmaf).
-template <int D>
-__device__ __forceinline__ float d2_fixed(const float* __restrict__ a, const float* __restrict__ b) {
-  float acc = 0.0f;
-#pragma unroll
-  for (int k = 0; k < D; ++k) {
-    float diff = a[k] - b[k];
-    acc = __builtin_fmaf(diff, diff, acc);
-  }
-  return acc;
-}
-
 // Bits of max(x, 0) for a ranking key: a negative float (sign bit set) is a
 // negative int, so one integer max clamps it, -0 included, to +0.
 __device__ __forceinline__ uint32_t nonneg_bits(float x) {
@@ -210,6 +195,10 @@ __device__ __forceinline__ void top_insert_med3(uint32_t (&top)[K], uint32_t key
   top[0] = top[0] < key ? top[0] : key;
 }
 
+// Squared L2 distance in FP32, accumulated in dimension order with fused
+// multiply-add.  Every distance of the kNN path goes through this one
+// formula, so the same pair always yields the same bits (the oracle uses the
+// identical formula with C fmaf).
 __device__ __forceinline__ float d2_any(const float* __restrict__ a, const float* __restrict__ b, int d) {
   float acc = 0.0f;
   for (int k = 0; k < d; ++k) {

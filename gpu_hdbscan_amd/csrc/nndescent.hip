@@ -1632,32 +1632,34 @@ int nnd_blocked(hdb_ctx* ctx, const float* X, int64_t n, int d, int blocks, cons
 }
 
 // ------------------------------------------------------ brute-force kNN --
-// One wave per query; each lane scans a strided share of the points keeping
-// a sorted top-kq (kq <= 32) in registers, then the wave pops the global
-// top-kq from the 64 lane lists.
-template <int D>
+// One wave per query and point chunk (blockIdx.y); each lane scans a strided
+// share of the chunk keeping a sorted top-kq (kq <= 32) in registers, then
+// the wave pops the chunk's top-kq from the 64 lane lists into
+// part[(qi * chunks + y) * 32 + s] (kKeyMax past the last), which k_bf_merge
+// merges.  Bound by the row reads (a lane per row, 16 bytes at a time where
+// rows are 16-byte aligned): the chunks let a few queries fill the chip.  16
+// queries against 100k x 128 took 25.4 ms with one wave each, 0.4 ms split.
 __global__ __launch_bounds__(256) void k_bruteforce(const float* __restrict__ X, int64_t n, int d,
                                                     const int32_t* __restrict__ qids, int64_t m, int kq,
-                                                    int32_t* __restrict__ out_ids, float* __restrict__ out_d2) {
+                                                    int64_t csize, uint64_t* __restrict__ part) {
   const unsigned lane = __lane_id();
   const int64_t qi = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (qi >= m) return;
+  uint64_t* out = part + (qi * gridDim.y + blockIdx.y) * 32;
   const uint32_t q = static_cast<uint32_t>(qids[qi]);
-  if (static_cast<int64_t>(q) >= n) {
-    for (int r = __lane_id(); r < kq; r += 64) {
-      out_ids[qi * kq + r] = -1;
-      if (out_d2) out_d2[qi * kq + r] = __uint_as_float(0x7F800000u);
-    }
+  if (static_cast<int64_t>(q) >= n) {  // an id outside [0, n): no neighbours
+    if (lane < 32) out[lane] = kKeyMax;
     return;
   }
   uint64_t top[32];
 #pragma unroll
   for (int i = 0; i < 32; ++i) top[i] = kKeyMax;
-  const float* xq = X + static_cast<int64_t>(q) * d;
-  for (int64_t i = lane; i < n; i += 64) {
+  const int64_t c0 = static_cast<int64_t>(blockIdx.y) * csize;
+  const int64_t c1 = c0 + csize < n ? c0 + csize : n;
+  for (int64_t i = c0 + lane; i < c1; i += 64) {
     if (static_cast<uint32_t>(i) == q) continue;
-    const float d2 = D > 0 ? d2_fixed<(D > 0 ? D : 1)>(xq, X + i * d) : d2_any(xq, X + i * d, d);
-    uint64_t key = (static_cast<uint64_t>(__float_as_uint(d2)) << 32) | static_cast<uint32_t>(i);
+    uint64_t key = (static_cast<uint64_t>(__float_as_uint(point_d2(X, d, q, static_cast<uint32_t>(i)))) << 32) |
+                   static_cast<uint32_t>(i);
     if (key < top[31]) {
 #pragma unroll
       for (int s = 0; s < 32; ++s) {
@@ -1670,6 +1672,7 @@ __global__ __launch_bounds__(256) void k_bruteforce(const float* __restrict__ X,
   }
   // pop kq minima across lanes
   int head = 0;
+  uint64_t mine = kKeyMax;  // lane r ends with the r-th smallest
   for (int r = 0; r < kq; ++r) {
     uint64_t h = kKeyMax;
 #pragma unroll
@@ -1682,11 +1685,9 @@ __global__ __launch_bounds__(256) void k_bruteforce(const float* __restrict__ X,
       mn = oth < mn ? oth : mn;
     }
     if (h == mn && mn != kKeyMax) head++;
-    if (lane == 0) {
-      out_ids[qi * kq + r] = mn == kKeyMax ? -1 : static_cast<int32_t>(static_cast<uint32_t>(mn));
-      if (out_d2) out_d2[qi * kq + r] = __uint_as_float(static_cast<uint32_t>(mn >> 32));
-    }
+    if (static_cast<int>(lane) == r) mine = mn;
   }
+  if (lane < 32) out[lane] = mine;
 }
 
 // Tiled brute force for D = 12 or 32: block (g, y) holds queries
@@ -1765,8 +1766,10 @@ __global__ __launch_bounds__(256) void k_bf_tile(const float* __restrict__ X, in
 
 // One wave per query: lane l merges lists l, l + 64, ... of the query's
 // `lists` sorted 32-key lists into its own top-32, then the wave pops the
-// kq smallest keys.
+// kq smallest keys.  qids (optional): an id outside [0, n) gets infinite
+// distances.
 __global__ __launch_bounds__(256) void k_bf_merge(const uint64_t* __restrict__ part, int64_t m, int lists, int kq,
+                                                  const int32_t* __restrict__ qids, int64_t n,
                                                   int32_t* __restrict__ out_ids, float* __restrict__ out_d2) {
   const unsigned lane = __lane_id();
   const int64_t qi = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
@@ -1803,7 +1806,8 @@ __global__ __launch_bounds__(256) void k_bf_merge(const uint64_t* __restrict__ p
     if (h == mn && mn != kKeyMax) head++;
     if (lane == 0) {
       out_ids[qi * kq + r] = mn == kKeyMax ? -1 : static_cast<int32_t>(static_cast<uint32_t>(mn));
-      if (out_d2) out_d2[qi * kq + r] = __uint_as_float(static_cast<uint32_t>(mn >> 32));
+      const bool bad = qids && static_cast<int64_t>(static_cast<uint32_t>(qids[qi])) >= n;
+      if (out_d2) out_d2[qi * kq + r] = __uint_as_float(bad ? 0x7F800000u : static_cast<uint32_t>(mn >> 32));
     }
   }
 }
@@ -1866,7 +1870,7 @@ static int bruteforce_tiled(hdb_ctx* ctx, const float* X, int64_t n, const int32
                      ctx->stream, X, n, qids, m, csize, static_cast<int>(chunks), part);
   HDB_LAUNCHED();
   hipLaunchKernelGGL(k_bf_merge, dim3(grid_for(m, 4)), dim3(256), 0, ctx->stream, part, m,
-                     static_cast<int>(chunks * 4), kq, out_ids, out_d2);
+                     static_cast<int>(chunks * 4), kq, nullptr, n, out_ids, out_d2);
   HDB_LAUNCHED();
   return HDB_OK;
 }
@@ -1880,15 +1884,17 @@ int bruteforce_knn(hdb_ctx* ctx, const float* X, int64_t n, int d, const int32_t
   Stage st(ctx, "bruteforce_knn");
   if (d == 12) return bruteforce_tiled<12>(ctx, X, n, qids, m, kq, out_ids, out_d2);
   if (d == 32) return bruteforce_tiled<32>(ctx, X, n, qids, m, kq, out_ids, out_d2);
-  if (d == 12)
-    hipLaunchKernelGGL(k_bruteforce<12>, dim3(grid_for(m, 4)), dim3(256), 0, ctx->stream, X, n, d, qids, m, kq,
-                       out_ids, out_d2);
-  else if (d == 32)
-    hipLaunchKernelGGL(k_bruteforce<32>, dim3(grid_for(m, 4)), dim3(256), 0, ctx->stream, X, n, d, qids, m, kq,
-                       out_ids, out_d2);
-  else
-    hipLaunchKernelGGL(k_bruteforce<0>, dim3(grid_for(m, 4)), dim3(256), 0, ctx->stream, X, n, d, qids, m, kq,
-                       out_ids, out_d2);
+  // about 8192 waves, chunks of at least 512 points
+  int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(8192 / m, (n + 511) / 512));
+  const int64_t csize = (n + chunks - 1) / chunks;
+  chunks = (n + csize - 1) / csize;
+  uint64_t* part;
+  HDB_CALL(scratch_t(ctx, kSlotBfTmp, m * chunks * 32, &part));
+  hipLaunchKernelGGL(k_bruteforce, dim3(grid_for(m, 4), static_cast<unsigned>(chunks)), dim3(256), 0, ctx->stream, X, n,
+                     d, qids, m, kq, csize, part);
+  HDB_LAUNCHED();
+  hipLaunchKernelGGL(k_bf_merge, dim3(grid_for(m, 4)), dim3(256), 0, ctx->stream, part, m, static_cast<int>(chunks), kq,
+                     qids, n, out_ids, out_d2);
   HDB_LAUNCHED();
   return HDB_OK;
 }

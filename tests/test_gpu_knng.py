@@ -114,6 +114,22 @@ def test_bruteforce_tiled_and_bad_ids(ctx, d):
     assert sorted(ids_s[0][ids_s[0] >= 0].tolist()) == [j for j in range(20) if j != 3]
 
 
+@pytest.mark.parametrize("d", [7, 33, 128])
+@pytest.mark.parametrize("m", [1, 16, 3000])
+def test_bruteforce_point_chunks(ctx, m, d):
+    """Other dimensions split the points into chunks for few queries: one
+    chunk of all points or many ragged ones, the same exact lists."""
+    print(f"case: bruteforce {m} queries of 5003x{d}", flush=True)
+    X = datasets.tiny_blobs(5003, d, 5, seed=m + d)
+    q = np.random.default_rng(m).choice(5003, m, replace=False).astype(np.int32)
+    ids, d2 = api.bruteforce_knn(ctx, X, q, 32)
+    want, wd = O.bruteforce_fp32(X, q, 32)
+    np.testing.assert_array_equal(ids, want)
+    np.testing.assert_array_equal(d2, wd)
+    few, _ = api.bruteforce_knn(ctx, X, q, 5)
+    np.testing.assert_array_equal(few, want[:, :5])
+
+
 def test_recall_on_device_matches_oracle(ctx):
     """hdb_recall (Evaluate, tools/evaluate.hpp:13-52) equals the oracle's
     recall on the same rows, for lists of varying quality."""
