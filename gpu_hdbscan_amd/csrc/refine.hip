@@ -208,7 +208,7 @@ __global__ void k_rf_thr(const hdb_nnd_element* __restrict__ lists, const float*
 // Query index qi < m is row act[qi] (qi without act), the point of row r is
 // ptid[r] (r without ptid); blockIdx.y streams tiles [y tpc, (y + 1) tpc).
 // SYM (the first round over every point): block b streams only the tiles
-// from its own points on, and for tiles past its own points also tests the
+// from its own points on (chunk y: y tpc past them), and for tiles past its own points also tests the
 // other direction (the tile's point y against query q, with y's threshold
 // thr_y from k_rf_thr): each pair's products are formed once, which halves
 // the matrix work.  Tiles before a block's points are covered by the
@@ -233,8 +233,10 @@ __global__ __launch_bounds__(kRfThreads) void k_rf_scan(const rf_bf16x8* __restr
   const int col = static_cast<int>(lane & 15), grp = static_cast<int>(lane >> 4);
   const int64_t qb = static_cast<int64_t>(blockIdx.x) * kRfBlockQ + static_cast<int64_t>(w) * (kRfQS * 16);
   constexpr int kOwnTiles = kRfBlockQ / kRfTile;  // tiles holding the block's own points (SYM)
-  const int64_t t0 = SYM ? static_cast<int64_t>(blockIdx.x) * kOwnTiles : static_cast<int64_t>(blockIdx.y) * tpc;
-  const int64_t t1 = SYM ? ntiles : (t0 + tpc < ntiles ? t0 + tpc : ntiles);
+  const int64_t own0 = SYM ? static_cast<int64_t>(blockIdx.x) * kOwnTiles : 0;
+  const int64_t t0 = own0 + static_cast<int64_t>(blockIdx.y) * tpc;
+  const int64_t t1 = t0 + tpc < ntiles ? t0 + tpc : ntiles;
+  if (t0 >= t1) return;  // uniform across the block: a stream that ends before this chunk
 
   // query fragments and thresholds; past m the thresholds are -inf
   rf_bf16x8 bh[kRfQS][KS], bl[kRfQS][KS];
@@ -298,7 +300,6 @@ __global__ __launch_bounds__(kRfThreads) void k_rf_scan(const rf_bf16x8* __restr
     if (threadIdx.x < kRfTile) s_pn[buf][threadIdx.x] = pv;
   };
 
-  if (t0 >= t1) return;  // uniform across the block
   rf_bf16x8 nxt[kLoads];
   float npv = 0.0f, ntv = 0.0f;
   load_tile(t0, nxt, npv, ntv);
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(kRfThreads) void k_rf_scan(const rf_bf16x8* __restr
       }
     }
     rf_survivors(acc, s_pn[buf], thr, qrow, qpt, t, grp, cnt, cand);
-    if (SYM && t >= t0 + kOwnTiles) rf_reverse(acc, s_thr[buf], qn2, qpt, t, grp, cnt, cand);
+    if (SYM && t >= own0 + kOwnTiles) rf_reverse(acc, s_thr[buf], qn2, qpt, t, grp, cnt, cand);
     if (more) store_tile(buf ^ 1, nxt, npv, ntv);
     __syncthreads();
   }
@@ -571,17 +572,27 @@ __global__ void k_rf_rows_out(const hdb_nnd_element* __restrict__ rows, int64_t 
 }
 
 // thr_pt != nullptr: the symmetric first round over every point (rows are
-// the points, no active list), one block per 256 points, in order (the
-// longest streams first).
+// the points, no active list).  Its streams shrink from all tiles to none, so
+// the longest alone would set the time while the point blocks are few (100k
+// points: 391 blocks): they are cut into equal chunks for about
+// kRfSymBlocks blocks, eight for each that a CU holds at once.  From 2M
+// points on one or two chunks take the whole stream (scan at 30k x 128: 3.45 ->
+// 1.11 ms, at 100k x 128 8.9 -> 7.6 ms).
+constexpr int64_t kRfSymBlocks = 4096;
+
 template <int KS>
 int launch_scan(hdb_ctx* ctx, const __bf16* xh, const __bf16* xl, const float* pn, const hdb_nnd_element* rows,
                 int64_t n, const int32_t* ptid, const int32_t* act, int64_t m, int64_t ntiles, const float* thr_pt,
                 int32_t* cnt, int32_t* cand) {
   const int64_t qblocks = (m + kRfBlockQ - 1) / kRfBlockQ;
   if (thr_pt) {
-    hipLaunchKernelGGL((k_rf_scan<KS, true>), dim3(static_cast<unsigned>(qblocks)), dim3(kRfThreads), 0, ctx->stream,
-                       reinterpret_cast<const rf_bf16x8*>(xh), reinterpret_cast<const rf_bf16x8*>(xl), pn, rows, n,
-                       ptid, act, m, ntiles, ntiles, thr_pt, cnt, cand);
+    const int64_t steps = qblocks * (ntiles + 1) / 2;
+    const int64_t cut = std::min<int64_t>(ntiles, std::max<int64_t>(32, (steps + kRfSymBlocks - 1) / kRfSymBlocks));
+    hipLaunchKernelGGL((k_rf_scan<KS, true>),
+                       dim3(static_cast<unsigned>(qblocks), static_cast<unsigned>((ntiles + cut - 1) / cut)),
+                       dim3(kRfThreads), 0, ctx->stream, reinterpret_cast<const rf_bf16x8*>(xh),
+                       reinterpret_cast<const rf_bf16x8*>(xl), pn, rows, n, ptid, act, m, ntiles, cut, thr_pt, cnt,
+                       cand);
     HDB_LAUNCHED();
     return HDB_OK;
   }
