@@ -59,7 +59,7 @@ typedef __bf16 rf_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float rf_f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kRfCap = 128;    // survivors kept per query (two per lane in the re-rank)
-constexpr int kRfQS = 2;       // 16-query sub-tiles per wave
+constexpr int kRfQS = 2;       // 16-query sub-tiles per wave (the survivor masks' layout)
 constexpr int kRfWaves = 8;    // waves per block: 8 x 32 = 256 queries share each tile
 constexpr int kRfThreads = kRfWaves * 64;
 constexpr int kRfBlockQ = kRfWaves * kRfQS * 16;
@@ -105,13 +105,84 @@ __global__ void k_rf_norms(const float* __restrict__ X, int64_t n, int d, int64_
   pn[i] = s;
 }
 
+// A wave's queue of survivors in LDS.  A survivor costs an atomic on its
+// row's count, whose result the wave has to wait for; at 100k points every
+// tile holds one or two, and a wait for each left the matrix cores idle most
+// of the time.  Survivors are queued instead and 64 at a time take their
+// atomics together, one wait for all.  An entry is (row | tag << 24, id):
+// rows are below 2^24; the tag is the query's place in the wave (0..31), or
+// kRfNoTag for a reverse survivor.
+constexpr int kRfQueue = 128;
+constexpr uint32_t kRfNoTag = 0xFFu;
+
+struct RfQueue {
+  uint32_t* row;   // this wave's kRfQueue entries
+  int32_t* id;
+  uint32_t* stop;  // this wave's queries past the cap, a bit each
+  int len;         // wave-uniform, below 64 between pushes
+};
+
+__device__ __forceinline__ void rf_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sends the first `k` (at most 64) entries to their rows' candidates and
+// moves the rest to the front.  A row past the cap takes no more; its
+// query's bit is set in `stop`.
+__device__ __forceinline__ void rf_flush(RfQueue& qu, int k, int32_t* __restrict__ cnt, int32_t* __restrict__ cand) {
+  const int lane = static_cast<int>(__lane_id());
+  rf_wave_sync();
+  if (lane < k) {
+    const uint32_t e = qu.row[lane];
+    const int64_t r = e & 0xFFFFFFu;
+    const int slot = atomicAdd(cnt + r, 1);
+    if (slot < kRfCap) cand[r * kRfCap + slot] = qu.id[lane];
+    else if ((e >> 24) != kRfNoTag) atomicOr(qu.stop, 1u << (e >> 24));
+  }
+  const int rest = qu.len - k;
+  uint32_t r = 0;
+  int32_t i = 0;
+  if (lane < rest) {
+    r = qu.row[k + lane];
+    i = qu.id[k + lane];
+  }
+  rf_wave_sync();
+  if (lane < rest) {
+    qu.row[lane] = r;
+    qu.id[lane] = i;
+  }
+  qu.len = rest;
+}
+
+// Queues every set bit of each lane's mask; entry(bit, &row, &id) names it.
+template <typename F>
+__device__ __forceinline__ void rf_push(RfQueue& qu, uint32_t mask, F entry, int32_t* __restrict__ cnt,
+                                        int32_t* __restrict__ cand) {
+  while (true) {
+    const uint64_t bal = __ballot(mask != 0);
+    if (!bal) return;  // uniform
+    if (mask) {
+      uint32_t row;
+      int32_t id;
+      entry(__builtin_ctz(mask), &row, &id);
+      const int at = qu.len + __popcll(bal & lanemask_lt());
+      qu.row[at] = row;
+      qu.id[at] = id;
+      mask &= mask - 1;
+    }
+    qu.len += __popcll(bal);
+    if (qu.len >= 64) rf_flush(qu, 64, cnt, cand);
+  }
+}
+
 // Survivors of one 64-point tile t for the wave's 32 query rows: lane l
 // holds |y|^2 - 2 x.y for points 16 r + 4 (l / 16) + q of the tile and query
-// sub-tile s; a survivor's id goes to its row's candidates (one atomic on
-// the row's count).  Past the cap a row stops collecting in this lane.
+// sub-tile s; bit 8 r + 4 s + q of a lane's mask is that pair.
 __device__ __forceinline__ void rf_survivors(const rf_f32x4 (&acc)[4][kRfQS], const float* s_pn,
-                                             float (&thr)[kRfQS], const int64_t (&qrow)[kRfQS],
-                                             const int64_t (&qpt)[kRfQS], int64_t t, int grp,
+                                             const float (&thr)[kRfQS], const int64_t (&qrow)[kRfQS],
+                                             const int64_t (&qpt)[kRfQS], int64_t t, int grp, int col, RfQueue& qu,
                                              int32_t* __restrict__ cnt, int32_t* __restrict__ cand) {
   float4 p4[4];
 #pragma unroll
@@ -126,7 +197,8 @@ __device__ __forceinline__ void rf_survivors(const rf_f32x4 (&acc)[4][kRfQS], co
       any |= __builtin_fmaf(-2.0f, acc[r][s][2], p4[r].z) < thr[s];
       any |= __builtin_fmaf(-2.0f, acc[r][s][3], p4[r].w) < thr[s];
     }
-  if (!__ballot(any)) return;  // rare once past a query's first tiles: wave-uniform
+  if (!__ballot(any)) return;  // wave-uniform
+  uint32_t mask = 0;
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -134,15 +206,23 @@ __device__ __forceinline__ void rf_survivors(const rf_f32x4 (&acc)[4][kRfQS], co
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const float pq = q == 0 ? p4[r].x : q == 1 ? p4[r].y : q == 2 ? p4[r].z : p4[r].w;
-        if (__builtin_fmaf(-2.0f, acc[r][s][q], pq) < thr[s]) {
-          const int64_t pid = t * kRfTile + r * 16 + grp * 4 + q;
-          if (pid != qpt[s]) {
-            const int slot = atomicAdd(cnt + qrow[s], 1);
-            if (slot < kRfCap) cand[qrow[s] * kRfCap + slot] = static_cast<int32_t>(pid);
-            else thr[s] = -__uint_as_float(0x7F800000u);
-          }
-        }
+        mask |= __builtin_fmaf(-2.0f, acc[r][s][q], pq) < thr[s] ? 1u << (8 * r + 4 * s + q) : 0u;
       }
+  // the query itself is no neighbour: its bit is cleared
+  const int64_t first = t * kRfTile + grp * 4;
+#pragma unroll
+  for (int s = 0; s < kRfQS; ++s) {
+    const int64_t o = qpt[s] - first;  // 16 r + q for the lane that holds it
+    if (o >= 0 && o < kRfTile && (o & 15) < 4) mask &= ~(1u << (8 * (o >> 4) + 4 * s + (o & 15)));
+  }
+  rf_push(
+      qu, mask,
+      [&](int bit, uint32_t* row, int32_t* id) {
+        const int s = (bit >> 2) & 1;
+        *row = static_cast<uint32_t>(s ? qrow[1] : qrow[0]) | (static_cast<uint32_t>(16 * s + col) << 24);
+        *id = static_cast<int32_t>(first + 16 * (bit >> 3) + (bit & 3));
+      },
+      cnt, cand);
 }
 
 // The other direction of a tile (SYM): point y = 16 r + 4 (l / 16) + q of
@@ -150,7 +230,8 @@ __device__ __forceinline__ void rf_survivors(const rf_f32x4 (&acc)[4][kRfQS], co
 // are points here (the first round over every point).
 __device__ __forceinline__ void rf_reverse(const rf_f32x4 (&acc)[4][kRfQS], const float* s_thr,
                                            const float (&qn)[kRfQS], const int64_t (&qpt)[kRfQS], int64_t t,
-                                           int grp, int32_t* __restrict__ cnt, int32_t* __restrict__ cand) {
+                                           int grp, RfQueue& qu, int32_t* __restrict__ cnt,
+                                           int32_t* __restrict__ cand) {
   float4 t4[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) t4[r] = *reinterpret_cast<const float4*>(&s_thr[r * 16 + grp * 4]);
@@ -165,6 +246,7 @@ __device__ __forceinline__ void rf_reverse(const rf_f32x4 (&acc)[4][kRfQS], cons
       any |= __builtin_fmaf(-2.0f, acc[r][s][3], qn[s]) < t4[r].w;
     }
   if (!__ballot(any)) return;
+  uint32_t mask = 0;
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -172,12 +254,16 @@ __device__ __forceinline__ void rf_reverse(const rf_f32x4 (&acc)[4][kRfQS], cons
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const float tq = q == 0 ? t4[r].x : q == 1 ? t4[r].y : q == 2 ? t4[r].z : t4[r].w;
-        if (__builtin_fmaf(-2.0f, acc[r][s][q], qn[s]) < tq) {
-          const int64_t pid = t * kRfTile + r * 16 + grp * 4 + q;
-          const int slot = atomicAdd(cnt + pid, 1);
-          if (slot < kRfCap) cand[pid * kRfCap + slot] = static_cast<int32_t>(qpt[s]);
-        }
+        mask |= __builtin_fmaf(-2.0f, acc[r][s][q], qn[s]) < tq ? 1u << (8 * r + 4 * s + q) : 0u;
       }
+  const int64_t first = t * kRfTile + grp * 4;
+  rf_push(
+      qu, mask,
+      [&](int bit, uint32_t* row, int32_t* id) {
+        *row = static_cast<uint32_t>(first + 16 * (bit >> 3) + (bit & 3)) | (kRfNoTag << 24);
+        *id = static_cast<int32_t>(((bit >> 2) & 1) ? qpt[1] : qpt[0]);
+      },
+      cnt, cand);
 }
 
 // Threshold of every point as a query (SYM's reverse tests): tau + delta -
@@ -228,8 +314,12 @@ __global__ __launch_bounds__(kRfThreads) void k_rf_scan(const rf_bf16x8* __restr
   __shared__ __attribute__((aligned(16))) __bf16 s_l[2][kRfTile * RS];
   __shared__ __attribute__((aligned(16))) float s_pn[2][kRfTile];
   __shared__ __attribute__((aligned(16))) float s_thr[SYM ? 2 : 1][SYM ? kRfTile : 4];
+  __shared__ uint32_t s_qrow[kRfWaves][kRfQueue], s_stop[kRfWaves];
+  __shared__ int32_t s_qid[kRfWaves][kRfQueue];
   const unsigned lane = __lane_id();
   const unsigned w = threadIdx.x >> 6;
+  RfQueue qu{s_qrow[w], s_qid[w], &s_stop[w], 0};
+  if (threadIdx.x < kRfWaves) s_stop[threadIdx.x] = 0;
   const int col = static_cast<int>(lane & 15), grp = static_cast<int>(lane >> 4);
   const int64_t qb = static_cast<int64_t>(blockIdx.x) * kRfBlockQ + static_cast<int64_t>(w) * (kRfQS * 16);
   constexpr int kOwnTiles = kRfBlockQ / kRfTile;  // tiles holding the block's own points (SYM)
@@ -332,11 +422,18 @@ __global__ __launch_bounds__(kRfThreads) void k_rf_scan(const rf_bf16x8* __restr
           acc[r][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh[s][kk], acc[r][s], 0, 0, 0);
       }
     }
-    rf_survivors(acc, s_pn[buf], thr, qrow, qpt, t, grp, cnt, cand);
-    if (SYM && t >= own0 + kOwnTiles) rf_reverse(acc, s_thr[buf], qn2, qpt, t, grp, cnt, cand);
+    {  // queries past the cap stop collecting
+      const uint32_t stop = s_stop[w];
+#pragma unroll
+      for (int s = 0; s < kRfQS; ++s)
+        if ((stop >> (16 * s + col)) & 1u) thr[s] = -__uint_as_float(0x7F800000u);
+    }
+    rf_survivors(acc, s_pn[buf], thr, qrow, qpt, t, grp, col, qu, cnt, cand);
+    if (SYM && t >= own0 + kOwnTiles) rf_reverse(acc, s_thr[buf], qn2, qpt, t, grp, qu, cnt, cand);
     if (more) store_tile(buf ^ 1, nxt, npv, ntv);
     __syncthreads();
   }
+  rf_flush(qu, qu.len, cnt, cand);
 }
 
 // FP32 form for d <= 32, where the split-BF16 bound (relative to |x| |y|)
@@ -369,8 +466,12 @@ __global__ __launch_bounds__(kRfThreads) void k_rf_scan32(const float* __restric
   static_assert(kChunks <= kRfThreads, "one chunk per thread");
   __shared__ float s_x[2][kRfTile * RSF];
   __shared__ __attribute__((aligned(16))) float s_pn[2][kRfTile];
+  __shared__ uint32_t s_qrow[kRfWaves][kRfQueue], s_stop[kRfWaves];
+  __shared__ int32_t s_qid[kRfWaves][kRfQueue];
   const unsigned lane = __lane_id();
   const unsigned w = threadIdx.x >> 6;
+  RfQueue qu{s_qrow[w], s_qid[w], &s_stop[w], 0};
+  if (threadIdx.x < kRfWaves) s_stop[threadIdx.x] = 0;
   const int col = static_cast<int>(lane & 15), grp = static_cast<int>(lane >> 4);
   const int64_t qb = static_cast<int64_t>(blockIdx.x) * kRfBlockQ + static_cast<int64_t>(w) * (kRfQS * 16);
   const int64_t t0 = static_cast<int64_t>(blockIdx.y) * tpc;
@@ -450,10 +551,17 @@ __global__ __launch_bounds__(kRfThreads) void k_rf_scan32(const float* __restric
         for (int s = 0; s < kRfQS; ++s) acc[r][s] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bq[s][kk], acc[r][s], 0, 0, 0);
       }
     }
-    rf_survivors(acc, s_pn[buf], thr, qrow, qpt, t, grp, cnt, cand);
+    {  // queries past the cap stop collecting
+      const uint32_t stop = s_stop[w];
+#pragma unroll
+      for (int s = 0; s < kRfQS; ++s)
+        if ((stop >> (16 * s + col)) & 1u) thr[s] = -__uint_as_float(0x7F800000u);
+    }
+    rf_survivors(acc, s_pn[buf], thr, qrow, qpt, t, grp, col, qu, cnt, cand);
     if (more) store_tile(buf ^ 1, nxt, npv);
     __syncthreads();
   }
+  rf_flush(qu, qu.len, cnt, cand);
 }
 
 // One wave per query index qi < m (row act[qi], point ptid[row]): its kept
