@@ -821,6 +821,208 @@ __global__ __launch_bounds__(kJoinWaves * 64, 8) void k_nnd_join2(const float* _
   join_emit<WPB, kSlots>(b, top64, active, my_id, lim, nc, rev_drop);
 }
 
+// FP32 join for d <= 31 other than 12 (d = 12 and 32 have k_nnd_join2): exact
+// distances, with the candidates' padded rows in LDS and the lane's own row
+// in registers (DP: d rounded up to a multiple of 4 or so; the zeros past d
+// add nothing to a distance).  As in k_nnd_join2 each old-new pair is
+// evaluated once (a distance has the same bits both ways) and passed to the
+// new lane through an LDS block.  Ranking uses 32-bit keys, the distance's
+// bits with the low 6 replaced by the partner's index; the `keep` nearest by
+// such keys are exactly the `keep` nearest unless the last of them and the
+// next one share all 26 distance bits, and then (about one wave in a hundred)
+// the wave ranks its partners again by full (distance, id) keys.  KEEP is 0,
+// or the largest join_keep the kernel serves.  Bound by VALU issue (two
+// instructions per dimension and pair): six launches at 200k points and
+// join_keep 4 take 1.76 ms at d = 8, 2.56 at 16, 3.13 at 20 and 4.98 at 31,
+// where u64 keys and the lane's own row read from LDS took 3.47, 4.57, 5.96
+// and 11.15.
+template <int DP, bool NEWNEW, int KEEP>
+__global__ __launch_bounds__(kJoinWaves * 64) void k_nnd_join_rows(int64_t n, int d, int S, int keep, NndBufs b) {
+  constexpr int WPB = kJoinWaves;
+  constexpr int kSlots = KEEP == 0 ? 2 : KEEP;
+  constexpr int kRank = KEEP == 0 ? 3 : KEEP + 2;  // the kept, the next one, and the lane itself
+  constexpr int kBlock = 384;                      // as in k_nnd_join2
+  constexpr uint32_t kNone = 0xFFFFFFFFu;
+  __shared__ __attribute__((aligned(16))) float s_vec[WPB][64 * DP];
+  __shared__ float s_blk[WPB][kBlock];
+  __shared__ uint32_t s_new[WPB][64];
+  __shared__ uint32_t s_cand[WPB][64];
+  const unsigned lane = __lane_id();
+  const unsigned w = threadIdx.x >> 6;
+  const int64_t p = static_cast<int64_t>(blockIdx.x) * WPB + w;
+  uint32_t* s_old_w = reinterpret_cast<uint32_t*>(s_blk[w]);
+
+  int nn, nc, rev_drop;
+  join_candidates(b, p, p < n, S, s_new[w], s_old_w, s_cand[w], &nn, &nc, &rev_drop);
+  const int no = nc - nn;
+  const bool active = lane < static_cast<unsigned>(nc);
+  const bool is_new = lane < static_cast<unsigned>(nn);
+  const uint32_t my_id = active ? s_cand[w][lane] : 0u;
+  float own[DP];
+  float lim = 0.0f;
+#pragma unroll
+  for (int k = 0; k < DP; ++k) own[k] = 0.0f;
+  if (active) {
+    // the row ends with the list bound; columns in [d, rstride - 1) are zero
+    const float* src = b.rows + static_cast<int64_t>(my_id) * b.rstride;
+#pragma unroll
+    for (int q = 0; q < DP / 4; ++q) {
+      const float4 v = reinterpret_cast<const float4*>(src)[q];
+      own[4 * q] = v.x, own[4 * q + 1] = v.y, own[4 * q + 2] = v.z, own[4 * q + 3] = v.w;
+    }
+    lim = src[b.rstride - 1];
+    if (DP == b.rstride) own[DP - 1] = 0.0f;
+#pragma unroll
+    for (int q = 0; q < DP / 4; ++q)
+      *reinterpret_cast<float4*>(&s_vec[w][lane * DP + 4 * q]) =
+          make_float4(own[4 * q], own[4 * q + 1], own[4 * q + 2], own[4 * q + 3]);
+  }
+  wave_sync();
+
+  auto partner = [&](int j) {
+    const float* row = s_vec[w] + j * DP;
+    float acc = 0.0f;
+#pragma unroll
+    for (int q = 0; q < DP / 4; ++q) {
+      const float4 v = *reinterpret_cast<const float4*>(row + 4 * q);
+      float diff = own[4 * q] - v.x;
+      acc = __builtin_fmaf(diff, diff, acc);
+      diff = own[4 * q + 1] - v.y;
+      acc = __builtin_fmaf(diff, diff, acc);
+      diff = own[4 * q + 2] - v.z;
+      acc = __builtin_fmaf(diff, diff, acc);
+      diff = own[4 * q + 3] - v.w;
+      acc = __builtin_fmaf(diff, diff, acc);
+    }
+    return acc;
+  };
+  const uint32_t mask_v = 0xFFFFFFC0u;
+  auto rank_key = [&](float acc, int j) {
+    uint32_t r;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(__float_as_uint(acc)), "v"(mask_v), "s"(j));
+    return r;
+  };
+  // top: partners among the new candidates (phase 1), then for a new lane
+  // the old ones too; KEEP == 0 ranks the old ones apart (told)
+  uint32_t top[kRank], told[2] = {kNone, kNone};
+#pragma unroll
+  for (int s = 0; s < kRank; ++s) top[s] = kNone;
+  const int bst = nn + 1;  // odd-or-padded row stride of the old x new block
+  const bool blocked = no * bst <= kBlock;  // uniform
+  const bool store_old = active && !is_new && blocked;
+  float* blk_row = s_blk[w] + (store_old ? (static_cast<int>(lane) - nn) * bst : 0);  // + j
+  int j = 0;
+  for (; j + 2 <= nn; j += 2) {
+    const float a0 = partner(j);
+    const float a1 = partner(j + 1);
+    if (store_old) {
+      blk_row[j] = a0;
+      blk_row[j + 1] = a1;
+    }
+    top_insert32<kRank>(top, rank_key(a0, j));
+    top_insert32<kRank>(top, rank_key(a1, j + 1));
+  }
+  if (j < nn) {
+    const float a0 = partner(j);
+    if (store_old) blk_row[j] = a0;
+    top_insert32<kRank>(top, rank_key(a0, j));
+  }
+  if (!NEWNEW && is_new) {  // merge mode: new candidates skip new partners
+#pragma unroll
+    for (int s = 0; s < kRank; ++s) top[s] = kNone;
+  }
+  wave_sync();
+  uint32_t keep_top[kRank];
+#pragma unroll
+  for (int s = 0; s < kRank; ++s) keep_top[s] = top[s];
+  const float* blk_col = s_blk[w] + (is_new ? static_cast<int>(lane) : 0);
+  auto rank_old = [&](float acc, int jj) {
+    if (KEEP == 0) top_insert32<2>(told, rank_key(acc, jj));
+    else top_insert32<kRank>(top, rank_key(acc, jj));
+  };
+  int o = 0;
+  if (blocked) {
+    for (; o + 4 <= no; o += 4) {  // four reads in flight a step
+      const float a0 = blk_col[o * bst], a1 = blk_col[(o + 1) * bst];
+      const float a2 = blk_col[(o + 2) * bst], a3 = blk_col[(o + 3) * bst];
+      rank_old(a0, nn + o);
+      rank_old(a1, nn + o + 1);
+      rank_old(a2, nn + o + 2);
+      rank_old(a3, nn + o + 3);
+    }
+    for (; o < no; ++o) rank_old(blk_col[o * bst], nn + o);
+  } else {
+    for (; o < no; ++o) rank_old(partner(nn + o), nn + o);
+  }
+  if (!is_new) {
+#pragma unroll
+    for (int s = 0; s < kRank; ++s) top[s] = keep_top[s];
+    told[0] = told[1] = kNone;
+  }
+  // drop the lane itself (it ranks at most once, in phase 1), pick the kept
+  // partners, and see whether the choice is certain
+  uint32_t fin[kSlots];
+  bool tie = false;
+  {
+    uint32_t f[kRank - 1];
+    bool seen = false;
+#pragma unroll
+    for (int s = 0; s < kRank - 1; ++s) {
+      seen = seen || (top[s] != kNone && (top[s] & 63u) == lane);
+      f[s] = seen ? top[s + 1] : top[s];
+    }
+    if (KEEP == 0) {
+      fin[0] = f[0];
+      fin[1] = told[0];
+      tie = (f[1] != kNone && ((f[0] ^ f[1]) >> 6) == 0) || (told[1] != kNone && ((told[0] ^ told[1]) >> 6) == 0);
+    } else {
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) {
+        fin[s] = s < keep ? f[s] : kNone;
+        if (s + 1 == keep) tie = f[s + 1] != kNone && ((f[s] ^ f[s + 1]) >> 6) == 0;
+      }
+    }
+  }
+  uint64_t top64[kSlots];
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s) {
+    top64[s] = kKeyMax;
+    if (active && fin[s] != kNone) {
+      const int jj = static_cast<int>(fin[s] & 63u);
+      const float* row = s_vec[w] + jj * DP;
+      float acc = 0.0f;
+#pragma unroll
+      for (int k = 0; k < DP; ++k) {
+        const float diff = own[k] - row[k];
+        acc = __builtin_fmaf(diff, diff, acc);
+      }
+      top64[s] = make_key(acc, s_cand[w][jj], 1u);
+    }
+  }
+  if (__ballot(active && tie)) {  // uniform: rank every partner by its full key
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) top64[s] = kKeyMax;
+    const int jb = is_new ? (NEWNEW ? 0 : nn) : 0, je = is_new ? nc : nn;
+    for (int jj = 0; jj < nc; ++jj) {
+      const float acc = partner(jj);
+      const bool ok = active && jj >= jb && jj < je && jj != static_cast<int>(lane);
+      const uint64_t key = ok ? make_key(acc, s_cand[w][jj], 1u) : kKeyMax;
+      if (KEEP == 0) {
+        if (jj < nn) top64[0] = key < top64[0] ? key : top64[0];
+        else top64[1] = key < top64[1] ? key : top64[1];
+      } else {
+        top_insert<kSlots>(top64, key);
+      }
+    }
+    if (KEEP != 0) {
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s)
+        if (s >= keep) top64[s] = kKeyMax;
+    }
+  }
+  join_emit<WPB, kSlots>(b, top64, active, my_id, lim, nc, rev_drop);
+}
+
 // BF16 join (distance_mode 1): the 64 x 64 Gram matrix of the candidates is
 // computed with v_mfma_f32_16x16x32_bf16 (BF16 inputs, FP32 accumulation)
 // from the FP32 rows staged in LDS, with the operands swapped so that lane l
@@ -1386,6 +1588,19 @@ static int launch_join_t(hdb_ctx* ctx, const float* X, int64_t n, int d, int S, 
   }
 }
 
+template <int DP, bool NEWNEW>
+static int launch_join_rows(hdb_ctx* ctx, int64_t n, int d, int S, const NndBufs& b) {
+  const dim3 grid(grid_for(n, kJoinWaves)), block(kJoinWaves * 64);
+  if (b.join_keep == 0)
+    hipLaunchKernelGGL((k_nnd_join_rows<DP, NEWNEW, 0>), grid, block, 0, ctx->stream, n, d, S, 0, b);
+  else if (b.join_keep <= 4)
+    hipLaunchKernelGGL((k_nnd_join_rows<DP, NEWNEW, 4>), grid, block, 0, ctx->stream, n, d, S, b.join_keep, b);
+  else
+    hipLaunchKernelGGL((k_nnd_join_rows<DP, NEWNEW, 8>), grid, block, 0, ctx->stream, n, d, S, b.join_keep, b);
+  HDB_LAUNCHED();
+  return HDB_OK;
+}
+
 // rerank_keep 0: the join_keep + 2 nearest partners by the BF16 Gram
 // matrix are re-ranked in FP32; 16: the 16 nearest.
 template <bool NEWNEW, int KEEP>
@@ -1418,6 +1633,13 @@ static int launch_join(hdb_ctx* ctx, const float* X, int64_t n, int d, int S, co
   }
   if (d == 12) return launch_join_t<12, NEWNEW>(ctx, X, n, d, S, b);
   if (d == 32) return launch_join_t<32, NEWNEW>(ctx, X, n, d, S, b);
+  if (d <= 4) return launch_join_rows<4, NEWNEW>(ctx, n, d, S, b);
+  if (d <= 8) return launch_join_rows<8, NEWNEW>(ctx, n, d, S, b);
+  if (d <= 12) return launch_join_rows<12, NEWNEW>(ctx, n, d, S, b);
+  if (d <= 16) return launch_join_rows<16, NEWNEW>(ctx, n, d, S, b);
+  if (d <= 20) return launch_join_rows<20, NEWNEW>(ctx, n, d, S, b);
+  if (d <= 24) return launch_join_rows<24, NEWNEW>(ctx, n, d, S, b);
+  if (d < 32) return launch_join_rows<32, NEWNEW>(ctx, n, d, S, b);
   return launch_join_t<0, NEWNEW>(ctx, X, n, d, S, b);
 }
 

@@ -279,3 +279,40 @@ def test_list_distances_never_grow(ctx, keep):
             assert np.all(d[:, -1] <= prev[:, -1])
             assert np.all(d.sum(1) <= prev.sum(1) * (1 + 1e-12))
         prev = d
+
+
+def _points_with_ties(n, d, seed, ties):
+    """A mixture; `ties`: coordinates on a coarse grid, with repeated points,
+    so that many candidate distances are equal."""
+    X = datasets.tiny_blobs(n, d, 6, seed=seed, spread=4.0)
+    if ties:
+        X = np.round(X).astype(np.float32)
+        X[: n // 8] = X[n // 2: n // 2 + n // 8]
+    return X
+
+
+@pytest.mark.parametrize("d", [1, 2, 4, 5, 8, 9, 11, 13, 15, 16, 17, 20, 21, 24, 25, 31])
+@pytest.mark.parametrize("ties", [False, True])
+def test_join_rows_equals_wider_join(ctx, d, ties):
+    """Zero columns change no distance, so the same points padded past the
+    dimensions of the register-row join take another join kernel to the same
+    lists, bit for bit, for every join_keep and for the merge schedule."""
+    print(f"case: join at d={d} against the same points padded to d=40, ties={ties}", flush=True)
+    n = 3001
+    X = _points_with_ties(n, d, 90 + d, ties)
+    P = np.zeros((n, 40), np.float32)
+    P[:, :d] = X
+    for keep in (0, 1, 2, 3, 4, 8):
+        p = api.default_params(join_keep=keep, bucket_cap=1024)  # room for every proposal of join_keep 8
+        a = api.NNDescent(ctx, X, iteration=4, params=p)
+        b = api.NNDescent(ctx, P, iteration=4, params=p)
+        assert ctx.nnd_stats()["bucket_drops"] == 0
+        np.testing.assert_array_equal(a["label"], b["label"])
+        np.testing.assert_array_equal(a["distance"].view(np.uint32), b["distance"].view(np.uint32))
+    for keep in (0, 4):
+        p = api.default_params(join_keep=keep, bucket_cap=1024)
+        a = api.GenLargeKNNGraph(ctx, X, 2, params=p)
+        b = api.GenLargeKNNGraph(ctx, P, 2, params=p)
+        assert ctx.nnd_stats()["bucket_drops"] == 0
+        np.testing.assert_array_equal(a["label"], b["label"])
+        np.testing.assert_array_equal(a["distance"].view(np.uint32), b["distance"].view(np.uint32))
