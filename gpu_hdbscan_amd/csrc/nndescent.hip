@@ -21,7 +21,7 @@
 //   radix sort     PrepareReverseGraph (:293-346) without global atomics;
 //                  each reverse list keeps S of its pairs, evenly spaced
 //                  in source order (the reference keeps the first S arrivals)
-//   k_nnd_join     ShrinkGraph + NewNeighborsCompareKernel +
+//   k_nnd_join*    ShrinkGraph + NewNeighborsCompareKernel +
 //                  TiledNewOldNeighborsCompareKernel (:405-510, :1030-1326):
 //                  one wave64 per point; candidates propose their nearest
 //                  partners to their own lists
@@ -484,97 +484,17 @@ __device__ __forceinline__ void top_insert(uint64_t (&top)[SLOTS], uint64_t key)
   }
 }
 
-// FP32 join.  Candidate c (lane c) computes the squared distance to each
+// FP32 joins.  Candidate c (lane c) takes the squared distance to each
 // partner -- the other new candidates and the old ones if c is new (NEWNEW),
 // only the old ones if c is new in merge mode, the new ones if c is old --
 // and proposes its nearest partners (GetMinElement/2/3 :852-961) to its own
-// list unless they cannot beat the list's current 32nd entry.
-template <int D, bool NEWNEW, int KEEP>
-__global__ __launch_bounds__(kJoinWaves * 64) void k_nnd_join(const float* __restrict__ X, int64_t n, int d, int S,
-                                                              NndBufs b) {
-  constexpr int WPB = kJoinWaves;
-  constexpr bool kOwnReg = (D > 0 && D <= 32);
-  constexpr int kStride = kOwnReg ? ((D + 3) & ~3) : 0;
-  constexpr int kSlots = KEEP == 0 ? 2 : KEEP;
-  extern __shared__ __attribute__((aligned(16))) float lds_dyn[];
-  __shared__ uint32_t s_new[WPB][64];
-  __shared__ uint32_t s_old[WPB][64];
-  __shared__ uint32_t s_cand[WPB][64];
-  const unsigned lane = __lane_id();
-  const unsigned w = threadIdx.x >> 6;
-  const int64_t p = static_cast<int64_t>(blockIdx.x) * WPB + w;
-  const int dd = D > 0 ? D : d;
-  const int stride = kOwnReg ? kStride : ((dd + 3) & ~3) + 4;  // 16-byte aligned rows
-  float* vec = lds_dyn + static_cast<int64_t>(w) * 64 * stride;
-
-  int nn, nc, rev_drop;
-  join_candidates(b, p, p < n, S, s_new[w], s_old[w], s_cand[w], &nn, &nc, &rev_drop);
-
-  const bool active = lane < static_cast<unsigned>(nc);
-  const uint32_t my_id = active ? s_cand[w][lane] : 0u;
-  const float lim = active ? b.worst[static_cast<int64_t>(my_id) * b.wstride] : 0.0f;
-  float own[kOwnReg ? kStride : 1];
-  if (kOwnReg) {
-    if (active) {
-      const float* src = X + static_cast<int64_t>(my_id) * D;
-#pragma unroll
-      for (int k = 0; k < D; ++k) own[k] = src[k];
-    } else {
-#pragma unroll
-      for (int k = 0; k < D; ++k) own[k] = 0.0f;
-    }
-#pragma unroll
-    for (int k = D; k < kStride; ++k) own[k] = 0.0f;
-    if (active) {
-#pragma unroll
-      for (int k = 0; k < kStride; ++k) vec[lane * kStride + k] = own[k];
-    }
-  } else if (active) {
-    // lane c gathers candidate c's row: all rows are in flight together
-    const float* src = b.rows + static_cast<int64_t>(my_id) * b.rstride;
-    for (int k = 0; k < dd; ++k) vec[lane * stride + k] = src[k];
-  }
-  __syncthreads();
-
-  int jb, je;  // partner range of this lane
-  if (static_cast<int>(lane) < nn) {
-    jb = NEWNEW ? 0 : nn;
-    je = nc;
-  } else {
-    jb = 0;
-    je = nn;
-  }
-  // KEEP == 0: the reference's two kernels -- a new candidate takes its
-  // nearest new partner (NewNeighborsCompareKernel) and its nearest old
-  // partner (TiledNewOldNeighborsCompareKernel), an old one its nearest new
-  // partner.  KEEP == T > 0: every candidate proposes its T nearest partners.
-  uint64_t top[kSlots];
-#pragma unroll
-  for (int s = 0; s < kSlots; ++s) top[s] = kKeyMax;
-  for (int j = 0; j < nc; ++j) {
-    const float* row = vec + j * stride;
-    float acc;
-    if (kOwnReg) {
-      acc = 0.0f;
-#pragma unroll
-      for (int k = 0; k < D; ++k) {
-        const float diff = own[k] - row[k];
-        acc = __builtin_fmaf(diff, diff, acc);
-      }
-    } else {
-      acc = (dd & 3) == 0 ? d2_vec4(vec + lane * stride, row, dd) : d2_any(vec + lane * stride, row, dd);
-    }
-    const bool ok = active && j >= jb && j < je && j != static_cast<int>(lane);
-    const uint64_t key = ok ? make_key(acc, s_cand[w][j], 1u) : kKeyMax;
-    if (KEEP == 0) {
-      if (j < nn) top[0] = key < top[0] ? key : top[0];
-      else top[1] = key < top[1] ? key : top[1];
-    } else {
-      top_insert<kSlots>(top, key);
-    }
-  }
-  join_emit<WPB, kSlots>(b, top, active, my_id, lim, nc, rev_drop);
-}
+// list unless they cannot beat the list's current 32nd entry.  KEEP == 0: the
+// reference's two kernels -- a new candidate takes its nearest new partner
+// (NewNeighborsCompareKernel) and its nearest old partner
+// (TiledNewOldNeighborsCompareKernel), an old one its nearest new partner.
+// KEEP > 0: every candidate proposes its nearest partners.  k_nnd_join2
+// serves d = 12 and 32, k_nnd_join_rows the other d <= 31, k_nnd_join_wide
+// d > 32.
 
 // Order-preserving u32 image of a float of any sign (NaN excluded).
 __device__ __forceinline__ uint32_t order_bits(float x) {
@@ -594,7 +514,7 @@ __device__ __forceinline__ void top_insert32(uint32_t (&top)[SLOTS], uint32_t ke
 // keys -- the bits of that value without the sign, with the low 6 bits
 // replaced by the partner's index -- and the KEEP winners' exact squared
 // distances are then recomputed from the same rows in the same operation
-// order as k_nnd_join, so proposals carry exactly its distances; only the
+// order as the other joins, so proposals carry exactly its distances; only the
 // choice among partners whose distances agree to about 1e-4 relative can
 // differ.
 template <int D, bool NEWNEW, int KEEP>
@@ -821,21 +741,96 @@ __global__ __launch_bounds__(kJoinWaves * 64, 8) void k_nnd_join2(const float* _
   join_emit<WPB, kSlots>(b, top64, active, my_id, lim, nc, rev_drop);
 }
 
+// Key of a ranking value with no sign: its bits, the low 6 replaced by the
+// partner's index j, which is wave-uniform.
+__device__ __forceinline__ uint32_t rank_key6(float acc, int j) {
+  const uint32_t mask_v = 0xFFFFFFC0u;  // a VGPR operand: VOP3 takes no literal here
+  uint32_t r;
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(__float_as_uint(acc)), "v"(mask_v), "s"(j));
+  return r;
+}
+
+// The kept partners of one candidate from its smallest 26-bit ranking keys
+// (ascending): top holds one slot more than the kept and the next one, for
+// the lane itself, which ranks at most once and is dropped here; KEEP == 0
+// has its old partners' two smallest in told.  The `keep` smallest are
+// exactly the `keep` nearest unless the last of them and the next one share
+// all their distance bits, and then (about one wave in a hundred on
+// continuous data) the wave ranks its partners again by full (distance, id)
+// keys.  dist(j): the exact distance to partner j.
+template <bool NEWNEW, int KEEP, int SLOTS, int RANK, typename F>
+__device__ __forceinline__ void join_choose(const uint32_t (&top)[RANK], const uint32_t (&told)[2], int nn, int nc,
+                                            int keep, const uint32_t* s_cand, F dist, uint64_t (&top64)[SLOTS]) {
+  constexpr uint32_t kNone = 0xFFFFFFFFu;
+  static_assert(RANK == (KEEP == 0 ? 3 : KEEP + 2) && SLOTS == (KEEP == 0 ? 2 : KEEP), "slots of the join");
+  const int lane = static_cast<int>(__lane_id());
+  const bool active = lane < nc, is_new = lane < nn;
+  uint32_t fin[SLOTS], f[RANK - 1];
+  bool seen = false, tie = false;
+#pragma unroll
+  for (int s = 0; s < RANK - 1; ++s) {
+    // values first, then the choice: a choice between elements would become
+    // an index, and the array would go to scratch memory
+    const uint32_t here = top[s], next = top[s + 1];
+    seen = seen || (here != kNone && static_cast<int>(here & 63u) == lane);
+    f[s] = here ^ ((here ^ next) & (seen ? 0xFFFFFFFFu : 0u));
+  }
+  if (KEEP == 0) {
+    fin[0] = f[0];
+    fin[1] = told[0];
+    tie = (f[1] != kNone && ((f[0] ^ f[1]) >> 6) == 0) || (told[1] != kNone && ((told[0] ^ told[1]) >> 6) == 0);
+  } else {
+    // bit s: slots s and s + 1 agree (a bit mask, so that no slot is indexed
+    // by keep and the arrays stay in registers)
+    uint32_t same = 0;
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) {
+      fin[s] = s < keep ? f[s] : kNone;
+      same |= (f[s + 1] != kNone && ((f[s] ^ f[s + 1]) >> 6) == 0 ? 1u : 0u) << s;
+    }
+    tie = ((same >> (keep - 1)) & 1u) != 0;
+  }
+#pragma unroll
+  for (int s = 0; s < SLOTS; ++s) {
+    top64[s] = kKeyMax;
+    if (active && fin[s] != kNone) {
+      const int j = static_cast<int>(fin[s] & 63u);
+      top64[s] = make_key(dist(j), s_cand[j], 1u);
+    }
+  }
+  if (__ballot(active && tie)) {  // uniform: rank every partner by its full key
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) top64[s] = kKeyMax;
+    const int jb = is_new ? (NEWNEW ? 0 : nn) : 0, je = is_new ? nc : nn;
+    for (int j = 0; j < nc; ++j) {
+      if (!(active && j >= jb && j < je && j != lane)) continue;
+      const uint64_t key = make_key(dist(j), s_cand[j], 1u);
+      if (KEEP == 0) {
+        if (j < nn) top64[0] = key < top64[0] ? key : top64[0];
+        else top64[1] = key < top64[1] ? key : top64[1];
+      } else {
+        top_insert<SLOTS>(top64, key);
+      }
+    }
+    if (KEEP != 0) {
+#pragma unroll
+      for (int s = 0; s < SLOTS; ++s)
+        if (s >= keep) top64[s] = kKeyMax;
+    }
+  }
+}
+
 // FP32 join for d <= 31 other than 12 (d = 12 and 32 have k_nnd_join2): exact
 // distances, with the candidates' padded rows in LDS and the lane's own row
 // in registers (DP: d rounded up to a multiple of 4 or so; the zeros past d
 // add nothing to a distance).  As in k_nnd_join2 each old-new pair is
 // evaluated once (a distance has the same bits both ways) and passed to the
-// new lane through an LDS block.  Ranking uses 32-bit keys, the distance's
-// bits with the low 6 replaced by the partner's index; the `keep` nearest by
-// such keys are exactly the `keep` nearest unless the last of them and the
-// next one share all 26 distance bits, and then (about one wave in a hundred)
-// the wave ranks its partners again by full (distance, id) keys.  KEEP is 0,
-// or the largest join_keep the kernel serves.  Bound by VALU issue (two
-// instructions per dimension and pair): six launches at 200k points and
-// join_keep 4 take 1.76 ms at d = 8, 2.56 at 16, 3.13 at 20 and 4.98 at 31,
-// where u64 keys and the lane's own row read from LDS took 3.47, 4.57, 5.96
-// and 11.15.
+// new lane through an LDS block.  Ranking uses 32-bit keys (rank_key6,
+// join_choose).  KEEP is 0, or the largest join_keep the kernel serves.
+// Bound by VALU issue (two instructions per dimension and pair): six launches
+// at 200k points and join_keep 4 take 1.76 ms at d = 8, 2.56 at 16, 3.13 at
+// 20 and 4.98 at 31, where u64 keys and the lane's own row read from LDS took
+// 3.47, 4.57, 5.96 and 11.15.
 template <int DP, bool NEWNEW, int KEEP>
 __global__ __launch_bounds__(kJoinWaves * 64) void k_nnd_join_rows(int64_t n, int d, int S, int keep, NndBufs b) {
   constexpr int WPB = kJoinWaves;
@@ -896,12 +891,6 @@ __global__ __launch_bounds__(kJoinWaves * 64) void k_nnd_join_rows(int64_t n, in
     }
     return acc;
   };
-  const uint32_t mask_v = 0xFFFFFFC0u;
-  auto rank_key = [&](float acc, int j) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(__float_as_uint(acc)), "v"(mask_v), "s"(j));
-    return r;
-  };
   // top: partners among the new candidates (phase 1), then for a new lane
   // the old ones too; KEEP == 0 ranks the old ones apart (told)
   uint32_t top[kRank], told[2] = {kNone, kNone};
@@ -919,13 +908,13 @@ __global__ __launch_bounds__(kJoinWaves * 64) void k_nnd_join_rows(int64_t n, in
       blk_row[j] = a0;
       blk_row[j + 1] = a1;
     }
-    top_insert32<kRank>(top, rank_key(a0, j));
-    top_insert32<kRank>(top, rank_key(a1, j + 1));
+    top_insert32<kRank>(top, rank_key6(a0, j));
+    top_insert32<kRank>(top, rank_key6(a1, j + 1));
   }
   if (j < nn) {
     const float a0 = partner(j);
     if (store_old) blk_row[j] = a0;
-    top_insert32<kRank>(top, rank_key(a0, j));
+    top_insert32<kRank>(top, rank_key6(a0, j));
   }
   if (!NEWNEW && is_new) {  // merge mode: new candidates skip new partners
 #pragma unroll
@@ -937,8 +926,8 @@ __global__ __launch_bounds__(kJoinWaves * 64) void k_nnd_join_rows(int64_t n, in
   for (int s = 0; s < kRank; ++s) keep_top[s] = top[s];
   const float* blk_col = s_blk[w] + (is_new ? static_cast<int>(lane) : 0);
   auto rank_old = [&](float acc, int jj) {
-    if (KEEP == 0) top_insert32<2>(told, rank_key(acc, jj));
-    else top_insert32<kRank>(top, rank_key(acc, jj));
+    if (KEEP == 0) top_insert32<2>(told, rank_key6(acc, jj));
+    else top_insert32<kRank>(top, rank_key6(acc, jj));
   };
   int o = 0;
   if (blocked) {
@@ -959,67 +948,145 @@ __global__ __launch_bounds__(kJoinWaves * 64) void k_nnd_join_rows(int64_t n, in
     for (int s = 0; s < kRank; ++s) top[s] = keep_top[s];
     told[0] = told[1] = kNone;
   }
-  // drop the lane itself (it ranks at most once, in phase 1), pick the kept
-  // partners, and see whether the choice is certain
-  uint32_t fin[kSlots];
-  bool tie = false;
-  {
-    uint32_t f[kRank - 1];
-    bool seen = false;
+  uint64_t top64[kSlots];
+  join_choose<NEWNEW, KEEP>(top, told, nn, nc, keep, s_cand[w], partner, top64);
+  join_emit<WPB, kSlots>(b, top64, active, my_id, lim, nc, rev_drop);
+}
+
+// FP32 join for d > 32: exact distances, the dimensions taken 16 at a time.
+// Per chunk the wave stages its candidates' 16 columns in LDS (quad q of row
+// r at q ^ ((r >> 1) & 3), so that the lanes' 16-byte stores spread over the
+// banks)
+// and every lane adds the chunk to its distances to the new candidates, which
+// stay in registers (at most 32); the additions run in dimension order, so
+// the distances have the bits of the other forms.  The distances then go to
+// LDS in place of the rows (entry (j, lane) at 65 j + lane), where the new
+// lanes also find theirs to the old candidates.  Bound by VALU issue, two
+// instructions per dimension and pair: six launches at join_keep 4 take 5.8 ms
+// at 200k x 40, 7.0 at 200k x 64 and 6.0 at 100k x 128, where the lane's own row
+// read from LDS and u64 keys took 11.6, 19.7 and 30.4.
+template <bool NEWNEW, int KEEP>
+__global__ __launch_bounds__(kJoinWaves * 64, 4) void k_nnd_join_wide(const float* __restrict__ X, int64_t n, int d,
+                                                                   int S, int keep, NndBufs b) {
+  constexpr int WPB = kJoinWaves;
+  constexpr int kSlots = KEEP == 0 ? 2 : KEEP;
+  constexpr int kRank = KEEP == 0 ? 3 : KEEP + 2;
+  constexpr int kNew = 32;  // new candidates at most (join_candidates)
+  constexpr int kC = 16;    // columns per chunk
+  constexpr int kM = 65;    // stride of the distance block
+  constexpr uint32_t kNone = 0xFFFFFFFFu;
+  __shared__ __attribute__((aligned(16))) float s_buf[WPB][kNew * kM];
+  static_assert(kNew * kM >= 64 * kC && (kNew * kM) % 4 == 0, "rows and distances share the buffer");
+  __shared__ uint32_t s_new[WPB][64];
+  __shared__ uint32_t s_cand[WPB][64];
+  const unsigned lane = __lane_id();
+  const unsigned w = threadIdx.x >> 6;
+  const int64_t p = static_cast<int64_t>(blockIdx.x) * WPB + w;
+  float* buf = s_buf[w];
+
+  int nn, nc, rev_drop;
+  join_candidates(b, p, p < n, S, s_new[w], reinterpret_cast<uint32_t*>(buf), s_cand[w], &nn, &nc, &rev_drop);
+  const int no = nc - nn;
+  const bool active = lane < static_cast<unsigned>(nc);
+  const bool is_new = lane < static_cast<unsigned>(nn);
+  const uint32_t my_id = active ? s_cand[w][lane] : 0u;
+  const float lim = active ? b.worst[static_cast<int64_t>(my_id) * b.wstride] : 0.0f;
+  const float* src = X + static_cast<int64_t>(my_id) * d;
+  const bool vec4 = (d & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;  // uniform
+
+  float acc[kNew];
 #pragma unroll
-    for (int s = 0; s < kRank - 1; ++s) {
-      seen = seen || (top[s] != kNone && (top[s] & 63u) == lane);
-      f[s] = seen ? top[s + 1] : top[s];
-    }
-    if (KEEP == 0) {
-      fin[0] = f[0];
-      fin[1] = told[0];
-      tie = (f[1] != kNone && ((f[0] ^ f[1]) >> 6) == 0) || (told[1] != kNone && ((told[0] ^ told[1]) >> 6) == 0);
-    } else {
+  for (int j = 0; j < kNew; ++j) acc[j] = 0.0f;
+  for (int c0 = 0; c0 < d; c0 += kC) {
+    float own[kC];
 #pragma unroll
-      for (int s = 0; s < kSlots; ++s) {
-        fin[s] = s < keep ? f[s] : kNone;
-        if (s + 1 == keep) tie = f[s + 1] != kNone && ((f[s] ^ f[s + 1]) >> 6) == 0;
+    for (int k = 0; k < kC; ++k) own[k] = 0.0f;
+    if (active) {
+      if (vec4) {
+#pragma unroll
+        for (int q = 0; q < kC / 4; ++q)
+          if (c0 + 4 * q < d) {
+            const float4 v = *reinterpret_cast<const float4*>(src + c0 + 4 * q);
+            own[4 * q] = v.x, own[4 * q + 1] = v.y, own[4 * q + 2] = v.z, own[4 * q + 3] = v.w;
+          }
+      } else {
+#pragma unroll
+        for (int k = 0; k < kC; ++k)
+          if (c0 + k < d) own[k] = src[c0 + k];
       }
     }
+    wave_sync();  // the previous chunk (and the candidate scratch) has been read
+#pragma unroll
+    for (int q = 0; q < kC / 4; ++q)
+      *reinterpret_cast<float4*>(buf + lane * kC + 4 * (q ^ static_cast<int>((lane >> 1) & 3))) =
+          make_float4(own[4 * q], own[4 * q + 1], own[4 * q + 2], own[4 * q + 3]);
+    wave_sync();
+#pragma unroll
+    for (int j0 = 0; j0 < kNew; j0 += 4) {
+      if (j0 < nn) {  // uniform
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int j = j0 + u;
+          float a = acc[j];
+#pragma unroll
+          for (int q = 0; q < kC / 4; ++q) {
+            const float4 v = *reinterpret_cast<const float4*>(buf + j * kC + 4 * (q ^ ((j >> 1) & 3)));
+            float diff = own[4 * q] - v.x;
+            a = __builtin_fmaf(diff, diff, a);
+            diff = own[4 * q + 1] - v.y;
+            a = __builtin_fmaf(diff, diff, a);
+            diff = own[4 * q + 2] - v.z;
+            a = __builtin_fmaf(diff, diff, a);
+            diff = own[4 * q + 3] - v.w;
+            a = __builtin_fmaf(diff, diff, a);
+          }
+          acc[j] = a;
+        }
+      }
+    }
+  }
+  wave_sync();
+  uint32_t top[kRank], told[2] = {kNone, kNone};
+#pragma unroll
+  for (int s = 0; s < kRank; ++s) top[s] = kNone;
+#pragma unroll
+  for (int j = 0; j < kNew; ++j) {
+    if (j < nn) {  // uniform
+      buf[j * kM + lane] = acc[j];
+      top_insert32<kRank>(top, rank_key6(acc[j], j));
+    }
+  }
+  if (!NEWNEW && is_new) {  // merge mode: new candidates skip new partners
+#pragma unroll
+    for (int s = 0; s < kRank; ++s) top[s] = kNone;
+  }
+  wave_sync();
+  uint32_t keep_top[kRank];
+#pragma unroll
+  for (int s = 0; s < kRank; ++s) keep_top[s] = top[s];
+  const float* to_old = buf + (is_new ? static_cast<int>(lane) : 0) * kM + nn;
+  auto rank_old = [&](float a, int jj) {
+    if (KEEP == 0) top_insert32<2>(told, rank_key6(a, jj));
+    else top_insert32<kRank>(top, rank_key6(a, jj));
+  };
+  int o = 0;
+  for (; o + 4 <= no; o += 4) {  // four reads in flight a step
+    const float a0 = to_old[o], a1 = to_old[o + 1], a2 = to_old[o + 2], a3 = to_old[o + 3];
+    rank_old(a0, nn + o);
+    rank_old(a1, nn + o + 1);
+    rank_old(a2, nn + o + 2);
+    rank_old(a3, nn + o + 3);
+  }
+  for (; o < no; ++o) rank_old(to_old[o], nn + o);
+  if (!is_new) {
+#pragma unroll
+    for (int s = 0; s < kRank; ++s) top[s] = keep_top[s];
+    told[0] = told[1] = kNone;
   }
   uint64_t top64[kSlots];
-#pragma unroll
-  for (int s = 0; s < kSlots; ++s) {
-    top64[s] = kKeyMax;
-    if (active && fin[s] != kNone) {
-      const int jj = static_cast<int>(fin[s] & 63u);
-      const float* row = s_vec[w] + jj * DP;
-      float acc = 0.0f;
-#pragma unroll
-      for (int k = 0; k < DP; ++k) {
-        const float diff = own[k] - row[k];
-        acc = __builtin_fmaf(diff, diff, acc);
-      }
-      top64[s] = make_key(acc, s_cand[w][jj], 1u);
-    }
-  }
-  if (__ballot(active && tie)) {  // uniform: rank every partner by its full key
-#pragma unroll
-    for (int s = 0; s < kSlots; ++s) top64[s] = kKeyMax;
-    const int jb = is_new ? (NEWNEW ? 0 : nn) : 0, je = is_new ? nc : nn;
-    for (int jj = 0; jj < nc; ++jj) {
-      const float acc = partner(jj);
-      const bool ok = active && jj >= jb && jj < je && jj != static_cast<int>(lane);
-      const uint64_t key = ok ? make_key(acc, s_cand[w][jj], 1u) : kKeyMax;
-      if (KEEP == 0) {
-        if (jj < nn) top64[0] = key < top64[0] ? key : top64[0];
-        else top64[1] = key < top64[1] ? key : top64[1];
-      } else {
-        top_insert<kSlots>(top64, key);
-      }
-    }
-    if (KEEP != 0) {
-#pragma unroll
-      for (int s = 0; s < kSlots; ++s)
-        if (s >= keep) top64[s] = kKeyMax;
-    }
-  }
+  join_choose<NEWNEW, KEEP>(
+      top, told, nn, nc, keep, s_cand[w],
+      [&](int j) { return j < nn ? buf[j * kM + lane] : buf[lane * kM + j]; }, top64);
   join_emit<WPB, kSlots>(b, top64, active, my_id, lim, nc, rev_drop);
 }
 
@@ -1561,16 +1628,7 @@ static int read_stats(hdb_ctx* ctx, int64_t n, const NndBufs& b) {
 
 template <int D, bool NEWNEW, int KEEP>
 static int launch_join_k(hdb_ctx* ctx, const float* X, int64_t n, int d, int S, const NndBufs& b) {
-  constexpr bool kOwnReg = (D > 0 && D <= 32);
-  if (kOwnReg) {
-    hipLaunchKernelGGL((k_nnd_join2<kOwnReg ? D : 12, NEWNEW, KEEP>), dim3(grid_for(n, kJoinWaves)),
-                       dim3(kJoinWaves * 64), 0, ctx->stream, X, n, d, S, b);
-    HDB_LAUNCHED();
-    return HDB_OK;
-  }
-  const int stride = kOwnReg ? ((D + 3) & ~3) : ((d + 3) & ~3) + 4;
-  const size_t lds = static_cast<size_t>(kJoinWaves) * 64 * stride * sizeof(float);
-  hipLaunchKernelGGL((k_nnd_join<D, NEWNEW, KEEP>), dim3(grid_for(n, kJoinWaves)), dim3(kJoinWaves * 64), lds,
+  hipLaunchKernelGGL((k_nnd_join2<D, NEWNEW, KEEP>), dim3(grid_for(n, kJoinWaves)), dim3(kJoinWaves * 64), 0,
                      ctx->stream, X, n, d, S, b);
   HDB_LAUNCHED();
   return HDB_OK;
@@ -1597,6 +1655,19 @@ static int launch_join_rows(hdb_ctx* ctx, int64_t n, int d, int S, const NndBufs
     hipLaunchKernelGGL((k_nnd_join_rows<DP, NEWNEW, 4>), grid, block, 0, ctx->stream, n, d, S, b.join_keep, b);
   else
     hipLaunchKernelGGL((k_nnd_join_rows<DP, NEWNEW, 8>), grid, block, 0, ctx->stream, n, d, S, b.join_keep, b);
+  HDB_LAUNCHED();
+  return HDB_OK;
+}
+
+template <bool NEWNEW>
+static int launch_join_wide(hdb_ctx* ctx, const float* X, int64_t n, int d, int S, const NndBufs& b) {
+  const dim3 grid(grid_for(n, kJoinWaves)), block(kJoinWaves * 64);
+  if (b.join_keep == 0)
+    hipLaunchKernelGGL((k_nnd_join_wide<NEWNEW, 0>), grid, block, 0, ctx->stream, X, n, d, S, 0, b);
+  else if (b.join_keep <= 4)
+    hipLaunchKernelGGL((k_nnd_join_wide<NEWNEW, 4>), grid, block, 0, ctx->stream, X, n, d, S, b.join_keep, b);
+  else
+    hipLaunchKernelGGL((k_nnd_join_wide<NEWNEW, 8>), grid, block, 0, ctx->stream, X, n, d, S, b.join_keep, b);
   HDB_LAUNCHED();
   return HDB_OK;
 }
@@ -1640,7 +1711,7 @@ static int launch_join(hdb_ctx* ctx, const float* X, int64_t n, int d, int S, co
   if (d <= 20) return launch_join_rows<20, NEWNEW>(ctx, n, d, S, b);
   if (d <= 24) return launch_join_rows<24, NEWNEW>(ctx, n, d, S, b);
   if (d < 32) return launch_join_rows<32, NEWNEW>(ctx, n, d, S, b);
-  return launch_join_t<0, NEWNEW>(ctx, X, n, d, S, b);
+  return launch_join_wide<NEWNEW>(ctx, X, n, d, S, b);
 }
 
 // first_full: the first update merges every list, which also removes

@@ -316,3 +316,25 @@ def test_join_rows_equals_wider_join(ctx, d, ties):
         assert ctx.nnd_stats()["bucket_drops"] == 0
         np.testing.assert_array_equal(a["label"], b["label"])
         np.testing.assert_array_equal(a["distance"].view(np.uint32), b["distance"].view(np.uint32))
+
+
+@pytest.mark.parametrize("d", [33, 37, 63, 64, 65, 100, 128, 255])
+@pytest.mark.parametrize("ties", [False, True])
+def test_join_wide_dimensions(ctx, d, ties):
+    """The chunked join at ragged dimensions: its lists hold the oracle's
+    distances and do not change when zero columns move the chunk ends."""
+    print(f"case: join at d={d} against zero columns before it, ties={ties}", flush=True)
+    n = 1501
+    X = _points_with_ties(n, d, 190 + d, ties)
+    lead = min(255 - d, 7)
+    P = np.zeros((n, d + lead), np.float32)
+    P[:, lead:] = X
+    for keep in (0, 2, 4, 8):
+        p = api.default_params(join_keep=keep, bucket_cap=1024)
+        a = api.NNDescent(ctx, X, iteration=3, params=p)
+        b = api.NNDescent(ctx, P, iteration=3, params=p)
+        assert ctx.nnd_stats()["bucket_drops"] == 0
+        np.testing.assert_array_equal(a["label"], b["label"])
+        np.testing.assert_array_equal(a["distance"].view(np.uint32), b["distance"].view(np.uint32))
+    for i in range(0, n, 150):
+        np.testing.assert_array_equal(a["distance"][i], np.array([O.d2(X[i], X[j]) for j in a["label"][i]], np.float32))
