@@ -72,6 +72,7 @@ struct NndBufs {
   // one aligned 64- or 128-byte row brings both; otherwise rows = X
   // (rstride = d) and the bounds are an array of their own (wstride = 1).
   float* worst;
+  const float* norms;  // BF16 join: |x|^2 of every point
   const float* rows;
   int rstride;
   int wstride;
@@ -1091,16 +1092,26 @@ __global__ __launch_bounds__(kJoinWaves * 64, 4) void k_nnd_join_wide(const floa
 }
 
 // BF16 join (distance_mode 1): the 64 x 64 Gram matrix of the candidates is
-// computed with v_mfma_f32_16x16x32_bf16 (BF16 inputs, FP32 accumulation)
-// from the FP32 rows staged in LDS, with the operands swapped so that lane l
-// holds row I*16 + (l % 16) and columns J*16 + 4*(l / 16) + q of tile (I, J).
-// Each lane ranks its rows' partners by the approximate |x|^2 + |y|^2 - 2 x.y
-// (32-bit keys), the four lanes that share a row merge their shortlists, and
-// each candidate's SHORT nearest partners are re-ranked with the exact FP32
-// formula, so proposals -- and therefore lists, core distances and MST
-// weights -- carry exact FP32 distances only.
+// computed with v_mfma_f32_16x16x32_bf16 (BF16 inputs, FP32 accumulation),
+// with the operands swapped so that lane l holds row I*16 + (l % 16) and
+// columns J*16 + 4*(l / 16) + q of tile (I, J).  Each lane ranks its rows'
+// partners by the approximate |x|^2 + |y|^2 - 2 x.y (32-bit keys), the four
+// lanes that share a row merge their shortlists, and each candidate's SHORT
+// nearest partners are re-ranked with the exact FP32 formula, so proposals --
+// and therefore lists, core distances and MST weights -- carry exact FP32
+// distances only.
 // Lane layout of the 16x16x32 instruction: A/B lane l holds row (l % 16),
 // k = 8*(l/16) .. +7; the result lane l holds rows 4*(l/16) + q, column l % 16.
+// The gather uses that layout: lane l loads 8 columns of its row of each
+// tile, which are the tile's fragment once rounded (one for both operands),
+// and all 16 tiles accumulate in registers.  The re-rank gathers the rows a
+// second time, 32 columns at a time through LDS, and every lane adds each
+// chunk to the distances of its whole shortlist: reading them again (from a
+// cache, mostly) keeps the LDS of a wave at 10 KB and its chains in parallel,
+// where holding 64 whole FP32 rows left four waves to a CU, each ranking one
+// partner after the other.  A launch at 100k x 128 and join_keep 4 takes 0.85
+// ms (2.25 in that form; 0.99 with the next chunk's columns in registers of
+// their own, which spill).
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -1114,54 +1125,90 @@ __device__ __forceinline__ void merge_short(uint32_t (&a)[N], int xor_mask) {
 }
 
 template <bool NEWNEW, int KEEP, int SHORT>
-__global__ __launch_bounds__(64) void k_nnd_join_mfma(const float* __restrict__ X, int64_t n, int d, int dp, int S,
+__global__ __launch_bounds__(64, SHORT <= 6 ? 3 : 2) void k_nnd_join_mfma(const float* __restrict__ X, int64_t n, int d, int dp, int S,
                                                       NndBufs b) {
   constexpr int WPB = 1;
   constexpr int kSlots = KEEP == 0 ? 2 : KEEP;
   constexpr int kShort = SHORT;  // BF16 shortlist re-ranked in FP32 per candidate
   static_assert(KEEP == 0 ? SHORT == 2 : SHORT >= KEEP, "the shortlist holds the kept partners");
   constexpr uint32_t kNone = 0xFFFFFFFFu;
-  extern __shared__ __attribute__((aligned(16))) float lds_dyn[];
+  constexpr int kRs = 36;  // LDS row stride of a 32-column chunk (16-byte aligned rows)
+  __shared__ __attribute__((aligned(16))) float s_vec[64 * kRs];
   __shared__ uint32_t s_new[WPB][64];
   __shared__ uint32_t s_old[WPB][64];
   __shared__ uint32_t s_cand[WPB][64];
   __shared__ float s_norm[64];
   const unsigned lane = __lane_id();
   const int64_t p = blockIdx.x;
-  const int rs = dp + 4;  // fp32 row stride (16-byte aligned rows)
-  float* vec = lds_dyn;   // 64 x rs
 
   int nn, nc, rev_drop;
   join_candidates(b, p, p < n, S, s_new[0], s_old[0], s_cand[0], &nn, &nc, &rev_drop);
 
-  // stage the FP32 rows, lane c loading candidate c's row so that all 64
-  // gathers are in flight together (zero rows past nc, zero columns past d)
-  {
-    float* dst = vec + static_cast<int64_t>(lane) * rs;
-    int k0 = 0;
-    if (static_cast<int>(lane) < nc) {
-      const float* src = X + static_cast<int64_t>(s_cand[0][lane]) * d;
-      if ((d & 3) == 0) {
-        for (; k0 < d; k0 += 4) *reinterpret_cast<float4*>(dst + k0) = *reinterpret_cast<const float4*>(src + k0);
-      } else {
-        for (; k0 < d; ++k0) dst[k0] = src[k0];
+  const bool active = lane < static_cast<unsigned>(nc);
+  const uint32_t my_id = active ? s_cand[0][lane] : 0u;
+  const float lim = active ? b.worst[static_cast<int64_t>(my_id) * b.wstride] : 0.0f;
+  s_norm[lane] = active ? b.norms[my_id] : 0.0f;
+  const int tiles = (nc + 15) >> 4;
+  const int r16 = static_cast<int>(lane & 15), kq = static_cast<int>(lane >> 4);
+  const bool vec4 = (d & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;  // uniform
+  // this lane's row of tile I, from its first column 8 kq on
+  const float* src[4];
+  bool has[4];
+#pragma unroll
+  for (int I = 0; I < 4; ++I) {
+    has[I] = I * 16 + r16 < nc;
+    src[I] = X + static_cast<int64_t>(has[I] ? s_cand[0][I * 16 + r16] : 0u) * d + 8 * kq;
+  }
+  // columns [k0 + 8 kq, + 8) of those rows; zeros past d and past nc
+  auto load = [&](int k0, float (&v)[4][8]) {
+#pragma unroll
+    for (int I = 0; I < 4; ++I) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[I][e] = 0.0f;
+      if (I < tiles && has[I]) {
+        const int left = d - k0 - 8 * kq;
+        if (vec4) {
+          if (left >= 4) {
+            const float4 x = *reinterpret_cast<const float4*>(src[I] + k0);
+            v[I][0] = x.x, v[I][1] = x.y, v[I][2] = x.z, v[I][3] = x.w;
+          }
+          if (left >= 8) {
+            const float4 x = *reinterpret_cast<const float4*>(src[I] + k0 + 4);
+            v[I][4] = x.x, v[I][5] = x.y, v[I][6] = x.z, v[I][7] = x.w;
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (e < left) v[I][e] = src[I][k0 + e];
+        }
       }
     }
-    for (int k = k0; k < dp; ++k) dst[k] = 0.0f;
-    float nrm = 0.0f;
-    for (int k = 0; k < dp; k += 4) {  // dp is a multiple of 32; rows are 16-byte aligned
-      const float4 x = *reinterpret_cast<const float4*>(dst + k);
-      nrm = __builtin_fmaf(x.x, x.x, nrm);
-      nrm = __builtin_fmaf(x.y, x.y, nrm);
-      nrm = __builtin_fmaf(x.z, x.z, nrm);
-      nrm = __builtin_fmaf(x.w, x.w, nrm);
+  };
+  f32x4_t acc[4][4];
+#pragma unroll
+  for (int I = 0; I < 4; ++I)
+#pragma unroll
+    for (int J = 0; J < 4; ++J) acc[I][J] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  float cur[4][8];
+  load(0, cur);
+  for (int k0 = 0; k0 < dp; k0 += 32) {
+    bf16x8_t f[4];
+#pragma unroll
+    for (int I = 0; I < 4; ++I) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[I][e] = static_cast<__bf16>(cur[I][e]);
     }
-    s_norm[lane] = nrm;
+    if (k0 + 32 < dp) load(k0 + 32, cur);  // uniform: in flight during this chunk's products
+#pragma unroll
+    for (int I = 0; I < 4; ++I)
+#pragma unroll
+      for (int J = 0; J < 4; ++J)
+        // uniform; old x old tiles are never joined
+        if (I < tiles && J < tiles && !(I * 16 >= nn && J * 16 >= nn))
+          acc[I][J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[J], f[I], acc[I][J], 0, 0, 0);
   }
   __syncthreads();
 
-  const int tiles = (nc + 15) >> 4;
-  const int r16 = static_cast<int>(lane & 15), kq = static_cast<int>(lane >> 4);
   uint32_t sl[4][kShort];
 #pragma unroll
   for (int I = 0; I < 4; ++I) {
@@ -1171,26 +1218,15 @@ __global__ __launch_bounds__(64) void k_nnd_join_mfma(const float* __restrict__ 
       const int row = I * 16 + r16;
       const bool row_new = row < nn, row_live = row < nc;
       const float nrow = s_norm[row];
-      for (int J = 0; J < tiles; ++J) {
-        if (I * 16 >= nn && J * 16 >= nn) continue;  // old x old tile: never joined
-        f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int k0 = 0; k0 < dp; k0 += 32) {
-          const float* ra = vec + (J * 16 + r16) * rs + k0 + 8 * kq;
-          const float* rb = vec + (I * 16 + r16) * rs + k0 + 8 * kq;
-          bf16x8_t fa, fb;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            fa[e] = static_cast<__bf16>(ra[e]);
-            fb[e] = static_cast<__bf16>(rb[e]);
-          }
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb, acc, 0, 0, 0);
-        }
+      for (int J = 0; J < 4; ++J) {
+        if (J >= tiles || (I * 16 >= nn && J * 16 >= nn)) continue;  // uniform
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int col = J * 16 + 4 * kq + q;
           const bool ok = row_live && col < nc && col != row &&
                           (row_new ? (NEWNEW || col >= nn) : (col < nn));
-          const float a = nrow + s_norm[col] - 2.0f * acc[q];
+          const float a = nrow + s_norm[col] - 2.0f * acc[I][J][q];
           const uint32_t key = ok ? ((order_bits(a) & ~63u) | static_cast<uint32_t>(col)) : kNone;
           if (KEEP == 0) {
             if (col < nn) sl[I][0] = key < sl[I][0] ? key : sl[I][0];
@@ -1225,27 +1261,68 @@ __global__ __launch_bounds__(64) void k_nnd_join_mfma(const float* __restrict__ 
     mine[s] = kq == 0 ? v0 : (kq == 1 ? v1 : (kq == 2 ? v2 : v3));
   }
 
-  const bool active = lane < static_cast<unsigned>(nc);
-  const uint32_t my_id = active ? s_cand[0][lane] : 0u;
-  // exact FP32 re-rank of the shortlist
+  // exact FP32 re-rank of the shortlist (zeros past d add nothing)
+  int js[kShort];
+  float e[kShort];
+#pragma unroll
+  for (int s = 0; s < kShort; ++s) {
+    js[s] = mine[s] == kNone ? 0 : static_cast<int>(mine[s] & 63u);
+    e[s] = 0.0f;
+  }
+  load(0, cur);
+  for (int k0 = 0; k0 < dp; k0 += 32) {
+    wave_sync();  // the previous chunk has been read
+#pragma unroll
+    for (int I = 0; I < 4; ++I) {
+      float* dst = s_vec + (I * 16 + r16) * kRs + 8 * kq;
+      *reinterpret_cast<float4*>(dst) = make_float4(cur[I][0], cur[I][1], cur[I][2], cur[I][3]);
+      *reinterpret_cast<float4*>(dst + 4) = make_float4(cur[I][4], cur[I][5], cur[I][6], cur[I][7]);
+    }
+    wave_sync();
+    if (k0 + 32 < dp) load(k0 + 32, cur);  // uniform: in flight during this chunk's sums
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const float4 x = *reinterpret_cast<const float4*>(s_vec + lane * kRs + 4 * q);
+#pragma unroll
+      for (int s = 0; s < kShort; ++s) {
+        const float4 y = *reinterpret_cast<const float4*>(s_vec + js[s] * kRs + 4 * q);
+        float diff = x.x - y.x;
+        e[s] = __builtin_fmaf(diff, diff, e[s]);
+        diff = x.y - y.y;
+        e[s] = __builtin_fmaf(diff, diff, e[s]);
+        diff = x.z - y.z;
+        e[s] = __builtin_fmaf(diff, diff, e[s]);
+        diff = x.w - y.w;
+        e[s] = __builtin_fmaf(diff, diff, e[s]);
+      }
+    }
+  }
   uint64_t top[kSlots];
 #pragma unroll
   for (int s = 0; s < kSlots; ++s) top[s] = kKeyMax;
 #pragma unroll
   for (int s = 0; s < kShort; ++s) {
     if (!active || mine[s] == kNone) continue;
-    const int j = static_cast<int>(mine[s] & 63u);
-    const float e = (d & 3) == 0 ? d2_vec4(vec + lane * rs, vec + j * rs, d) : d2_any(vec + lane * rs, vec + j * rs, d);
-    const uint64_t key = make_key(e, s_cand[0][j], 1u);
+    const uint64_t key = make_key(e[s], s_cand[0][js[s]], 1u);
     if (KEEP == 0) {
-      if (j < nn) top[0] = key < top[0] ? key : top[0];
+      if (js[s] < nn) top[0] = key < top[0] ? key : top[0];
       else top[1] = key < top[1] ? key : top[1];
     } else {
       top_insert<kSlots>(top, key);
     }
   }
-  join_emit<WPB, kSlots>(b, top, active, my_id, active ? b.worst[static_cast<int64_t>(my_id) * b.wstride] : 0.0f,
-                         nc, rev_drop);
+  join_emit<WPB, kSlots>(b, top, active, my_id, lim, nc, rev_drop);
+}
+
+// |x|^2 of every point in dimension order (the BF16 join's ranking).
+__global__ __launch_bounds__(256) void k_nnd_norms(const float* __restrict__ X, int64_t n, int d,
+                                                   float* __restrict__ norms) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const float* r = X + i * d;
+  float s = 0.0f;
+  for (int k = 0; k < d; ++k) s = __builtin_fmaf(r[k], r[k], s);
+  norms[i] = s;
 }
 
 // ----------------------------------------------------------- list update --
@@ -1594,6 +1671,13 @@ static int get_bufs(hdb_ctx* ctx, const float* X, int64_t n, int d, const hdb_pa
     b->wstride = rs;
   } else {
     HDB_CALL(scratch_t(ctx, kSlotWorst, n, &b->worst));
+    if (prm.distance_mode >= 1) {
+      float* norms;
+      HDB_CALL(scratch_t(ctx, kSlotNndRows, n, &norms));
+      hipLaunchKernelGGL(k_nnd_norms, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, X, n, d, norms);
+      HDB_LAUNCHED();
+      b->norms = norms;
+    }
     b->rows = X;
     b->rstride = d;
     b->wstride = 1;
@@ -1608,6 +1692,7 @@ static int get_bufs(hdb_ctx* ctx, const float* X, int64_t n, int d, const hdb_pa
   b->join_keep = prm.join_keep;
   b->distance_mode = prm.distance_mode;
   b->iter = 0;
+  if (prm.distance_mode == 0) b->norms = nullptr;
   b->rerank_deep = prm.rerank_keep == 16 ? 1 : 0;
   return HDB_OK;
 }
@@ -1677,14 +1762,13 @@ static int launch_join_wide(hdb_ctx* ctx, const float* X, int64_t n, int d, int 
 template <bool NEWNEW, int KEEP>
 static int launch_join_mfma_k(hdb_ctx* ctx, const float* X, int64_t n, int d, int S, const NndBufs& b) {
   const int dp = (d + 31) & ~31;
-  const size_t lds = static_cast<size_t>(64) * (dp + 4) * sizeof(float);
   constexpr int kShort = KEEP == 0 ? 2 : KEEP + 2;
   constexpr int kDeep = KEEP == 0 ? 2 : 16;
   if (b.rerank_deep)
-    hipLaunchKernelGGL((k_nnd_join_mfma<NEWNEW, KEEP, kDeep>), dim3(static_cast<unsigned>(n)), dim3(64), lds,
+    hipLaunchKernelGGL((k_nnd_join_mfma<NEWNEW, KEEP, kDeep>), dim3(static_cast<unsigned>(n)), dim3(64), 0,
                        ctx->stream, X, n, d, dp, S, b);
   else
-    hipLaunchKernelGGL((k_nnd_join_mfma<NEWNEW, KEEP, kShort>), dim3(static_cast<unsigned>(n)), dim3(64), lds,
+    hipLaunchKernelGGL((k_nnd_join_mfma<NEWNEW, KEEP, kShort>), dim3(static_cast<unsigned>(n)), dim3(64), 0,
                        ctx->stream, X, n, d, dp, S, b);
   HDB_LAUNCHED();
   return HDB_OK;

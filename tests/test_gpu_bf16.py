@@ -32,3 +32,25 @@ def test_bf16_join_exact_distances_and_recall(ctx):
     j = ids[:, 31]
     f64 = np.sqrt(((X.astype(np.float64) - X[j].astype(np.float64)) ** 2).sum(1))
     assert np.max(np.abs(core - f64) / f64) < 1e-6
+
+
+@pytest.mark.parametrize("d", [5, 20, 33, 66, 101, 127, 160])
+def test_bf16_join_ragged_dimensions(ctx, d):
+    """Zero columns change neither the BF16 products nor the exact distances:
+    dimensions off the 32-column chunks (and rows that are not 16-byte
+    aligned) give the lists of the padded points, bit for bit, for every
+    join_keep and re-rank depth; stored distances are the oracle's."""
+    print(f"case: BF16 join at d={d} against its padded points", flush=True)
+    n = 2003
+    X = datasets.tiny_blobs(n, d, 6, seed=300 + d, spread=4.0)
+    P = np.zeros((n, (d + 31) // 32 * 32), np.float32)
+    P[:, :d] = X
+    for keep, rerank in ((0, 0), (1, 0), (2, 16), (4, 0), (4, 16), (8, 0)):
+        p = api.default_params(join_keep=keep, rerank_keep=rerank, distance_mode=1, bucket_cap=1024)
+        a = api.NNDescent(ctx, X, iteration=3, params=p)
+        b = api.NNDescent(ctx, P, iteration=3, params=p)
+        assert ctx.nnd_stats()["bucket_drops"] == 0
+        np.testing.assert_array_equal(a["label"], b["label"])
+        np.testing.assert_array_equal(a["distance"].view(np.uint32), b["distance"].view(np.uint32))
+    for i in range(0, n, 200):
+        np.testing.assert_array_equal(a["distance"][i], np.array([O.d2(X[i], X[j]) for j in a["label"][i]], np.float32))
