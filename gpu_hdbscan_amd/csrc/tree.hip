@@ -62,23 +62,23 @@ constexpr int kLkBits = 10;             // segments of 1024 edges are finished i
 constexpr int kLkEdges = 1 << kLkBits;  // one per thread of k_lk_local
 constexpr int32_t kNoName = INT_MAX;
 
-// Entries of the union-find are read and written with device-scope
-// atomics: the union kernel's blocks run on every XCD, each behind its own
-// L2, and a plain load could keep returning a line that another XCD has
-// since changed (a failed compare-and-swap would then retry forever).
+// Entries of the union-find only ever fall, from an element to one of its
+// ancestors, so a stale value (another XCD's L2 may hold a newer one) is
+// still an ancestor: finds use plain cached loads, and path halving, which
+// rewrites non-roots only, may race harmlessly with other finds and hooks.
+// Only the hook itself decides what is a root, with a compare-and-swap at
+// device scope.
 __device__ __forceinline__ int32_t uf_load(const int32_t* uf, int32_t x) {
-  return __hip_atomic_load(uf + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return __hip_atomic_load(uf + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
 
-// Root of x; roots only ever point to smaller roots, so entries decrease
-// along a path and path halving (which rewrites only non-roots, each to one
-// of its ancestors) may race harmlessly with other finds and hooks.
+// Root of x, as far as this XCD knows.
 __device__ __forceinline__ int32_t uf_find(int32_t* uf, int32_t x) {
   int32_t cur = uf_load(uf, x);
   if (cur != x) {
     int32_t next, prev = x;
     while (cur > (next = uf_load(uf, cur))) {
-      __hip_atomic_store(uf + prev, next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(uf + prev, next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
       prev = cur;
       cur = next;
     }
@@ -86,7 +86,9 @@ __device__ __forceinline__ int32_t uf_find(int32_t* uf, int32_t x) {
   return cur;
 }
 
-// The larger root is hooked under the smaller with a compare-and-swap.
+// The larger root c is hooked under the smaller.  A failed swap returns what
+// c points to by now, a smaller element, and the search goes on from there:
+// every failure moves down, so the loop ends whatever the caches hold.
 __device__ __forceinline__ void uf_join(int32_t* uf, int32_t a, int32_t c) {
   while (true) {
     a = uf_find(uf, a);
@@ -97,7 +99,9 @@ __device__ __forceinline__ void uf_join(int32_t* uf, int32_t a, int32_t c) {
       a = c;
       c = t;
     }
-    if (atomicCAS(&uf[c], c, a) == c) return;
+    const int32_t was = atomicCAS(&uf[c], c, a);
+    if (was == c) return;
+    c = was;
   }
 }
 
@@ -105,7 +109,7 @@ __device__ __forceinline__ void uf_join(int32_t* uf, int32_t a, int32_t c) {
 // read only costs an atomic) is already there: the members of a component
 // arrive roughly in ascending order, so a large one takes few atomics.
 __device__ __forceinline__ void lower_to(int32_t* p, int32_t v) {
-  if (v < uf_load(p, 0)) atomicMin(p, v);
+  if (v < __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(p, v);
 }
 
 // The union-find and the per-component accumulators of one level: names of
@@ -148,54 +152,85 @@ __global__ void k_lk_init(const hdb_mst_edge* __restrict__ e, int64_t m, int64_t
   lk_reset(a, q);
 }
 
+// Combines updates per component in an LDS table before the global atomics:
+// at every level a few huge components take most of them, and same-address
+// atomics serialise (a quarter of a million on one name made the union take
+// 340 us a level at 1M edges).  Linear probing over four slots, one
+// global atomic per root and block; a root that finds no slot goes to the
+// global atomic directly.  Max, min and integer sums do not depend on the
+// order.
+constexpr int kAggSlots = 1024;
+enum class Agg { kMin, kMax, kSum };
+
+template <Agg OP>
+__device__ __forceinline__ void agg_apply(int32_t* p, int32_t v) {
+  if (OP == Agg::kMin) atomicMin(p, v);
+  else if (OP == Agg::kMax) atomicMax(p, v);
+  else atomicAdd(p, v);
+}
+
+template <Agg OP>
+struct AggTable {
+  int32_t keys[kAggSlots], acc[kAggSlots];
+  __device__ __forceinline__ void init() {
+    for (int s = threadIdx.x; s < kAggSlots; s += 256) {
+      keys[s] = -1;
+      acc[s] = OP == Agg::kMin ? INT_MAX : OP == Agg::kMax ? -1 : 0;
+    }
+  }
+  __device__ __forceinline__ void put(int32_t* glob, int32_t root, int32_t v) {
+    uint32_t h = static_cast<uint32_t>(root) * 0x9E3779B1u;
+    h >>= 22;  // 10 bits: kAggSlots
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int slot = static_cast<int>((h + p) & (kAggSlots - 1));
+      const int32_t k = atomicCAS(&keys[slot], -1, root);
+      if (k == -1 || k == root) {
+        agg_apply<OP>(&acc[slot], v);
+        return;
+      }
+    }
+    agg_apply<OP>(&glob[root], v);
+  }
+  __device__ __forceinline__ void flush(int32_t* glob) {
+    for (int s = threadIdx.x; s < kAggSlots; s += 256)
+      if (keys[s] >= 0) agg_apply<OP>(&glob[keys[s]], acc[s]);
+  }
+};
+
 // Level b, first kernel: the first-half edges (bit b clear) of every segment
 // join their ends' components, and the components they touch get their name
-// in the first half.
-__global__ void k_lk_union(int64_t m, int b, const int32_t* __restrict__ vid, LkLevel a) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= m || ((i >> b) & 1)) return;
-  const int32_t v0 = vid[2 * i], v1 = vid[2 * i + 1];
-  lower_to(a.rep_l + v0, static_cast<int32_t>(2 * i));
-  lower_to(a.rep_l + v1, static_cast<int32_t>(2 * i + 1));
-  uf_join(a.uf, v0, v1);
+// in the first half.  `items` edges per thread.
+__global__ __launch_bounds__(256) void k_lk_union(int64_t m, int b, int items, const int32_t* __restrict__ vid,
+                                                  LkLevel a) {
+  __shared__ AggTable<Agg::kMin> name;
+  name.init();
+  __syncthreads();
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * (256 * items);
+  for (int k = 0; k < items; ++k) {
+    const int64_t i = base + k * 256 + threadIdx.x;
+    if (i >= m) break;
+    if ((i >> b) & 1) continue;
+    const int32_t v0 = vid[2 * i], v1 = vid[2 * i + 1];
+    name.put(a.rep_l, v0, static_cast<int32_t>(2 * i));
+    name.put(a.rep_l, v1, static_cast<int32_t>(2 * i + 1));
+    uf_join(a.uf, v0, v1);
+  }
+  __syncthreads();
+  name.flush(a.rep_l);
 }
 
 // Per merged component: its last (highest) first-half edge, its point count
 // (each component a first-half edge touches counts once, at its name) and
-// its name in the second half.  A few huge components take most of the
-// updates at the top levels, so a block combines maxima and sums in two LDS
-// tables keyed by component root (linear probing, four slots) and sends one
-// global atomic per root it saw; a root that finds no slot goes to the
-// global atomic directly.  Max, min and integer sums do not depend on the
-// order.
-constexpr int kAggSlots = 1024;
-
-template <bool MAX>
-__device__ __forceinline__ void agg_put(int32_t* keys, int32_t* acc, int32_t* glob, int32_t root, int32_t v) {
-  uint32_t h = static_cast<uint32_t>(root) * 0x9E3779B1u;
-  h >>= 22;  // 10 bits: kAggSlots
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    const int slot = static_cast<int>((h + p) & (kAggSlots - 1));
-    const int32_t k = atomicCAS(&keys[slot], -1, root);
-    if (k == -1 || k == root) {
-      if (MAX) atomicMax(&acc[slot], v);
-      else atomicAdd(&acc[slot], v);
-      return;
-    }
-  }
-  if (MAX) atomicMax(&glob[root], v);
-  else atomicAdd(&glob[root], v);
-}
-
-// `items` edges per thread.
+// its name in the second half.
 __global__ __launch_bounds__(256) void k_lk_merge(int64_t m, int b, int items, int32_t* __restrict__ vid,
                                                   const int32_t* __restrict__ sz, LkLevel a) {
-  __shared__ int32_t kmax[kAggSlots], vmax[kAggSlots], ksum[kAggSlots], vsum[kAggSlots];
-  for (int s = threadIdx.x; s < kAggSlots; s += 256) {
-    kmax[s] = ksum[s] = vmax[s] = -1;
-    vsum[s] = 0;
-  }
+  __shared__ AggTable<Agg::kMax> last;
+  __shared__ AggTable<Agg::kSum> count;
+  __shared__ AggTable<Agg::kMin> name;
+  last.init();
+  count.init();
+  name.init();
   __syncthreads();
   const int64_t base = static_cast<int64_t>(blockIdx.x) * (256 * items);
   for (int k = 0; k < items; ++k) {
@@ -205,22 +240,21 @@ __global__ __launch_bounds__(256) void k_lk_merge(int64_t m, int b, int items, i
     const int32_t r0 = uf_find(a.uf, v0);
     const int32_t q0 = static_cast<int32_t>(2 * i);
     if (!((i >> b) & 1)) {
-      agg_put<true>(kmax, vmax, a.cmax, r0, static_cast<int32_t>(i));
+      last.put(a.cmax, r0, static_cast<int32_t>(i));
       const int32_t s = (a.rep_l[v0] == q0 ? sz[v0] : 0) + (a.rep_l[v1] == q0 + 1 ? sz[v1] : 0);
-      if (s) agg_put<false>(ksum, vsum, a.csize, r0, s);
+      if (s) count.put(a.csize, r0, s);
     } else {
       const int32_t r1 = uf_find(a.uf, v1);
       vid[2 * i] = r0;
       vid[2 * i + 1] = r1;
-      lower_to(a.rep_r + r0, q0);
-      lower_to(a.rep_r + r1, q0 + 1);
+      name.put(a.rep_r, r0, q0);
+      name.put(a.rep_r, r1, q0 + 1);
     }
   }
   __syncthreads();
-  for (int s = threadIdx.x; s < kAggSlots; s += 256) {
-    if (kmax[s] >= 0) atomicMax(&a.cmax[kmax[s]], vmax[s]);
-    if (ksum[s] >= 0) atomicAdd(&a.csize[ksum[s]], vsum[s]);
-  }
+  last.flush(a.cmax);
+  count.flush(a.csize);
+  name.flush(a.rep_r);
 }
 
 // Every end takes its component's name in its half, and the component's
@@ -780,11 +814,11 @@ int labels_gpu(hdb_ctx* ctx, const hdb_mst_edge* edges, int64_t m, int64_t n, in
                      leaf_par);
   HDB_LAUNCHED();
   const int L = bits_for(m - 1);
-  // edges per thread of k_lk_merge: blocks of 4096 edges where they fill the
+  // edges per thread of k_lk_union and k_lk_merge: blocks of 4096 edges where they fill the
   // chip, fewer where that would leave it idle
   const int items = static_cast<int>(std::min<int64_t>(16, std::max<int64_t>(1, m / (256 * 1024))));
   for (int b = L - 1; b >= kLkBits; --b) {
-    hipLaunchKernelGGL(k_lk_union, dim3(gm), dim3(256), 0, ctx->stream, m, b, vid, cur);
+    hipLaunchKernelGGL(k_lk_union, dim3(grid_for(m, 256 * items)), dim3(256), 0, ctx->stream, m, b, items, vid, cur);
     HDB_LAUNCHED();
     hipLaunchKernelGGL(k_lk_merge, dim3(grid_for(m, 256 * items)), dim3(256), 0, ctx->stream, m, b, items, vid, sz,
                        cur);
