@@ -286,26 +286,37 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
   return lane == 0 ? 0ull : (~0ull >> (64 - lane));
 }
 
-// One DPP move within rows of 16 lanes (every source lane lies in the row,
-// so no lane reads outside it).
+// One DPP move (a lane without a source lane gets 0).
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
-  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, false));
+  return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), CTRL, 0xF, 0xF, true));
+}
+
+// The value of the lane below (lane 0: unspecified), one DPP move each word.
+__device__ __forceinline__ uint32_t lane_below(uint32_t v) { return dpp_u32<0x138>(v); }  // wave_shr:1
+__device__ __forceinline__ uint64_t lane_below(uint64_t v) {
+  return (static_cast<uint64_t>(lane_below(static_cast<uint32_t>(v >> 32))) << 32) | lane_below(static_cast<uint32_t>(v));
 }
 
 // The value of lane (lane ^ j), for a full wave.  j = 1, 2: one DPP
 // quad_perm; j = 4: half-row mirror (i <- 7 - i) then quad reversal
-// (i <- 3 - i), two DPP moves; j = 8: DPP row rotation by 8; j = 16: a
-// ds_swizzle in bit mode (and 0x1f, xor 16); j = 32: a bpermute.  DPP moves
-// are ALU operations, free of the LDS round trip of a swizzle.
+// (i <- 3 - i), two DPP moves; j = 8: DPP row rotation by 8; j = 16, 32:
+// a swap of rows (halves) between two copies and a select.  All are ALU
+// operations, free of the LDS round trip of a swizzle.
 __device__ __forceinline__ uint32_t lane_xor_u32(uint32_t v, int j) {
   switch (j) {
     case 1: return dpp_u32<0xB1>(v);                  // quad_perm(1, 0, 3, 2)
     case 2: return dpp_u32<0x4E>(v);                  // quad_perm(2, 3, 0, 1)
     case 4: return dpp_u32<0x1B>(dpp_u32<0x141>(v));  // quad_perm(3, 2, 1, 0) of row_half_mirror
     case 8: return dpp_u32<0x128>(v);                 // row_ror:8
-    case 16: return static_cast<uint32_t>(__builtin_amdgcn_ds_swizzle(static_cast<int>(v), 0x1f | (16 << 10)));
-    default: return static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), j));
+    case 16: {
+      const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+      return __builtin_amdgcn_inverse_ballot_w64(0x0000FFFF0000FFFFull) ? r[1] : r[0];
+    }
+    default: {
+      const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+      return __builtin_amdgcn_inverse_ballot_w64(0x00000000FFFFFFFFull) ? r[1] : r[0];
+    }
   }
 }
 __device__ __forceinline__ uint64_t lane_xor_u64(uint64_t v, int j) {
@@ -322,32 +333,60 @@ __device__ __forceinline__ T bitonic_ce(T v, T o, bool want_min) {
   return ((o < v) == want_min) ? o : v;
 }
 
+// Lanes whose index has bit j clear (j a power of two below 64).
+__device__ __forceinline__ constexpr uint64_t lanes_without(int j) {
+  return j == 1    ? 0x5555555555555555ull
+         : j == 2  ? 0x3333333333333333ull
+         : j == 4  ? 0x0F0F0F0F0F0F0F0Full
+         : j == 8  ? 0x00FF00FF00FF00FFull
+         : j == 16 ? 0x0000FFFF0000FFFFull
+                   : 0x00000000FFFFFFFFull;
+}
+// Lanes that keep the smaller value in step j of stage k of a bitonic sort
+// of groups of `group` lanes.
+__device__ __forceinline__ constexpr uint64_t bitonic_min_lanes(int group, int k, int j) {
+  return k == group ? lanes_without(j) : ~(lanes_without(j) ^ lanes_without(k));
+}
+
+// The two values of a lane pair (lane, lane ^ j), in either order.
+__device__ __forceinline__ void lane_pair_u32(uint32_t v, int j, uint32_t& a, uint32_t& b) {
+  if (j >= 16) {
+    // rows (halves) of the two copies swapped: both lanes of a pair then
+    // hold both values, without an LDS round trip
+    const auto r = j == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false)
+                           : __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    a = r[0];
+    b = r[1];
+  } else {
+    a = v;
+    b = lane_xor_u32(v, j);
+  }
+}
+
 // Bitonic sort (ascending) of one u64 per lane within aligned groups of
 // GROUP lanes (GROUP = 32 or 64).
 template <int GROUP>
 __device__ __forceinline__ uint64_t bitonic_group(uint64_t v) {
-  const unsigned lane = __lane_id() & (GROUP - 1);
 #pragma unroll
   for (int k = 2; k <= GROUP; k <<= 1) {
 #pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      const bool up = (k == GROUP) ? true : ((lane & k) == 0);
-      const bool low = (lane & j) == 0;
-      v = bitonic_ce(v, lane_xor_u64(v, j), low == up);
-    }
+    for (int j = k >> 1; j > 0; j >>= 1)
+      v = bitonic_ce(v, lane_xor_u64(v, j), __builtin_amdgcn_inverse_ballot_w64(bitonic_min_lanes(GROUP, k, j)));
   }
   return v;
 }
+// The u32 form takes the minimum and the maximum, which read the other lane
+// by DPP themselves, and one select: three instructions for most steps.
 template <int GROUP>
 __device__ __forceinline__ uint32_t bitonic_group_u32(uint32_t v) {
-  const unsigned lane = __lane_id() & (GROUP - 1);
 #pragma unroll
   for (int k = 2; k <= GROUP; k <<= 1) {
 #pragma unroll
     for (int j = k >> 1; j > 0; j >>= 1) {
-      const bool up = (k == GROUP) ? true : ((lane & k) == 0);
-      const bool low = (lane & j) == 0;
-      v = bitonic_ce(v, lane_xor_u32(v, j), low == up);
+      uint32_t a, b;
+      lane_pair_u32(v, j, a, b);
+      const uint32_t mn = a < b ? a : b, mx = a < b ? b : a;
+      v = __builtin_amdgcn_inverse_ballot_w64(bitonic_min_lanes(GROUP, k, j)) ? mn : mx;
     }
   }
   return v;

@@ -34,10 +34,13 @@
 //                  first 32 distinct keys of the union whatever the proposal
 //                  order.
 #include <algorithm>
+#include <type_traits>
 
 #include "hdb_internal.hpp"
 
 namespace hdb {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kSMax = 16;  // sample list stride (SAMPLE_NUM <= 16)
 // Largest point count: the n x 32 reverse pairs and list entries are
@@ -80,6 +83,8 @@ struct NndBufs {
   int join_keep;
   int distance_mode;  // 0: FP32 join, 1: BF16 MFMA shortlist + exact FP32 re-rank
   int iter;           // iteration index: seeds the rotation of the sample choice
+  uint32_t s_recip;   // floor(2^32 / S) + 1 (S >= 2) and ceil(65536 / S): divisions by the sample count
+  uint32_t s_recip16;
   int rerank_deep;    // BF16 join: re-rank the 16 nearest BF16 partners (else join_keep + 2)
 };
 
@@ -326,6 +331,12 @@ __global__ __launch_bounds__(256) void k_nnd_sample(const hdb_nnd_element* __res
 }
 
 // ------------------------------------------------------------ local join --
+// Lanes below this one in the mask m.
+__device__ __forceinline__ int lanes_below(uint64_t m) {
+  return static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
+}
+
 // Orders a wave's LDS writes before its later LDS reads by other lanes of
 // the same wave: LDS instructions of a wave execute in order, so a compiler
 // fence and scheduling barrier at wavefront scope are enough (the waves of a
@@ -338,14 +349,14 @@ __device__ __forceinline__ void wave_sync() {
 
 // Per point p (one wave): new = sort/dedup(fwd_new + rev_new), old =
 // sort/dedup(fwd_old + rev_old), new -= old (ShrinkGraph :405-510).  The
-// candidate ids land in s_cand (new first).  s_new, s_old and s_cand are
-// this wave's own 64-entry LDS rows: waves run it independently, so no row
-// may be shared with another wave.
-__device__ __forceinline__ void join_candidates(const NndBufs& b, int64_t p, bool live, int S, uint32_t* s_new,
-                                                uint32_t* s_old, uint32_t* s_cand, int* nn_out, int* nc_out,
-                                                int* rev_drop_out) {
+// candidate ids land in s_cand (new first, each kind ascending), the wave's
+// own 64-entry LDS row: waves run it independently.  All 64 slots go through
+// one sort by (id, old before new), where an id's first slot is the one to
+// keep: two sorts of 32, a search of every new id among the old ones and
+// five-instruction sort steps took a third of the join's instructions.
+__device__ __forceinline__ void join_candidates(const NndBufs& b, int64_t p, bool live, int S, uint32_t* s_cand,
+                                                int* nn_out, int* nc_out, int* rev_drop_out) {
   const unsigned lane = __lane_id();
-  const unsigned w = threadIdx.x >> 6;
   uint32_t v = 0xFFFFFFFFu;
   int rev_drop = 0;
   if (live) {  // uniform: p is the wave's point
@@ -364,59 +375,41 @@ __device__ __forceinline__ void join_candidates(const NndBufs& b, int64_t p, boo
     // r (len / S) + floor(r (len mod S) / S); the last term has r (len mod S)
     // < 256, where multiplying by ceil(65536 / S) and shifting is exact.
     const int len = oldk ? lo : ln;
-    int rot = 0;
-    if (ln > S || lo > S) {
-      const uint32_t hn = static_cast<uint32_t>(sample_rotation(static_cast<uint64_t>(2 * pu), b.iter));
-      const uint32_t ho = static_cast<uint32_t>(sample_rotation(static_cast<uint64_t>(2 * pu + 1), b.iter));
-      const int rn = ln > S ? static_cast<int>(hn % static_cast<uint32_t>(ln)) : 0;
-      const int ro = lo > S ? static_cast<int>(ho % static_cast<uint32_t>(lo)) : 0;
-      rot = oldk ? ro : rn;
-    }
-    const uint32_t mS = (65536u + static_cast<uint32_t>(S) - 1u) / static_cast<uint32_t>(S);
     int off = r;
-    if (len > S) {
-      const int q = r * (len / S) + static_cast<int>((static_cast<uint32_t>(r * (len % S)) * mS) >> 16);
-      off = q + rot;
-      off = off >= len ? off - len : off;
+    if (ln > S || lo > S) {
+      int rn = 0, ro = 0;
+      if (ln > S)
+        rn = static_cast<int>(static_cast<uint32_t>(sample_rotation(static_cast<uint64_t>(2 * pu), b.iter)) %
+                              static_cast<uint32_t>(ln));
+      if (lo > S)
+        ro = static_cast<int>(static_cast<uint32_t>(sample_rotation(static_cast<uint64_t>(2 * pu + 1), b.iter)) %
+                              static_cast<uint32_t>(lo));
+      // both quotients on the scalar unit: x / S = x m >> 32 with m =
+      // floor(2^32 / S) + 1, exact for x < 2^28 and 2 <= S <= 16
+      const int qn = S == 1 ? ln : static_cast<int>(__umulhi(static_cast<uint32_t>(ln), b.s_recip));
+      const int qo = S == 1 ? lo : static_cast<int>(__umulhi(static_cast<uint32_t>(lo), b.s_recip));
+      const int q = oldk ? qo : qn, rem = oldk ? lo - qo * S : ln - qn * S, rot = oldk ? ro : rn;
+      if (len > S) {
+        off = r * q + static_cast<int>((static_cast<uint32_t>(r * rem) * b.s_recip16) >> 16) + rot;
+        off = off >= len ? off - len : off;
+      }
     }
     const int cnt = rev ? min(len, S) : (oldk ? co : cn);
     const uint32_t* src = rev ? b.rev_val + (oldk ? s0o : s0n)
                               : reinterpret_cast<const uint32_t*>(oldk ? b.fwd_old : b.fwd_new) + pu * kSMax;
-    if (r < cnt) v = src[rev ? off : r];
+    if (r < cnt) v = (src[rev ? off : r] << 1) | (oldk ? 0u : 1u);  // ids are below 2^26
     if (rev && r == 0 && len > S) rev_drop = len - S;
   }
-  v = bitonic_group_u32<32>(v);
-  const uint32_t prev = __shfl_up(v, 1);
-  const bool keep = v != 0xFFFFFFFFu && ((lane & 31u) == 0 || v != prev);
-  const uint64_t bal = __ballot(keep);
-  const uint32_t half = static_cast<uint32_t>(bal >> (lane & 32u));
-  const int pos = __popc(half & ((1u << (lane & 31u)) - 1u));
-  if (keep) {
-    if (lane < 32) s_new[pos] = v;
-    else s_old[pos] = v;
-  }
-  const int nn0 = __popc(static_cast<uint32_t>(bal));
-  const int no = __popc(static_cast<uint32_t>(bal >> 32));
-  wave_sync();
-  // new -= old (binary search in the sorted old ids)
-  bool keep_new = false;
-  uint32_t x = 0;
-  if (lane < static_cast<unsigned>(nn0)) {
-    x = s_new[lane];
-    int lo = 0, hi = no;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (s_old[mid] < x) lo = mid + 1; else hi = mid;
-    }
-    keep_new = !(lo < no && s_old[lo] == x);
-  }
-  const uint64_t bal2 = __ballot(keep_new);
-  const int nn = __popcll(bal2);
-  if (keep_new) s_cand[__popcll(bal2 & lanemask_lt())] = x;
-  if (lane < static_cast<unsigned>(no)) s_cand[nn + lane] = s_old[lane];
+  v = bitonic_group_u32<64>(v);
+  const uint32_t prev = lane_below(v);
+  const bool keep = v != 0xFFFFFFFFu && (lane == 0 || (v >> 1) != (prev >> 1));
+  const uint64_t all = __ballot(keep), fresh = __ballot(keep && (v & 1u));
+  const uint64_t old = all ^ fresh;
+  const int nn = __popcll(fresh);
+  if (keep) s_cand[(v & 1u) ? lanes_below(fresh) : nn + lanes_below(old)] = v >> 1;
   wave_sync();
   *nn_out = nn;
-  *nc_out = nn + no;
+  *nc_out = nn + __popcll(old);
   *rev_drop_out = rev_drop;
 }
 
@@ -437,8 +430,7 @@ __device__ __forceinline__ void join_emit(const NndBufs& b, uint64_t (&top)[SLOT
     const bool ok = active && top[s] != kKeyMax && key_d2(top[s]) < lim;
     if (!ok) top[s] = kKeyMax;
     const uint64_t m = __ballot(ok);
-    excl += static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
-                                                       __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
+    excl += lanes_below(m);
     wcnt += __popcll(m);
   }
   // reverse-sample drops: lanes 16 and 48 hold them
@@ -508,6 +500,31 @@ __device__ __forceinline__ void top_insert32(uint32_t (&top)[SLOTS], uint32_t ke
   top_insert_med3<SLOTS>(top, key);
 }
 
+// Ranking values of candidate `lane` against candidates 4 Q .. 4 Q + 3:
+// |b|^2 + sum_k (-2 a_k) b_k + |a|^2, the additions in that order with one
+// rounding each (the norms come in as products with 1).  The 4 x 4 x 1 matrix product works on 16 blocks of
+// 4 x 4; with the A operand's block Q broadcast to all of them its rows are
+// the four partners and its column is the lane's own candidate, so both
+// operands are the lanes' own registers and the four results are the lane's.
+template <int D, int Q, int DS>
+__device__ __forceinline__ f32x4 join_quad(const float (&own)[DS], const float (&own2)[D], float own_norm) {
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 acc = __builtin_amdgcn_mfma_f32_4x4x1f32(own_norm, 1.0f, zero, 4, Q, 0);
+#pragma unroll
+  for (int k = 0; k < D; ++k) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(own[k], own2[k], acc, 4, Q, 0);
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(1.0f, own_norm, acc, 4, Q, 0);
+}
+
+// f(integral_constant Q) for Q = Q0 .. Q1 - 1: the block selector of a matrix
+// product is an immediate.
+template <int Q0, int Q1, typename F>
+__device__ __forceinline__ void join_quads(F f) {
+  if constexpr (Q0 < Q1) {
+    f(std::integral_constant<int, Q0>{});
+    join_quads<Q0 + 1, Q1>(f);
+  }
+}
+
 // Partner-split FP32 join for D <= 32.  Phase 1: every candidate ranks each
 // new candidate by |a|^2 + |b|^2 - 2 a.b (so each old-new pair is evaluated
 // once) and old candidates store that value in an LDS block; phase 2: new
@@ -517,38 +534,43 @@ __device__ __forceinline__ void top_insert32(uint32_t (&top)[SLOTS], uint32_t ke
 // distances are then recomputed from the same rows in the same operation
 // order as the other joins, so proposals carry exactly its distances; only the
 // choice among partners whose distances agree to about 1e-4 relative can
-// differ.
+// differ.  Bound by VALU issue.  The ranking values come from the matrix
+// cores, four partners of all 64 candidates in D + 2 products (join_quad),
+// where the vector unit took D multiply-adds per partner and each wave read
+// the partners' rows from LDS again.
+// At 500k x 32 and KEEP = 3 a launch takes 1.17 ms instead of 1.63 (the block
+// and the rows in one buffer: five blocks on a CU, not four); at 1M x 12, where
+// the other work of a wave (sort of the candidates, ranking, emission) is
+// most of it, 1.44 ms as before.
 template <int D, bool NEWNEW, int KEEP>
-__global__ __launch_bounds__(kJoinWaves * 64, 8) void k_nnd_join2(const float* __restrict__ X, int64_t n, int d, int S,
+__global__ __launch_bounds__(kJoinWaves * 64, D <= 16 ? 8 : 5) void k_nnd_join2(const float* __restrict__ X, int64_t n, int d, int S,
                                                                NndBufs b) {
   static_assert(D > 0 && D <= 32, "register-resident rows only");
   constexpr int WPB = kJoinWaves;
   constexpr int kStride = (D + 3) & ~3;
   constexpr int kSlots = KEEP == 0 ? 2 : KEEP;
-  // old x new block: no * (nn + 1) values reach 32 * 33 = 1056 at most
-  // (nn + no <= 64), but rarely pass 384; a wave whose block would not fit
-  // computes its old-new pairs a second time in phase 2 instead.  That keeps
-  // LDS at 20 KB per block, so eight blocks fit a CU, and the launch bound
-  // asks for the registers of eight waves per SIMD (D = 12: 60-64 VGPRs)
+  // Old x new block, rows of kBst values (odd, so the old lanes' stores and
+  // the new lanes' column reads spread over the banks).  An old-new value
+  // with the norms added in the new candidate's order comes from the block;
+  // where no * (nn + 1) passes kBlock (rarely), phase 2 takes the values with
+  // the old candidate's norm first, from the products.
   constexpr int kBlock = 384;
+  constexpr int kBst = 33;
+  // The block's space takes the candidates' rows afterwards, kCols columns
+  // at a time (D = 32: two chunks, which lets five blocks share a CU).
+  constexpr int kCols = D <= 16 ? kStride : 16;
+  constexpr int kRow = kCols == 16 ? 20 : kCols;
+  constexpr int kBuf = 64 * kRow > 32 * kBst ? 64 * kRow : 32 * kBst;
   constexpr uint32_t kNone = 0xFFFFFFFFu;
-  // The norms borrow s_new, and the old-candidate scratch of join_candidates
-  // borrows the wave's own old x new block, which the wave first writes
-  // after that function returns.
-  __shared__ float s_vec[WPB][64 * kStride];
-  __shared__ float s_blk[WPB][kBlock];
-  __shared__ uint32_t s_new[WPB][64];
+  __shared__ __attribute__((aligned(16))) float s_buf[WPB][kBuf];
   __shared__ uint32_t s_cand[WPB][64];
-  static_assert(kBlock >= 64, "old-candidate scratch fits in a wave's block");
   (void)d;
   const unsigned lane = __lane_id();
   const unsigned w = threadIdx.x >> 6;
   const int64_t p = static_cast<int64_t>(blockIdx.x) * WPB + w;
-  // the wave's old-candidate scratch: the first 64 words of its own block
-  uint32_t* s_old_w = reinterpret_cast<uint32_t*>(s_blk[w]);
 
   int nn, nc, rev_drop;
-  join_candidates(b, p, p < n, S, s_new[w], s_old_w, s_cand[w], &nn, &nc, &rev_drop);
+  join_candidates(b, p, p < n, S, s_cand[w], &nn, &nc, &rev_drop);
   const int no = nc - nn;
   const bool active = lane < static_cast<unsigned>(nc);
   const bool is_new = lane < static_cast<unsigned>(nn);
@@ -588,14 +610,6 @@ __global__ __launch_bounds__(kJoinWaves * 64, 8) void k_nnd_join2(const float* _
   float own_norm = 0.0f;
 #pragma unroll
   for (int k = 0; k < D; ++k) own_norm = __builtin_fmaf(own[k], own[k], own_norm);
-  // the norms borrow s_new, free after join_candidates' last barrier
-  float* s_norm = reinterpret_cast<float*>(s_new[w]);
-  s_norm[lane] = own_norm;
-  if (active) {
-#pragma unroll
-    for (int k = 0; k < kStride; ++k) s_vec[w][lane * kStride + k] = own[k];
-  }
-  wave_sync();
 
   // Ranking value |b|^2 + sum_k (-2 a_k) b_k + |a|^2 (-2 a_k is exact).
   // Cancellation can leave it slightly below 0; the key's mask drops the
@@ -603,11 +617,6 @@ __global__ __launch_bounds__(kJoinWaves * 64, 8) void k_nnd_join2(const float* _
   float own2[D];
 #pragma unroll
   for (int k = 0; k < D; ++k) own2[k] = -2.0f * own[k];
-  const uint32_t mask_v = 0x7FFFFFC0u;  // a VGPR operand: VOP3 takes no literal here
-  // old x new block: row o (old candidate nn + o) holds its values against
-  // the new candidates; the odd-or-padded stride nn + 1 keeps the old lanes'
-  // stores and the new lanes' column reads free of bank conflicts
-  const int bst = nn + 1;
   // Phase 1 ranks the lane's own row too (a new lane meets itself among the
   // new partners): one slot more is kept and the lane itself dropped at the
   // end, which leaves the KEEP nearest of the others.  KEEP == 0: slots 0-1
@@ -616,25 +625,12 @@ __global__ __launch_bounds__(kJoinWaves * 64, 8) void k_nnd_join2(const float* _
   uint32_t top[kRank];
 #pragma unroll
   for (int s = 0; s < kRank; ++s) top[s] = kNone;
-  // phase 1: partners among the new candidates, four per step: the rows'
-  // LDS reads are issued before the dot products, and one branch covers
-  // the stores into the new x old block
-  const bool blocked = no * bst <= kBlock;  // uniform
+  const bool blocked = no * (nn + 1) <= kBlock;  // uniform
   const bool store_old = active && !is_new && blocked;
-  float* blk_row = s_blk[w] + (store_old ? (static_cast<int>(lane) - nn) * bst : 0);  // + j
-  auto partner = [&](int j) {
-    const float* row = s_vec[w] + j * kStride;
-    float acc = s_norm[j];
-#pragma unroll
-    for (int k = 0; k < D; ++k) acc = __builtin_fmaf(own2[k], row[k], acc);
-    return acc + own_norm;
-  };
-  auto rank_key = [&](float acc, int j) {
-    // (bits & 0x7FFFFFC0) | j in one instruction; j is wave-uniform
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(__float_as_uint(acc)), "v"(mask_v), "s"(j));
-    return r;
-  };
+  // row o: old candidate nn + o's values against the new candidates
+  float* blk_row = s_buf[w] + (store_old ? (static_cast<int>(lane) - nn) * kBst : 0);  // + j
+  // (bits & 0x7FFFFFC0) | j
+  auto rank_key = [&](float acc, int j) { return (__float_as_uint(acc) & 0x7FFFFFC0u) | static_cast<uint32_t>(j); };
   auto rank_new = [&](int j, float acc) {
     const uint32_t key = rank_key(acc, j);
     if (KEEP == 0) {
@@ -646,28 +642,29 @@ __global__ __launch_bounds__(kJoinWaves * 64, 8) void k_nnd_join2(const float* _
       top_insert32<kRank>(top, key);
     }
   };
-  int j = 0;
-  for (; j + 4 <= nn; j += 4) {  // four partners a step: pointer updates amortise
-    const float a0 = partner(j);
-    const float a1 = partner(j + 1);
-    const float a2 = partner(j + 2);
-    const float a3 = partner(j + 3);
-    if (store_old) {
-      blk_row[j] = a0;
-      blk_row[j + 1] = a1;
-      blk_row[j + 2] = a2;
-      blk_row[j + 3] = a3;
+  // phase 1: partners among the new candidates (at most 32), four per step
+  join_quads<0, 8>([&](auto quad) {
+    constexpr int Q = decltype(quad)::value, j = 4 * Q;
+    if (j >= nn) return;  // uniform, as are the conditions below
+    const f32x4 v = join_quad<D, Q>(own, own2, own_norm);
+    if (j + 4 <= nn) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float a = v[r];
+        if (store_old) blk_row[j + r] = a;
+        rank_new(j + r, a);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        if (j + r < nn) {
+          const float a = v[r];
+          if (store_old) blk_row[j + r] = a;
+          rank_new(j + r, a);
+        }
+      }
     }
-    rank_new(j, a0);
-    rank_new(j + 1, a1);
-    rank_new(j + 2, a2);
-    rank_new(j + 3, a3);
-  }
-  for (; j < nn; ++j) {
-    const float a0 = partner(j);
-    if (store_old) blk_row[j] = a0;
-    rank_new(j, a0);
-  }
+  });
   if (!NEWNEW && is_new) {  // merge mode: new candidates skip new partners
 #pragma unroll
     for (int s = 0; s < kRank; ++s) top[s] = kNone;
@@ -678,7 +675,7 @@ __global__ __launch_bounds__(kJoinWaves * 64, 8) void k_nnd_join2(const float* _
   uint32_t keep_top[kRank];
 #pragma unroll
   for (int s = 0; s < kRank; ++s) keep_top[s] = top[s];
-  const float* blk_col = s_blk[w] + (is_new ? static_cast<int>(lane) : 0);
+  const float* blk_col = s_buf[w] + (is_new ? static_cast<int>(lane) : 0);
   auto rank_old = [&](float acc, int j) {
     const uint32_t key = rank_key(acc, j);
     if (KEEP == 0) top[2] = key < top[2] ? key : top[2];
@@ -686,23 +683,24 @@ __global__ __launch_bounds__(kJoinWaves * 64, 8) void k_nnd_join2(const float* _
   };
   int o = 0;
   if (blocked) {
-    for (; o + 4 <= no; o += 4) {  // four reads in flight a step
-      const float a0 = blk_col[o * bst], a1 = blk_col[(o + 1) * bst];
-      const float a2 = blk_col[(o + 2) * bst], a3 = blk_col[(o + 3) * bst];
+    for (; o + 4 <= no; o += 4, blk_col += 4 * kBst) {  // four reads in flight a step
+      const float a0 = blk_col[0], a1 = blk_col[kBst];
+      const float a2 = blk_col[2 * kBst], a3 = blk_col[3 * kBst];
       rank_old(a0, nn + o);
       rank_old(a1, nn + o + 1);
       rank_old(a2, nn + o + 2);
       rank_old(a3, nn + o + 3);
     }
-    for (; o < no; ++o) rank_old(blk_col[o * bst], nn + o);
+    for (; o < no; ++o, blk_col += kBst) rank_old(*blk_col, nn + o);
   } else {
-    for (; o + 2 <= no; o += 2) {  // the pairs themselves, from the rows
-      const float a0 = partner(nn + o);
-      const float a1 = partner(nn + o + 1);
-      rank_old(a0, nn + o);
-      rank_old(a1, nn + o + 1);
-    }
-    for (; o < no; ++o) rank_old(partner(nn + o), nn + o);
+    join_quads<0, 16>([&](auto quad) {  // the pairs themselves
+      constexpr int Q = decltype(quad)::value, j = 4 * Q;
+      if (j + 4 <= nn || j >= nc) return;
+      const f32x4 v = join_quad<D, Q>(own, own2, own_norm);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (j + r >= nn && j + r < nc) rank_old(v[r], j + r);
+    });
   }
   if (!is_new) {
 #pragma unroll
@@ -723,21 +721,36 @@ __global__ __launch_bounds__(kJoinWaves * 64, 8) void k_nnd_join2(const float* _
     }
   }
   // exact keys of the winners
+  float dist[kSlots];
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s) dist[s] = 0.0f;
+#pragma unroll
+  for (int c = 0; c < D; c += kCols) {
+    wave_sync();
+#pragma unroll
+    for (int k = 0; k < kCols; k += 4)
+      *reinterpret_cast<float4*>(&s_buf[w][lane * kRow + k]) =
+          make_float4(own[c + k], own[c + k + 1], own[c + k + 2], own[c + k + 3]);
+    wave_sync();
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+      // a branch per slot, so that one row's reads are in flight at a time:
+      // with all the slots' reads first the kernel spills
+      if (active && fin[s] != kNone) {
+        const float* row = s_buf[w] + (fin[s] & 63u) * kRow;
+#pragma unroll
+        for (int k = 0; k < kCols && c + k < D; ++k) {
+          const float diff = own[c + k] - row[k];
+          dist[s] = __builtin_fmaf(diff, diff, dist[s]);
+        }
+      }
+    }
+  }
   uint64_t top64[kSlots];
 #pragma unroll
   for (int s = 0; s < kSlots; ++s) {
     top64[s] = kKeyMax;
-    if (active && fin[s] != kNone) {
-      const int j = static_cast<int>(fin[s] & 63u);
-      const float* row = s_vec[w] + j * kStride;
-      float acc = 0.0f;
-#pragma unroll
-      for (int k = 0; k < D; ++k) {
-        const float diff = own[k] - row[k];
-        acc = __builtin_fmaf(diff, diff, acc);
-      }
-      top64[s] = make_key(acc, s_cand[w][j], 1u);
-    }
+    if (active && fin[s] != kNone) top64[s] = make_key(dist[s], s_cand[w][fin[s] & 63u], 1u);
   }
   join_emit<WPB, kSlots>(b, top64, active, my_id, lim, nc, rev_drop);
 }
@@ -841,15 +854,13 @@ __global__ __launch_bounds__(kJoinWaves * 64) void k_nnd_join_rows(int64_t n, in
   constexpr uint32_t kNone = 0xFFFFFFFFu;
   __shared__ __attribute__((aligned(16))) float s_vec[WPB][64 * DP];
   __shared__ float s_blk[WPB][kBlock];
-  __shared__ uint32_t s_new[WPB][64];
   __shared__ uint32_t s_cand[WPB][64];
   const unsigned lane = __lane_id();
   const unsigned w = threadIdx.x >> 6;
   const int64_t p = static_cast<int64_t>(blockIdx.x) * WPB + w;
-  uint32_t* s_old_w = reinterpret_cast<uint32_t*>(s_blk[w]);
 
   int nn, nc, rev_drop;
-  join_candidates(b, p, p < n, S, s_new[w], s_old_w, s_cand[w], &nn, &nc, &rev_drop);
+  join_candidates(b, p, p < n, S, s_cand[w], &nn, &nc, &rev_drop);
   const int no = nc - nn;
   const bool active = lane < static_cast<unsigned>(nc);
   const bool is_new = lane < static_cast<unsigned>(nn);
@@ -978,7 +989,6 @@ __global__ __launch_bounds__(kJoinWaves * 64, 4) void k_nnd_join_wide(const floa
   constexpr uint32_t kNone = 0xFFFFFFFFu;
   __shared__ __attribute__((aligned(16))) float s_buf[WPB][kNew * kM];
   static_assert(kNew * kM >= 64 * kC && (kNew * kM) % 4 == 0, "rows and distances share the buffer");
-  __shared__ uint32_t s_new[WPB][64];
   __shared__ uint32_t s_cand[WPB][64];
   const unsigned lane = __lane_id();
   const unsigned w = threadIdx.x >> 6;
@@ -986,7 +996,7 @@ __global__ __launch_bounds__(kJoinWaves * 64, 4) void k_nnd_join_wide(const floa
   float* buf = s_buf[w];
 
   int nn, nc, rev_drop;
-  join_candidates(b, p, p < n, S, s_new[w], reinterpret_cast<uint32_t*>(buf), s_cand[w], &nn, &nc, &rev_drop);
+  join_candidates(b, p, p < n, S, s_cand[w], &nn, &nc, &rev_drop);
   const int no = nc - nn;
   const bool active = lane < static_cast<unsigned>(nc);
   const bool is_new = lane < static_cast<unsigned>(nn);
@@ -1134,15 +1144,13 @@ __global__ __launch_bounds__(64, SHORT <= 6 ? 3 : 2) void k_nnd_join_mfma(const 
   constexpr uint32_t kNone = 0xFFFFFFFFu;
   constexpr int kRs = 36;  // LDS row stride of a 32-column chunk (16-byte aligned rows)
   __shared__ __attribute__((aligned(16))) float s_vec[64 * kRs];
-  __shared__ uint32_t s_new[WPB][64];
-  __shared__ uint32_t s_old[WPB][64];
   __shared__ uint32_t s_cand[WPB][64];
   __shared__ float s_norm[64];
   const unsigned lane = __lane_id();
   const int64_t p = blockIdx.x;
 
   int nn, nc, rev_drop;
-  join_candidates(b, p, p < n, S, s_new[0], s_old[0], s_cand[0], &nn, &nc, &rev_drop);
+  join_candidates(b, p, p < n, S, s_cand[0], &nn, &nc, &rev_drop);
 
   const bool active = lane < static_cast<unsigned>(nc);
   const uint32_t my_id = active ? s_cand[0][lane] : 0u;
@@ -1350,7 +1358,7 @@ __device__ __forceinline__ uint64_t merge_proposals(uint64_t cur, uint64_t pr, u
   const unsigned lane = __lane_id();
   const uint64_t lt = lanemask_lt();
   pr = bitonic_group<64>(pr);
-  const uint64_t pp = shfl_u64(pr, static_cast<int>((lane + 63) & 63));
+  const uint64_t pp = lane_below(pr);
   const bool kp = pr != kKeyMax && (lane == 0 || pp != pr);
   const uint64_t bp = __ballot(kp);
   const int ppos = __popcll(bp & lt);
@@ -1364,7 +1372,7 @@ __device__ __forceinline__ uint64_t merge_proposals(uint64_t cur, uint64_t pr, u
   uint64_t v = lane < 32 ? cur : pv;
   __builtin_amdgcn_wave_barrier();
   v = bitonic_merge64(v);
-  const uint64_t prev = shfl_u64(v, static_cast<int>((lane + 63) & 63));
+  const uint64_t prev = lane_below(v);
   const bool keep = v != kKeyMax && (lane == 0 || (prev >> 1) != (v >> 1));
   const uint64_t bal = __ballot(keep);
   const int pos = __popcll(bal & lt);
@@ -1806,6 +1814,8 @@ static int iterate(hdb_ctx* ctx, const float* X, int64_t n, int d, int S, bool m
   const int rev_bits = bits_for(2 * n);
   const int tgt_bits = bits_for(n - 1);
   const int64_t ngroups = (n + (1 << kGroupBits) - 1) >> kGroupBits;
+  b.s_recip = S > 1 ? static_cast<uint32_t>((static_cast<uint64_t>(1) << 32) / static_cast<uint32_t>(S)) + 1u : 0u;
+  b.s_recip16 = (65536u + static_cast<uint32_t>(S) - 1u) / static_cast<uint32_t>(S);
   for (int it = 0; it < iterations; ++it) {
     b.iter = it;
     {

@@ -338,3 +338,28 @@ def test_join_wide_dimensions(ctx, d, ties):
         np.testing.assert_array_equal(a["distance"].view(np.uint32), b["distance"].view(np.uint32))
     for i in range(0, n, 150):
         np.testing.assert_array_equal(a["distance"][i], np.array([O.d2(X[i], X[j]) for j in a["label"][i]], np.float32))
+
+
+@pytest.mark.parametrize("d", [12, 32])
+@pytest.mark.parametrize("S", [1, 3, 4, 5, 11, 16])
+def test_join_matrix_values_equal_general(ctx, d, S):
+    """The joins of d = 12 and 32 rank by matrix products.  With small whole
+    coordinates every ranking value is exact, and in merge mode a candidate's
+    partners are of one kind, so ties go to the smaller id in every kernel: a
+    zero column, which takes the same points to the kernels of other
+    dimensions, changes no list.  S moves the candidate counts over the
+    products' blocks of four."""
+    print(f"case: merge join d={d} S={S} against d={d + 1}", flush=True)
+    n = 700
+    X = np.clip(np.round(datasets.tiny_blobs(2 * n, d, 6, seed=7 * d + S, spread=4.0)), -40, 40).astype(np.float32)
+    P = np.zeros((2 * n, d + 1), np.float32)
+    P[:, :d] = X
+    for keep in (0, 1, 2, 3, 4, 8):
+        p = api.default_params(join_keep=keep, merge_sample_num=S, bucket_cap=1024)
+        ga = api.NNDescent(ctx, P[:n], iteration=2, params=p)
+        gb = api.NNDescent(ctx, P[n:], iteration=2, params=p)
+        a = api.KNNMergeFromHost(ctx, X[:n], ga, X[n:], gb, params=p)
+        b = api.KNNMergeFromHost(ctx, P[:n], ga, P[n:], gb, params=p)
+        assert ctx.nnd_stats()["bucket_drops"] == 0
+        np.testing.assert_array_equal(a["label"], b["label"])
+        np.testing.assert_array_equal(a["distance"].view(np.uint32), b["distance"].view(np.uint32))
