@@ -1388,30 +1388,31 @@ __device__ __forceinline__ uint64_t merge_proposals(uint64_t cur, uint64_t pr, u
 }
 
 // The list in lanes 0..31 (sorted, distinct) merged with the proposals
-// `live` marks (each distinct from the list's entries, `pos` = # entries
+// (kKeyMax: none; each distinct from the list's entries, `pos` = # entries
 // below it): every element's new position is counted, with no sort.  Of
-// equal proposals the lowest lane's is kept.  Returns the new list in lanes
-// 0..31; s_top is the wave's 32-entry LDS row.
-__device__ __forceinline__ uint64_t insert_few(uint64_t cur, uint64_t pr, bool live, int pos, uint64_t* s_top) {
+// equal proposals one is kept: the step of the first takes the others out,
+// so a step is two reads, three compares and two additions (about twice
+// that with the repeated proposals found lane by lane: an update of 1M lists
+// at join_keep 3 took 1.04 ms, now 0.85; of 10M at join_keep 2 6.5, now 5.4).
+// Returns the new list in lanes 0..31; s_top is the wave's 32-entry LDS row.
+__device__ __forceinline__ uint64_t insert_few(uint64_t cur, uint64_t pr, int pos, uint64_t* s_top) {
   const unsigned lane = __lane_id();
-  bool dup = false;  // an equal proposal sits in a lower lane
+  const uint64_t live = __ballot(pr != kKeyMax);
+  uint64_t first = 0;  // the lanes whose proposal enters
   int below_cur = 0, below_pr = 0;
-  // uniform loop over the proposals in lane order: when step t is reached,
-  // lane t has met every lower lane, so its dup flag is final
-  for (uint64_t m = __ballot(live); m; m &= m - 1) {
+  for (uint64_t m = live; m;) {  // uniform
     const int t = __builtin_ctzll(m);
     const uint64_t x = (static_cast<uint64_t>(__builtin_amdgcn_readlane(static_cast<uint32_t>(pr >> 32), t)) << 32) |
                        __builtin_amdgcn_readlane(static_cast<uint32_t>(pr), t);
-    if (__builtin_amdgcn_readlane(dup ? 1u : 0u, t)) continue;  // uniform
+    first |= 1ull << t;
+    m &= ~__ballot(pr == x);
     below_cur += x < cur ? 1 : 0;
     below_pr += x < pr ? 1 : 0;
-    dup = dup || (t < static_cast<int>(lane) && (x >> 1) == (pr >> 1));
   }
-  live = live && !dup;
   const int pc = static_cast<int>(lane) + below_cur;
   if (lane < 32u && pc < kK) s_top[pc] = cur;
   const int pp = pos + below_pr;
-  if (live && pp < kK) s_top[pp] = pr;
+  if (((first >> lane) & 1u) && pp < kK) s_top[pp] = pr;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -1500,21 +1501,23 @@ __global__ __launch_bounds__(256, 7) void k_nnd_update(hdb_nnd_element* __restri
           // ranks past the 32nd entry, or equals an entry's (distance, id),
           // cannot change the list: drop it, and skip the merge when none is
           // left.
-          const uint64_t pk = pr >> 1;
           // entries below the proposal, capped at 31, in three dependent
           // rounds of LDS reads (an 8-entry block, a pair within it, then
-          // one entry) where a binary search takes five
-          int pos = ((lst[7] >> 1) < pk ? 8 : 0) + ((lst[15] >> 1) < pk ? 8 : 0) + ((lst[23] >> 1) < pk ? 8 : 0);
-          pos += ((lst[pos + 1] >> 1) < pk ? 2 : 0) + ((lst[pos + 3] >> 1) < pk ? 2 : 0) +
-                 ((lst[pos + 5] >> 1) < pk ? 2 : 0);
-          if ((lst[pos] >> 1) < pk) pos += 1;
+          // one entry) where a binary search takes five.  A proposal carries
+          // flag 1, so an entry's (distance, id) is below its own exactly if
+          // the entry is below the proposal's key with the flag clear.
+          const uint64_t pk = pr & ~1ull;
+          int pos = (lst[7] < pk ? 8 : 0) + (lst[15] < pk ? 8 : 0) + (lst[23] < pk ? 8 : 0);
+          pos += (lst[pos + 1] < pk ? 2 : 0) + (lst[pos + 3] < pk ? 2 : 0) + (lst[pos + 5] < pk ? 2 : 0);
+          if (lst[pos] < pk) pos += 1;
           // lst[pos] >= pk unless all 32 entries are below it (pos = 31)
-          const bool keep = pr != kKeyMax && (lst[pos] >> 1) > pk;
+          pr = lst[pos] > pr ? pr : kKeyMax;
+          const bool keep = pr != kKeyMax;
           const uint64_t km = __ballot(keep);
           if (km == 0) continue;
           // counting costs a step per proposal; past about 32 the sort wins
-          if (__popcll(km) <= 32) cur = insert_few(cur, pr, keep, pos, s_top[w]);
-          else cur = merge_proposals(cur, keep ? pr : kKeyMax, s_prop[w], s_top[w]);
+          if (__popcll(km) <= 32) cur = insert_few(cur, pr, pos, s_top[w]);
+          else cur = merge_proposals(cur, pr, s_prop[w], s_top[w]);
         } else {
           cur = merge_proposals(cur, pr, s_prop[w], s_top[w]);
         }
