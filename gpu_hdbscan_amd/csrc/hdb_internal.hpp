@@ -454,8 +454,10 @@ int radix_sort_u32_u64(hdb_ctx* ctx, uint32_t* keys, uint64_t* vals, int64_t n, 
 int radix_sort_u32_u32(hdb_ctx* ctx, uint32_t* keys, uint32_t* vals, int64_t n, int bit0, int bit1);
 // seg_start/seg_end[k] = [first, last+1) position of segment k = key >> shift
 // in keys sorted by that value (k < nseg); untouched segments keep 0.
+// count: a device pointer to the number of keys where the host does not know
+// it (at most m), or nullptr.
 int segment_bounds(hdb_ctx* ctx, const uint32_t* sorted_keys, int64_t m, int64_t nseg, int32_t* seg_start,
-                   int32_t* seg_end, int shift = 0);
+                   int32_t* seg_end, int shift = 0, const int64_t* count = nullptr);
 // The same with int64 positions (for streams that may pass 2^31 keys).
 int segment_bounds(hdb_ctx* ctx, const uint32_t* sorted_keys, int64_t m, int64_t nseg, int64_t* seg_start,
                    int64_t* seg_end, int shift = 0);
@@ -472,6 +474,11 @@ int radix_sort_u32_u64_segs(hdb_ctx* ctx, uint32_t* keys, uint64_t* vals, int64_
                             int nseg, int64_t seg_cap, int bit0, int bit1, uint32_t** kout, uint64_t** vout);
 int radix_sort_u32_u32_out(hdb_ctx* ctx, uint32_t* keys, uint32_t* vals, int64_t n, int bit0, int bit1,
                            uint32_t** kout, uint32_t** vout);
+// The same without the keys equal to `drop` (past every other key): *count
+// receives a device pointer to the number of the others, in the sort's
+// scratch (valid until the next sort), or nullptr where all were kept.
+int radix_sort_u32_u32_drop(hdb_ctx* ctx, uint32_t* keys, uint32_t* vals, int64_t n, int bit0, int bit1, uint32_t drop,
+                            uint32_t** kout, uint32_t** vout, const int64_t** count);
 int read_i64(hdb_ctx* ctx, const int64_t* p, int64_t* out);
 // Queue a copy of *p into pinned word `slot` (0 or 1) and mark it with
 // event `slot`; wait_i64 waits for that event only, so kernels queued after

@@ -264,7 +264,8 @@ __global__ __launch_bounds__(256) void k_nnd_init_merge(const float* __restrict_
 // that win an LDS atomic); in merge mode old entries are kept only from the
 // list's own half (PrepareGraphForMerge :100-166).  Every forward sample q of p becomes the
 // reverse pair (2q + old, p) at slot 16n*old + 16p + rank; unused slots get
-// the key 2n, which sorts after every real key.  New pairs all precede old
+// the key 2n, past every real key, which the sort leaves out (half the slots
+// of the first iteration, a quarter of the later ones).  New pairs all precede old
 // ones, so a stable sort on the key without its low bit orders the pairs by
 // the whole key (q, then new before old, then p).
 template <bool MERGE>
@@ -320,10 +321,8 @@ __global__ __launch_bounds__(256) void k_nnd_sample(const hdb_nnd_element* __res
       rv_old[r] = static_cast<uint32_t>(p);
     }
   }
-  if ((j < 16 && static_cast<int>(j) >= nn) || (j >= 16 && static_cast<int>(j) - 16 >= no)) {
+  if ((j < 16 && static_cast<int>(j) >= nn) || (j >= 16 && static_cast<int>(j) - 16 >= no))
     b.rev_key[half + (j & 15u)] = sentinel;
-    b.rev_val[half + (j & 15u)] = 0u;
-  }
   if (j == 0) {
     b.fwd_new_n[p] = nn;
     b.fwd_old_n[p] = no;
@@ -1838,8 +1837,10 @@ static int iterate(hdb_ctx* ctx, const float* X, int64_t n, int d, int S, bool m
       Stage st(ctx, "nnd_reverse_sort");
       uint32_t* rk = nullptr;
       // bit 0 (the kind) is already ordered: new pairs precede old ones
-      HDB_CALL(radix_sort_u32_u32_out(ctx, b.rev_key, b.rev_val, n * 32, 1, rev_bits, &rk, &bj.rev_val));
-      HDB_CALL(segment_bounds(ctx, rk, n * 32, 2 * n, b.rev_s, b.rev_e));
+      const int64_t* pairs = nullptr;
+      HDB_CALL(radix_sort_u32_u32_drop(ctx, b.rev_key, b.rev_val, n * 32, 1, rev_bits, static_cast<uint32_t>(2 * n),
+                                       &rk, &bj.rev_val, &pairs));
+      HDB_CALL(segment_bounds(ctx, rk, n * 32, 2 * n, b.rev_s, b.rev_e, 0, pairs));
       HDB_CALL(fill_u64(ctx, reinterpret_cast<uint64_t*>(b.prop_cnt), kPropSegs * kCtrStride, 0));
     }
     {

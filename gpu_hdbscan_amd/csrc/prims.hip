@@ -223,13 +223,25 @@ __device__ __forceinline__ int64_t rs_walk_phys(const RsSegs& sg, const int64_t*
   return static_cast<int64_t>(wk.seg) * sg.seg_cap + (i - s_pre[wk.seg]);
 }
 
+// Keys equal to `drop` leave the sort in its first pass (DROP kernels),
+// which leaves the number of the others at *count; the later passes read it
+// there.  count == nullptr: a plain sort.  (The reverse pairs of the kNN graph
+// fill half to nine tenths of their slots: path at 1M x 12 32.8 -> 32.1 ms, at
+// 10M 393 -> 387 ms.)
+template <typename K>
+struct RsDrop {
+  int64_t* count;
+  K drop;
+};
+
 // SEG: the input is read through a segment map (the first pass of a
 // segmented sort); otherwise logical and physical indices agree and the
 // chunk addresses are not kept in registers.
-template <typename K, bool SEG, int WAVES, int CH>
+template <typename K, bool SEG, bool DROP, int WAVES, int CH>
 __global__ __launch_bounds__(WAVES * 64) void k_rs_hist(const K* __restrict__ keys, int64_t n, int shift,
-                                                        int32_t* __restrict__ hist, RsSegs sg) {
+                                                        int32_t* __restrict__ hist, RsSegs sg, RsDrop<K> dr) {
   constexpr int kBlock = WAVES * 64;
+  if (!SEG && !DROP && dr.count) n = *dr.count;  // tiles past it count nothing
   __shared__ int32_t h[kRsBins];
   __shared__ int64_t s_pre[SEG ? kRsMaxSegs + 1 : 1];
   for (int i = threadIdx.x; i < kRsBins; i += kBlock) h[i] = 0;
@@ -256,7 +268,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_rs_hist(const K* __restrict__ ke
   }
 #pragma unroll
   for (int c = 0; c < CH; ++c)
-    if (wbase + c * 64 + lane < n) atomicAdd(&h[static_cast<unsigned>(kv[c] >> shift) & 0xFFu], 1);
+    if (wbase + c * 64 + lane < n && !(DROP && kv[c] == dr.drop)) atomicAdd(&h[static_cast<unsigned>(kv[c] >> shift) & 0xFFu], 1);
   __syncthreads();
   // tile-major: the block's 256 counts are one contiguous 1 KB row
   for (int i = threadIdx.x; i < kRsBins; i += kBlock) hist[static_cast<int64_t>(blockIdx.x) * kRsBins + i] = h[i];
@@ -370,14 +382,14 @@ __device__ __forceinline__ uint64_t rs_match(unsigned dg, bool act) {
 // Stable ranks of one wave's CH chunks: rank[c] = keys of the same digit
 // before this one in the wave; wcnt (the wave's 256 counters, zero on entry)
 // ends as the wave's digit counts.
-template <typename K, int CH>
-__device__ __forceinline__ void rs_wave_ranks(const K (&key)[CH], int64_t wbase, int64_t n, int shift, uint16_t* wcnt,
-                                              uint8_t (&dig)[CH], int32_t (&rank)[CH]) {
+template <typename K, bool DROP, int CH>
+__device__ __forceinline__ void rs_wave_ranks(const K (&key)[CH], int64_t wbase, int64_t n, int shift, K drop,
+                                              uint16_t* wcnt, uint8_t (&dig)[CH], int32_t (&rank)[CH]) {
   const unsigned lane = __lane_id();
   const uint64_t lt = lanemask_lt();
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const bool act = wbase + c * 64 + lane < n;
+    const bool act = wbase + c * 64 + lane < n && !(DROP && key[c] == drop);
     const unsigned dg = static_cast<unsigned>(key[c] >> shift) & 0xFFu;
     dig[c] = static_cast<uint8_t>(dg);
     const uint64_t m = rs_match(dg, act);
@@ -394,7 +406,8 @@ __device__ __forceinline__ void rs_wave_ranks(const K (&key)[CH], int64_t wbase,
 }
 
 // Per digit (the block's first 256 threads): the waves' counts become their
-// exclusive prefix in wave order; dstart[d] = the tile's start of digit d.
+// exclusive prefix in wave order; dstart[d] = the tile's start of digit d,
+// dstart[256] = its keys.
 // Every thread of the block calls it, after a barrier; wsum is LDS.
 template <int WAVES>
 __device__ __forceinline__ void rs_digit_starts(uint16_t (*wcnt)[kRsBins], int32_t* dstart, int32_t* wsum) {
@@ -422,6 +435,7 @@ __device__ __forceinline__ void rs_digit_starts(uint16_t (*wcnt)[kRsBins], int32
     int32_t wpre = 0;
     for (unsigned ww = 0; ww < w; ++ww) wpre += wsum[ww];
     dstart[dgt] = wpre + incl - tot;
+    if (dgt == kRsBins - 1) dstart[kRsBins] = wpre + incl;
   }
   __syncthreads();
 }
@@ -444,13 +458,13 @@ __device__ __forceinline__ void rs_digit_base(const int64_t* __restrict__ tot, i
   }
 }
 
-template <typename K, typename V, bool HAS_V, bool SEG, int WAVES, int CH>
+template <typename K, typename V, bool HAS_V, bool SEG, bool DROP, int WAVES, int CH>
 __global__ __launch_bounds__(WAVES * 64) void k_rs_scatter(const K* __restrict__ kin, const V* __restrict__ vin,
                                                            K* __restrict__ kout, V* __restrict__ vout, int64_t n,
                                                            int shift, const int32_t* __restrict__ hist,
                                                            const int64_t* __restrict__ base,
                                                            const int64_t* __restrict__ tot, int range_shift, RsSegs sg,
-                                                           int64_t ntiles, int64_t per) {
+                                                           int64_t ntiles, int64_t per, RsDrop<K> dr) {
   constexpr int kBlock = WAVES * 64;
   constexpr int kTile = kBlock * CH;
   // Workgroups go to the eight XCDs in turn, so blocks b, b + 8, b + 16, ...
@@ -459,11 +473,15 @@ __global__ __launch_bounds__(WAVES * 64) void k_rs_scatter(const K* __restrict__
   // in memory, fill their common cache lines in one L2.
   const int64_t tile = (static_cast<int64_t>(blockIdx.x) & 7) * per + (blockIdx.x >> 3);
   if (tile >= ntiles) return;  // uniform across the block
+  if (!SEG && !DROP && dr.count) {
+    n = *dr.count;
+    if (tile * kTile >= n) return;
+  }
   static_assert(kBlock >= kRsBins, "one thread per digit");
   static_assert(kTile <= 65535, "tile counts fit 16 bits");
   __shared__ uint16_t wcnt[WAVES][kRsBins];
   __shared__ int64_t goff[kRsBins];  // global position of the tile's first key of a digit, less its tile start
-  __shared__ int32_t dstart[kRsBins];
+  __shared__ int32_t dstart[kRsBins + 1];
   __shared__ int32_t wsum[4];
   __shared__ int64_t wsum64[4];
   __shared__ int64_t s_pre[SEG ? kRsMaxSegs + 1 : 1];
@@ -476,6 +494,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_rs_scatter(const K* __restrict__
   for (int i = threadIdx.x; i < WAVES * kRsBins / 2; i += kBlock) reinterpret_cast<uint32_t*>(&wcnt[0][0])[i] = 0;
   if (SEG) rs_load_segs(sg, s_pre);
   rs_digit_base(tot, goff, wsum64);
+  if (DROP && tile == 0 && threadIdx.x == kRsBins - 1) *dr.count = goff[kRsBins - 1] + tot[kRsBins - 1];
   if (threadIdx.x < kRsBins)
     goff[threadIdx.x] += base[(tile >> range_shift) * kRsBins + threadIdx.x] + hist[tile * kRsBins + threadIdx.x];
   __syncthreads();
@@ -518,7 +537,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_rs_scatter(const K* __restrict__
       }
     }
   }
-  rs_wave_ranks<K, CH>(key, wbase, n, shift, wcnt[w], dig, rank);
+  rs_wave_ranks<K, DROP, CH>(key, wbase, n, shift, dr.drop, wcnt[w], dig, rank);
   __syncthreads();
   rs_digit_starts<WAVES>(wcnt, dstart, wsum);
   if (threadIdx.x < kRsBins) goff[threadIdx.x] -= dstart[threadIdx.x];
@@ -528,12 +547,11 @@ __global__ __launch_bounds__(WAVES * 64) void k_rs_scatter(const K* __restrict__
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
     const int64_t idx = wbase + c * 64 + lane;
-    lp[c] = idx < n ? dstart[dig[c]] + wcnt[w][dig[c]] + rank[c] : -1;
+    lp[c] = idx < n && !(DROP && key[c] == dr.drop) ? dstart[dig[c]] + wcnt[w][dig[c]] + rank[c] : -1;
     if (lp[c] >= 0) skey[lp[c]] = key[c];
   }
   __syncthreads();
-  const int64_t tbase = tile * kTile;
-  const int32_t cnt = static_cast<int32_t>(n - tbase < kTile ? n - tbase : kTile);
+  const int32_t cnt = dstart[kRsBins];
   // each thread keeps the digits of the staged positions it writes
   // (threadIdx.x + kBlock t), for the values' pass
   uint8_t dpos[CH];
@@ -573,7 +591,7 @@ __global__ __launch_bounds__(kRsOneWaves * 64) void k_rs_one(K* __restrict__ key
                                                              int bit0, int bit1) {
   constexpr int CH = kRsOneCh;
   __shared__ uint16_t wcnt[kRsOneWaves][kRsBins];
-  __shared__ int32_t dstart[kRsBins];
+  __shared__ int32_t dstart[kRsBins + 1];
   __shared__ int32_t wsum[4];
   __shared__ uint64_t s_stage[kRsOne * (sizeof(K) > sizeof(V) || !HAS_V ? sizeof(K) : sizeof(V)) / 8];
   K* skey = reinterpret_cast<K*>(s_stage);
@@ -595,7 +613,7 @@ __global__ __launch_bounds__(kRsOneWaves * 64) void k_rs_one(K* __restrict__ key
     __syncthreads();
     uint8_t dig[CH];
     int32_t rank[CH];
-    rs_wave_ranks<K, CH>(key, wbase, n, shift, wcnt[w], dig, rank);
+    rs_wave_ranks<K, false, CH>(key, wbase, n, shift, K(0), wcnt[w], dig, rank);
     __syncthreads();
     rs_digit_starts<kRsOneWaves>(wcnt, dstart, wsum);
     int32_t lp[CH];
@@ -640,14 +658,20 @@ struct RsWork {
 // One pass (digit at `shift`) from (ka, va) to (kb, vb).
 template <typename K, typename V, bool HAS_V, int WAVES, int CH>
 static int radix_pass(hdb_ctx* ctx, const K* ka, const V* va, K* kb, V* vb, int64_t n, int shift, const RsSegs& sp,
-                      const RsWork& wk) {
+                      const RsDrop<K>& dr, bool first, const RsWork& wk) {
   constexpr int kTile = WAVES * 64 * CH;
   const int64_t ntiles = (n + kTile - 1) / kTile;
   const dim3 grid(static_cast<unsigned>(ntiles)), block(WAVES * 64);
+  constexpr bool kDrops = HAS_V && sizeof(K) == 4 && sizeof(V) == 4;  // the one sort that drops keys
   if (sp.pre)
-    hipLaunchKernelGGL((k_rs_hist<K, true, WAVES, CH>), grid, block, 0, ctx->stream, ka, n, shift, wk.hist, sp);
+    hipLaunchKernelGGL((k_rs_hist<K, true, false, WAVES, CH>), grid, block, 0, ctx->stream, ka, n, shift, wk.hist, sp,
+                       dr);
+  else if (kDrops && dr.count && first)
+    hipLaunchKernelGGL((k_rs_hist<K, false, kDrops, WAVES, CH>), grid, block, 0, ctx->stream, ka, n, shift, wk.hist,
+                       sp, dr);
   else
-    hipLaunchKernelGGL((k_rs_hist<K, false, WAVES, CH>), grid, block, 0, ctx->stream, ka, n, shift, wk.hist, sp);
+    hipLaunchKernelGGL((k_rs_hist<K, false, false, WAVES, CH>), grid, block, 0, ctx->stream, ka, n, shift, wk.hist,
+                       sp, dr);
   HDB_LAUNCHED();
   int range_shift = 62;  // one range
   if (ntiles <= kRsColTiles) {
@@ -666,11 +690,14 @@ static int radix_pass(hdb_ctx* ctx, const K* ka, const V* va, K* kb, V* vb, int6
   const int64_t per = (ntiles + 7) / 8;  // tiles per XCD
   const dim3 sgrid(static_cast<unsigned>(8 * per));
   if (sp.pre)
-    hipLaunchKernelGGL((k_rs_scatter<K, V, HAS_V, true, WAVES, CH>), sgrid, block, 0, ctx->stream, ka, va, kb, vb, n,
-                       shift, wk.hist, wk.base, wk.tot, range_shift, sp, ntiles, per);
+    hipLaunchKernelGGL((k_rs_scatter<K, V, HAS_V, true, false, WAVES, CH>), sgrid, block, 0, ctx->stream, ka, va, kb,
+                       vb, n, shift, wk.hist, wk.base, wk.tot, range_shift, sp, ntiles, per, dr);
+  else if (kDrops && dr.count && first)
+    hipLaunchKernelGGL((k_rs_scatter<K, V, HAS_V, false, kDrops, WAVES, CH>), sgrid, block, 0, ctx->stream, ka, va,
+                       kb, vb, n, shift, wk.hist, wk.base, wk.tot, range_shift, sp, ntiles, per, dr);
   else
-    hipLaunchKernelGGL((k_rs_scatter<K, V, HAS_V, false, WAVES, CH>), sgrid, block, 0, ctx->stream, ka, va, kb, vb, n,
-                       shift, wk.hist, wk.base, wk.tot, range_shift, sp, ntiles, per);
+    hipLaunchKernelGGL((k_rs_scatter<K, V, HAS_V, false, false, WAVES, CH>), sgrid, block, 0, ctx->stream, ka, va, kb,
+                       vb, n, shift, wk.hist, wk.base, wk.tot, range_shift, sp, ntiles, per, dr);
   HDB_LAUNCHED();
   return HDB_OK;
 }
@@ -679,9 +706,13 @@ static int radix_pass(hdb_ctx* ctx, const K* ka, const V* va, K* kb, V* vb, int6
 // input is read through that segment map (see RsSegs).  kout == nullptr: the
 // result ends in keys/vals; otherwise *kout/*vout receive the buffers that
 // hold it (keys/vals or the sort's own scratch), which saves a copy.
+// drop != nullptr (u32 keys and values only): keys equal to *drop, which sort
+// last, are left out; *count receives a device pointer to the number of the
+// others, in the sort's scratch (valid until the next sort), or nullptr where
+// they were kept.
 template <typename K, typename V, bool HAS_V>
 static int radix_sort_t(hdb_ctx* ctx, K* keys, V* vals, int64_t n, int bit0, int bit1, const RsSegs* seg,
-                        K** kout, V** vout) {
+                        K** kout, V** vout, const K* drop = nullptr, const int64_t** count = nullptr) {
   RsSegs sg{nullptr, 0, 0};
   if (seg) {
     if (seg->nseg < 1 || seg->nseg > kRsMaxSegs) return ctx->fail(HDB_EINVAL, "bad segment map");
@@ -691,6 +722,7 @@ static int radix_sort_t(hdb_ctx* ctx, K* keys, V* vals, int64_t n, int bit0, int
   if (n <= 1 && !seg) bit1 = bit0;
   if (kout) *kout = keys;
   if (vout) *vout = vals;
+  if (count) *count = nullptr;
   if (n <= 0 || bit1 <= bit0) return HDB_OK;
   if (!seg && n <= kRsOne) {
     hipLaunchKernelGGL((k_rs_one<K, V, HAS_V>), dim3(1), dim3(kRsOneWaves * 64), 0, ctx->stream, keys, vals,
@@ -717,9 +749,12 @@ static int radix_sort_t(hdb_ctx* ctx, K* keys, V* vals, int64_t n, int bit0, int
   if (HAS_V) HDB_CALL(scratch_t(ctx, kSlotSortVals, static_cast<size_t>(n), &v2));
   HDB_CALL(scratch_t(ctx, kSlotSortHist, static_cast<size_t>(kRsBins * ntiles), &wk.hist));
   const int64_t nrange = (ntiles + kRsColRows - 1) / kRsColRows;
-  HDB_CALL(scratch_t(ctx, kSlotSortAux, static_cast<size_t>(kRsBins * (1 + nrange + (nrange + 1) / 2)), &wk.tot));
+  HDB_CALL(scratch_t(ctx, kSlotSortAux, static_cast<size_t>(kRsBins * (1 + nrange + (nrange + 1) / 2) + 1), &wk.tot));
   wk.base = wk.tot + kRsBins;
   wk.q = reinterpret_cast<int32_t*>(wk.base + kRsBins * nrange);
+  // the count of a sort that drops keys follows the range totals
+  const RsDrop<K> dr{drop ? wk.tot + kRsBins * (1 + nrange + (nrange + 1) / 2) : nullptr, drop ? *drop : K(0)};
+  if (count) *count = dr.count;
   K* ka = keys;
   K* kb = k2;
   V* va = vals;
@@ -728,9 +763,9 @@ static int radix_sort_t(hdb_ctx* ctx, K* keys, V* vals, int64_t n, int bit0, int
   for (int shift = bit0; shift < bit1; shift += 8, ++passes) {
     const RsSegs sp = passes == 0 ? sg : RsSegs{nullptr, 0, 0};
     if (small)
-      HDB_CALL((radix_pass<K, V, HAS_V, 8, 4>(ctx, ka, va, kb, vb, n, shift, sp, wk)));
+      HDB_CALL((radix_pass<K, V, HAS_V, 8, 4>(ctx, ka, va, kb, vb, n, shift, sp, dr, passes == 0, wk)));
     else
-      HDB_CALL((radix_pass<K, V, HAS_V, 8, kCh>(ctx, ka, va, kb, vb, n, shift, sp, wk)));
+      HDB_CALL((radix_pass<K, V, HAS_V, 8, kCh>(ctx, ka, va, kb, vb, n, shift, sp, dr, passes == 0, wk)));
     std::swap(ka, kb);
     std::swap(va, vb);
   }
@@ -768,6 +803,10 @@ int radix_sort_u32_u32_out(hdb_ctx* ctx, uint32_t* keys, uint32_t* vals, int64_t
                            uint32_t** kout, uint32_t** vout) {
   return radix_sort_t<uint32_t, uint32_t, true>(ctx, keys, vals, n, bit0, bit1, nullptr, kout, vout);
 }
+int radix_sort_u32_u32_drop(hdb_ctx* ctx, uint32_t* keys, uint32_t* vals, int64_t n, int bit0, int bit1, uint32_t drop,
+                            uint32_t** kout, uint32_t** vout, const int64_t** count) {
+  return radix_sort_t<uint32_t, uint32_t, true>(ctx, keys, vals, n, bit0, bit1, nullptr, kout, vout, &drop, count);
+}
 
 }  // namespace hdb
 
@@ -776,7 +815,8 @@ namespace hdb {
 // -------------------------------------------------------- segment bounds --
 template <typename P>
 __global__ void k_seg_bounds(const uint32_t* __restrict__ keys, int64_t m, int64_t nseg, int shift,
-                             P* __restrict__ s, P* __restrict__ e) {
+                             P* __restrict__ s, P* __restrict__ e, const int64_t* __restrict__ count) {
+  if (count) m = *count;
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= m) return;
   const uint32_t k = keys[i] >> shift;
@@ -790,7 +830,8 @@ __global__ void k_seg_bounds(const uint32_t* __restrict__ keys, int64_t m, int64
 // just outside their four.  keys must be 16-byte aligned.
 template <typename P>
 __global__ void k_seg_bounds4(const uint32_t* __restrict__ keys, int64_t m, int64_t nseg, int shift,
-                              P* __restrict__ s, P* __restrict__ e) {
+                              P* __restrict__ s, P* __restrict__ e, const int64_t* __restrict__ count) {
+  if (count) m = *count;
   const int64_t i0 = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
   const unsigned lane = __lane_id();
   uint32_t k[4];
@@ -819,7 +860,8 @@ __global__ void k_seg_bounds4(const uint32_t* __restrict__ keys, int64_t m, int6
 }
 
 template <typename P>
-static int segment_bounds_t(hdb_ctx* ctx, const uint32_t* keys, int64_t m, int64_t nseg, P* s, P* e, int shift) {
+static int segment_bounds_t(hdb_ctx* ctx, const uint32_t* keys, int64_t m, int64_t nseg, P* s, P* e, int shift,
+                            const int64_t* count) {
   if (sizeof(P) == 4 && m > INT32_MAX) return ctx->fail(HDB_EUNSUPPORTED, "int32 segment bounds past 2^31 keys");
   if (sizeof(P) == 8) {
     HDB_CALL(fill_u64(ctx, reinterpret_cast<uint64_t*>(s), nseg, 0));
@@ -831,19 +873,20 @@ static int segment_bounds_t(hdb_ctx* ctx, const uint32_t* keys, int64_t m, int64
   if (m <= 0) return HDB_OK;
   if ((reinterpret_cast<uintptr_t>(keys) & 15) == 0)
     hipLaunchKernelGGL(k_seg_bounds4<P>, dim3(grid_for((m + 3) / 4, 256)), dim3(256), 0, ctx->stream, keys, m, nseg,
-                       shift, s, e);
+                       shift, s, e, count);
   else
     hipLaunchKernelGGL(k_seg_bounds<P>, dim3(grid_for(m, 256)), dim3(256), 0, ctx->stream, keys, m, nseg, shift, s,
-                       e);
+                       e, count);
   HDB_LAUNCHED();
   return HDB_OK;
 }
 
-int segment_bounds(hdb_ctx* ctx, const uint32_t* keys, int64_t m, int64_t nseg, int32_t* s, int32_t* e, int shift) {
-  return segment_bounds_t(ctx, keys, m, nseg, s, e, shift);
+int segment_bounds(hdb_ctx* ctx, const uint32_t* keys, int64_t m, int64_t nseg, int32_t* s, int32_t* e, int shift,
+                   const int64_t* count) {
+  return segment_bounds_t(ctx, keys, m, nseg, s, e, shift, count);
 }
 int segment_bounds(hdb_ctx* ctx, const uint32_t* keys, int64_t m, int64_t nseg, int64_t* s, int64_t* e, int shift) {
-  return segment_bounds_t(ctx, keys, m, nseg, s, e, shift);
+  return segment_bounds_t(ctx, keys, m, nseg, s, e, shift, nullptr);
 }
 
 int bits_for(int64_t max_key) {

@@ -363,3 +363,21 @@ def test_join_matrix_values_equal_general(ctx, d, S):
         assert ctx.nnd_stats()["bucket_drops"] == 0
         np.testing.assert_array_equal(a["label"], b["label"])
         np.testing.assert_array_equal(a["distance"].view(np.uint32), b["distance"].view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [256, 257, 12500, 12501, 40000])
+@pytest.mark.parametrize("S", [3, 16])
+def test_reverse_sort_without_unused_slots(ctx, n, S):
+    """The reverse sort leaves out the slots no sample uses: at the one-block
+    sort's largest point count and past it, at both sides of the change of
+    tile size (n x 32 slots), and with few of the slots in use (S = 3).  The
+    lists are distinct, sorted and hold the oracle's distances; with S = 16
+    they reach the recall of the other sizes."""
+    print(f"case: reverse sort n={n} S={S}", flush=True)
+    X = datasets.tiny_blobs(n, 12, 8, seed=n + S)
+    p = api.default_params(sample_num=S, bucket_cap=1024)
+    L = api.NNDescent(ctx, X, iteration=6, params=p)
+    _check_lists(X, L)
+    assert ctx.nnd_stats()["bucket_drops"] == 0
+    if S == 16:
+        assert _recall(X, L) >= 0.95
