@@ -533,14 +533,14 @@ __device__ __forceinline__ void join_quads(F f) {
 // distances are then recomputed from the same rows in the same operation
 // order as the other joins, so proposals carry exactly its distances; only the
 // choice among partners whose distances agree to about 1e-4 relative can
-// differ.  Bound by VALU issue.  The ranking values come from the matrix
-// cores, four partners of all 64 candidates in D + 2 products (join_quad),
-// where the vector unit took D multiply-adds per partner and each wave read
-// the partners' rows from LDS again.
-// At 500k x 32 and KEEP = 3 a launch takes 1.17 ms instead of 1.63 (the block
-// and the rows in one buffer: five blocks on a CU, not four); at 1M x 12, where
-// the other work of a wave (sort of the candidates, ranking, emission) is
-// most of it, 1.44 ms as before.
+// differ.  The ranking values come from the matrix cores, four partners of
+// all 64 candidates in D + 2 products (join_quad), where the vector unit took
+// D multiply-adds per partner and each wave read the partners' rows from LDS
+// again.  At D = 32 the kernel is bound by instruction issue: at 500k points
+// and KEEP = 3 a launch takes 1.17 ms instead of 1.63 (the block and the rows
+// in one buffer: five blocks on a CU, not four).  At D = 12 it is bound by the
+// gathers of the candidates' rows: 41M L2 misses a launch of 1M points, and
+// 1.44 ms with 738 vector instructions per wave as with 1034.
 template <int D, bool NEWNEW, int KEEP>
 __global__ __launch_bounds__(kJoinWaves * 64, D <= 16 ? 8 : 5) void k_nnd_join2(const float* __restrict__ X, int64_t n, int d, int S,
                                                                NndBufs b) {
