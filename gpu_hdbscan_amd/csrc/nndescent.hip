@@ -2025,28 +2025,26 @@ int nnd_blocked(hdb_ctx* ctx, const float* X, int64_t n, int d, int blocks, cons
 // ------------------------------------------------------ brute-force kNN --
 // One wave per query and point chunk (blockIdx.y); each lane scans a strided
 // share of the chunk keeping a sorted top-kq (kq <= 32) in registers, then
-// the wave pops the chunk's top-kq from the 64 lane lists into
+// the wave pops the chunk's top-kq from the 64 lane lists.  With one chunk
+// (part == nullptr) that is the result; otherwise it goes to
 // part[(qi * chunks + y) * 32 + s] (kKeyMax past the last), which k_bf_merge
 // merges.  Bound by the row reads (a lane per row, 16 bytes at a time where
 // rows are 16-byte aligned): the chunks let a few queries fill the chip.  16
 // queries against 100k x 128 took 25.4 ms with one wave each, 0.4 ms split.
 __global__ __launch_bounds__(256) void k_bruteforce(const float* __restrict__ X, int64_t n, int d,
                                                     const int32_t* __restrict__ qids, int64_t m, int kq,
-                                                    int64_t csize, uint64_t* __restrict__ part) {
+                                                    int64_t csize, uint64_t* __restrict__ part,
+                                                    int32_t* __restrict__ out_ids, float* __restrict__ out_d2) {
   const unsigned lane = __lane_id();
   const int64_t qi = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (qi >= m) return;
-  uint64_t* out = part + (qi * gridDim.y + blockIdx.y) * 32;
   const uint32_t q = static_cast<uint32_t>(qids[qi]);
-  if (static_cast<int64_t>(q) >= n) {  // an id outside [0, n): no neighbours
-    if (lane < 32) out[lane] = kKeyMax;
-    return;
-  }
+  const bool known = static_cast<int64_t>(q) < n;  // an id outside [0, n): no neighbours
   uint64_t top[32];
 #pragma unroll
   for (int i = 0; i < 32; ++i) top[i] = kKeyMax;
   const int64_t c0 = static_cast<int64_t>(blockIdx.y) * csize;
-  const int64_t c1 = c0 + csize < n ? c0 + csize : n;
+  const int64_t c1 = !known ? c0 : c0 + csize < n ? c0 + csize : n;
   for (int64_t i = c0 + lane; i < c1; i += 64) {
     if (static_cast<uint32_t>(i) == q) continue;
     uint64_t key = (static_cast<uint64_t>(__float_as_uint(point_d2(X, d, q, static_cast<uint32_t>(i)))) << 32) |
@@ -2078,7 +2076,13 @@ __global__ __launch_bounds__(256) void k_bruteforce(const float* __restrict__ X,
     if (h == mn && mn != kKeyMax) head++;
     if (static_cast<int>(lane) == r) mine = mn;
   }
-  if (lane < 32) out[lane] = mine;
+  if (part) {
+    if (lane < 32) part[(qi * gridDim.y + blockIdx.y) * 32 + lane] = mine;
+  } else if (static_cast<int>(lane) < kq) {
+    out_ids[qi * kq + lane] = mine == kKeyMax ? -1 : static_cast<int32_t>(static_cast<uint32_t>(mine));
+    if (out_d2)
+      out_d2[qi * kq + lane] = __uint_as_float(known ? static_cast<uint32_t>(mine >> 32) : 0x7F800000u);
+  }
 }
 
 // Tiled brute force for D = 12 or 32: block (g, y) holds queries
@@ -2275,15 +2279,23 @@ int bruteforce_knn(hdb_ctx* ctx, const float* X, int64_t n, int d, const int32_t
   Stage st(ctx, "bruteforce_knn");
   if (d == 12) return bruteforce_tiled<12>(ctx, X, n, qids, m, kq, out_ids, out_d2);
   if (d == 32) return bruteforce_tiled<32>(ctx, X, n, qids, m, kq, out_ids, out_d2);
-  // about 8192 waves, chunks of at least 512 points
-  int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(8192 / m, (n + 511) / 512));
+  // About 8192 waves, chunks of at least 512 points; one chunk, which needs no
+  // scratch and no merge, where a wave's whole scan (in loads, and six loads'
+  // time for the rest of a point) costs less than popping and merging the
+  // chunks' lists.  One chunk / split: 100 queries of 3000 x 7 134 / 151 us, of
+  // 3000 x 33 219 / 162; 1000 of 3000 x 33 225 / 255, of 10k x 7 356 / 273; 4096
+  // of 10k x 20 468 / 657, of 10k x 128 3388 / 3067.
+  const bool vec4 = (d & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
+  const bool split = n * (6 + (vec4 ? d / 4 : d)) >= 60000 + 60 * m;
+  int64_t chunks = split ? std::max<int64_t>(1, std::min<int64_t>(8192 / m, (n + 511) / 512)) : 1;
   const int64_t csize = (n + chunks - 1) / chunks;
   chunks = (n + csize - 1) / csize;
-  uint64_t* part;
-  HDB_CALL(scratch_t(ctx, kSlotBfTmp, m * chunks * 32, &part));
+  uint64_t* part = nullptr;
+  if (chunks > 1) HDB_CALL(scratch_t(ctx, kSlotBfTmp, m * chunks * 32, &part));
   hipLaunchKernelGGL(k_bruteforce, dim3(grid_for(m, 4), static_cast<unsigned>(chunks)), dim3(256), 0, ctx->stream, X, n,
-                     d, qids, m, kq, csize, part);
+                     d, qids, m, kq, csize, part, out_ids, out_d2);
   HDB_LAUNCHED();
+  if (!part) return HDB_OK;
   hipLaunchKernelGGL(k_bf_merge, dim3(grid_for(m, 4)), dim3(256), 0, ctx->stream, part, m, static_cast<int>(chunks), kq,
                      qids, n, out_ids, out_d2);
   HDB_LAUNCHED();

@@ -6,6 +6,8 @@ restatement of InitKNNGraphIndexKernel; NN-Descent lists sorted, self-free,
 duplicate-free, every stored distance bit-equal to the oracle's FP32 formula
 on the returned neighbour; recall@32 >= 0.95 against FP64 brute force.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -128,6 +130,31 @@ def test_bruteforce_point_chunks(ctx, m, d):
     np.testing.assert_array_equal(d2, wd)
     few, _ = api.bruteforce_knn(ctx, X, q, 5)
     np.testing.assert_array_equal(few, want[:, :5])
+
+
+@pytest.mark.parametrize("n,d", [(600, 7), (64, 128), (5000, 33)])
+def test_bruteforce_many_queries_keep_no_scratch(n, d):
+    """More queries than waves fill the chip: the lists are written by the
+    scan itself, and the context keeps no memory that grows with the queries
+    (it once kept 256 bytes for each: 51 MB here)."""
+    def free(c):  # through the library's own HIP runtime
+        a, b = C.c_size_t(), C.c_size_t()
+        assert c.lib.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    print(f"case: bruteforce 200000 queries of {n}x{d}", flush=True)
+    X = datasets.tiny_blobs(n, d, 5, seed=d)
+    q = (np.arange(200_000) % (n + 2) - 1).astype(np.int32)
+    with api.Context(0) as c:
+        api.bruteforce_knn(c, X, q[:1], 32)
+        before = free(c)
+        ids, d2 = api.bruteforce_knn(c, X, q, 32)
+        assert before - free(c) < 16 << 20
+    rows = np.r_[1:40, 1 + n // 2, n]
+    want, wd = O.bruteforce_fp32(X, q[rows], 32)
+    np.testing.assert_array_equal(ids[rows], want)
+    np.testing.assert_array_equal(d2[rows], wd)
+    assert np.all(ids[[0, n + 1]] == -1) and np.all(np.isinf(d2[[0, n + 1]]))
 
 
 def test_recall_on_device_matches_oracle(ctx):
