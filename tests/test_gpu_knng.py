@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 from gpu_hdbscan_amd import api, datasets
+from oracle import nnd_oracle as N
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -408,3 +409,55 @@ def test_reverse_sort_without_unused_slots(ctx, n, S):
     assert ctx.nnd_stats()["bucket_drops"] == 0
     if S == 16:
         assert _recall(X, L) >= 0.95
+
+
+def _whole_points(n, d, seed, kind):
+    """Points with whole coordinates, so that every distance, and every value
+    the joins rank by, is exact in FP32 (distances below 2^18 for d = 12 and 32,
+    whose keys drop six bits; below 2^24 otherwise), and their float32 squared
+    distances.  kind: fine, coarse (many equal distances and repeated points),
+    or nonfinite (some NaN and infinite coordinates)."""
+    r = int(np.sqrt((1 << (18 if d in (12, 32) else 24)) / d) / 2) - 1
+    X = np.clip(datasets.tiny_blobs(n, d, 6, seed=seed, spread=4.0) / 9, -1, 1)
+    X = np.round(X * (4 if kind == "coarse" else r)).astype(np.float32)
+    if kind == "coarse":
+        X[: n // 8] = X[n // 2: n // 2 + n // 8]
+    if kind == "nonfinite":
+        X[7::101, 0], X[31::101, d - 1], X[57::101, d // 2] = np.nan, np.inf, -np.inf
+    with np.errstate(invalid="ignore"):
+        D = np.stack([((X - x).astype(np.float64) ** 2).sum(1) for x in X]).astype(np.float32)
+    D.view(np.uint32)[np.isnan(D)] = 0x7FC00000
+    return X, D
+
+
+def _equal_lists(L, lists):
+    ids, bits = N.arrays(lists)
+    np.testing.assert_array_equal(np.where(L["label"] == 0x7FFFFFFF, -1, L["label"]), ids)
+    np.testing.assert_array_equal(L["distance"], bits.view(np.float32))  # a NaN's sign is the hardware's
+
+
+# d = 12 and 32 rank by |a|^2 - 2 a.b + |b|^2: no exact order among infinite values
+@pytest.mark.parametrize("d,kind", [(d, kind) for d in (2, 8, 11, 12, 13, 20, 24, 31, 32, 40)
+                                    for kind in ("fine", "coarse", "nonfinite")
+                                    if kind != "nonfinite" or d not in (12, 32)])
+def test_nndescent_equals_oracle(ctx, d, kind):
+    """Every list of three iterations, ids and distances, against the numpy
+    NN-Descent, for every pairing and a merge: each join kernel chooses the
+    nearest partners (equal distances: the smaller id; at d = 12 and 32 the
+    earlier candidate).  Pairs at no finite distance are never proposed."""
+    print(f"case: NN-Descent of 330x{d}, {kind} points, against the oracle", flush=True)
+    n = 330
+    X, D = _whole_points(n, d, 11 * d, kind)
+    B = D.view(np.uint32)
+    slot = d in (12, 32)
+    for keep, S in ((0, 16), (1, 16), (3, 7), (8, 16)):
+        p = api.default_params(join_keep=keep, sample_num=S, bucket_cap=1024)
+        L = api.NNDescent(ctx, X, iteration=3, params=p)
+        assert ctx.nnd_stats()["bucket_drops"] == 0
+        _equal_lists(L, N.descend(D, N.init_random(B), S, keep, 3, by_slot=slot))
+    n1 = 180
+    for keep in (0, 4):
+        p = api.default_params(join_keep=keep, merge_sample_num=9, merge_iteration=2, bucket_cap=1024)
+        g1, g2 = api.NNDescent(ctx, X[:n1], iteration=2, params=p), api.NNDescent(ctx, X[n1:], iteration=2, params=p)
+        L = api.KNNMergeFromHost(ctx, X[:n1], g1, X[n1:], g2, params=p)
+        _equal_lists(L, N.descend(D, N.init_merge(B, g1["label"], g2["label"]), 9, keep, 2, split=n1, by_slot=slot))

@@ -47,6 +47,26 @@ def test_refine_exact_from_nndescent_lists(ctx, d):
     assert cand >= 32 * (len(X) - ovf)
 
 
+@pytest.mark.parametrize("d", [20, 50, 128])
+def test_refine_with_nonfinite_points(ctx, d):
+    """Points with NaN or infinite coordinates are at no finite distance from
+    any other: they survive no test, and the lists of the other points are the
+    exact ones, from bounds that hold no finite distance too."""
+    print(f"case: refine 3000x{d} with NaN and infinite coordinates", flush=True)
+    X = _mixture(3000, d, 13)
+    X[7::97, 0], X[31::97, d - 1], X[57::97, d // 2] = np.nan, np.inf, -np.inf
+    L = api.NNDescent(ctx, X, iteration=2)
+    Ld = ctx.to_device(L)
+    api.refine_knng(ctx, ctx.to_device(X), Ld)
+    finite = np.flatnonzero(np.isfinite(X).all(1)).astype(np.int32)
+    assert not np.isfinite(L["distance"][finite, 31]).all()
+    at = np.arange(0, len(finite), 7, dtype=np.int32)  # the oracle ranks the finite points alone
+    ids, dd = O.bruteforce_fp32(X[finite], at, 32)
+    got = Ld.numpy()[finite[at]]
+    np.testing.assert_array_equal(got["label"], finite[ids])
+    np.testing.assert_array_equal(got["distance"], dd)
+
+
 def test_refine_overflow_falls_back_to_bruteforce(ctx):
     """Random initial lists bound nothing useful: (almost) every point has
     more than 128 survivors and is answered by the exact brute force; the

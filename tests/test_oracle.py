@@ -353,3 +353,25 @@ def test_unique_merge_is_sorted_set_union():
         want = sorted(a | b)[:K]
         assert [(float(d), int(g)) for d, g in zip(got[r]["distance"], got[r]["label"])][: len(want)] == want
         assert all(g == 0x7FFFFFFF for g in got[r]["label"][len(want):])
+
+
+def test_nnd_oracle_converges_to_exact_lists():
+    """The NN-Descent oracle: its start is or_init_random's, no list gets worse,
+    and with every partner kept it reaches the exact lists of 300 points."""
+    from oracle import nnd_oracle as N
+    rng = np.random.default_rng(3)
+    X = rng.integers(-40, 40, (300, 6)).astype(np.float32)
+    D = ((X[:, None].astype(np.int64) - X[None].astype(np.int64)) ** 2).sum(2).astype(np.float32)
+    L = N.init_random(np.ascontiguousarray(D).view(np.uint32))
+    ids, bits = N.arrays(L)
+    ref = O.init_random(X)
+    np.testing.assert_array_equal(ids, ref["label"])
+    np.testing.assert_array_equal(bits, ref["distance"].view(np.uint32))
+    for it in range(8):
+        L = N.descend(D, L, 16, 63, 1)
+        ids, now = N.arrays(L)
+        if it > 0:  # the first update drops the start's repeated ids
+            assert np.all(now <= bits)
+        bits = now
+    gt, _ = O.bruteforce_fp32(X, np.arange(300, dtype=np.int32), 32)
+    np.testing.assert_array_equal(ids, gt)
