@@ -94,6 +94,52 @@ def test_labels_gpu_long_clusters(ctx, per, weights):
         np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("m", [524_287, 524_288, 524_365, 4_194_381])
+@pytest.mark.parametrize("shape", ["path", "star", "random"])
+def test_labels_gpu_several_edges_per_thread(ctx, m, shape):
+    """From 524,288 edges on a block of the linkage's upper levels takes several
+    edges a thread (16 from 4,194,304), the last block a ragged share, and its
+    tables and the union-find meet whole trees' worth of contention."""
+    print(f"case: hdb_labels_gpu {shape} tree of {m} edges", flush=True)
+    rng = np.random.default_rng(m)
+    n = m + 1
+    ids = rng.permutation(n).astype(np.int32)
+    e = np.empty(m, api.MST_EDGE)
+    e["from_node"] = {"path": ids[:-1], "star": ids[0], "random": ids[(rng.random(m) * np.arange(1, n)).astype(np.int64)]}[shape]
+    e["to_node"] = ids[1:]
+    e = e[rng.permutation(m)]
+    e["weight"] = np.sort(rng.gamma(2.0, 1.0, m).astype(np.float32).round(3))
+    for mpts in (3, 32):
+        want, wnc = api.get_clusters(e, n, mpts)
+        got, gnc = api.get_clusters_gpu(ctx, e, n, mpts)
+        assert gnc == wnc
+        np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("weights", ["inf", "nan", "subnormal", "negative"])
+@pytest.mark.parametrize("n", [50, 3000, 30_011])
+def test_labels_gpu_unusual_weights(ctx, n, weights):
+    """Infinite, NaN, subnormal and negative weights give the host's labels
+    (lambda 0 or infinity's stand-in, stabilities that are not finite)."""
+    print(f"case: hdb_labels_gpu {n} points, {weights} weights", flush=True)
+    rng = np.random.default_rng(n)
+    e = _random_tree(rng, n, 0)
+    w = e["weight"]
+    some = rng.random(n - 1) < 0.1
+    if weights == "subnormal":
+        w *= np.float32(1e-42)
+    elif weights == "negative":
+        w[some] *= -1
+    else:
+        w[some] = np.inf if weights == "inf" else np.nan
+    e = e[np.argsort(w, kind="stable")]
+    for mpts in (2, 7, 32, 1000):
+        want, wnc = api.get_clusters(e, n, mpts)
+        got, gnc = api.get_clusters_gpu(ctx, e, n, mpts)
+        assert gnc == wnc
+        np.testing.assert_array_equal(got, want)
+
+
 def test_labels_gpu_quirk_cases(ctx):
     from test_labels import HAND_CASES, _edges
     for name, rows, n, want, want_nc in HAND_CASES:
