@@ -531,9 +531,14 @@ __device__ __forceinline__ void join_quads(F f) {
 // keys -- the bits of that value without the sign, with the low 6 bits
 // replaced by the partner's index -- and the KEEP winners' exact squared
 // distances are then recomputed from the same rows in the same operation
-// order as the other joins, so proposals carry exactly its distances; only the
-// choice among partners whose distances agree to about 1e-4 relative can
-// differ.  The ranking values come from the matrix cores, four partners of
+// order as the other joins, so proposals carry exactly its distances.  A
+// ranking value carries the roundings of the norms and of D products, about
+// 2^-22 (|a|^2 + |b|^2) and at most (D + 2) 2^-24 of it, and the key a relative
+// 2^-18: partners whose distances differ by less may be chosen in either
+// order.  Data far from the origin for its neighbour distances leaves nothing
+// but that error (unit clusters 3000 off it: recall 0.33 at 300k x 12), so a
+// wave whose last winners show it (below) ranks every partner by its
+// distance.  The ranking values come from the matrix cores, four partners of
 // all 64 candidates in D + 2 products (join_quad), where the vector unit took
 // D multiply-adds per partner and each wave read the partners' rows from LDS
 // again.  At D = 32 the kernel is bound by instruction issue: at 500k points
@@ -750,6 +755,35 @@ __global__ __launch_bounds__(kJoinWaves * 64, D <= 16 ? 8 : 5) void k_nnd_join2(
   for (int s = 0; s < kSlots; ++s) {
     top64[s] = kKeyMax;
     if (active && fin[s] != kNone) top64[s] = make_key(dist[s], s_cand[w][fin[s] & 63u], 1u);
+  }
+  // Far from the origin the ranking values are rounding errors: where the
+  // last winner's is off by a sixteenth of its distance for most candidates,
+  // the wave ranks every partner by its distance.  (Unit clusters at 300k x 12,
+  // join_keep 4: 300 off the origin no wave does, recall 0.987 in 9.4 ms; 1000 off
+  // 0.960 -> 0.987 for 12.2 ms, 3000 off 0.334 -> 0.988 for 12.7 ms.)
+  constexpr int kLast = KEEP == 0 ? 0 : kSlots - 1;
+  const float last = dist[kLast];
+  const bool has = active && fin[kLast] != kNone && last > 0.0f && last < __uint_as_float(0x7F800000u);
+  const bool off = !(16.0f * __builtin_fabsf(__uint_as_float(fin[kLast] & ~63u) - last) <= last);
+  if (2 * __popcll(__ballot(has && off)) > __popcll(__ballot(has))) {  // uniform
+    const int me = static_cast<int>(lane), jb = is_new && !NEWNEW ? nn : 0, je = is_new ? nc : nn;
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) top64[s] = kKeyMax;
+#pragma unroll 1
+    for (int j = 0; j < nc; ++j) {
+      const uint32_t id = __builtin_amdgcn_readfirstlane(s_cand[w][j]);
+      const float* row = kPadded ? b.rows + static_cast<int64_t>(id) * 16 : X + static_cast<int64_t>(id) * D;
+      float acc = 0.0f;
+#pragma unroll
+      for (int k = 0; k < D; ++k) {
+        const float diff = own[k] - row[k];
+        acc = __builtin_fmaf(diff, diff, acc);
+      }
+      const uint64_t key = active && j >= jb && j < je && j != me ? make_key(acc, id, 1u) : kKeyMax;
+      if (KEEP != 0) top_insert<kSlots>(top64, key);
+      else if (j < nn) top64[0] = key < top64[0] ? key : top64[0];
+      else top64[1] = key < top64[1] ? key : top64[1];
+    }
   }
   join_emit<WPB, kSlots>(b, top64, active, my_id, lim, nc, rev_drop);
 }

@@ -411,6 +411,28 @@ def test_reverse_sort_without_unused_slots(ctx, n, S):
         assert _recall(X, L) >= 0.95
 
 
+@pytest.mark.parametrize("d", [12, 32])
+@pytest.mark.parametrize("shift", [300, 1000, 3000, 30000])
+def test_join_far_from_the_origin(ctx, d, shift):
+    """A shift of every point changes neighbours by the points' own rounding
+    only: the joins that rank by |a|^2 - 2 a.b + |b|^2 reach the recall of the
+    kernels that rank by distances (the same points with a zero column), for
+    every pairing and a merge."""
+    print(f"case: join at d={d}, points {shift} from the origin", flush=True)
+    n = 20000
+    X = (datasets.tiny_blobs(n, d, 12, seed=d) + np.float32(shift)).astype(np.float32)
+    P = np.zeros((n, d + 1), np.float32)
+    P[:, :d] = X
+    for keep in (0, 1, 2, 3, 4, 8):
+        p = api.default_params(join_keep=keep)
+        a, b = (_recall(X, api.NNDescent(ctx, Y, iteration=8, params=p)) for Y in (X, P))
+        assert a > b - 0.01, (keep, a, b)
+    for keep in (0, 4):
+        p = api.default_params(join_keep=keep)
+        a, b = (_recall(X, api.GenLargeKNNGraph(ctx, Y, 2, params=p)) for Y in (X, P))
+        assert a > b - 0.01, (keep, a, b)
+
+
 def _whole_points(n, d, seed, kind):
     """Points with whole coordinates, so that every distance, and every value
     the joins rank by, is exact in FP32 (distances below 2^18 for d = 12 and 32,
