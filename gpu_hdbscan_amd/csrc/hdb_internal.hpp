@@ -18,7 +18,6 @@ namespace hdb {
 constexpr int kK = 32;                       // NEIGHB_NUM_PER_LIST
 constexpr uint32_t kInvalidId = 0x7FFFFFFFu;  // empty list slot label
 constexpr uint64_t kKeyMax = ~0ull;
-constexpr int kWave = 64;
 // No-allocation entry point (hdb_sort_edges_noalloc): its scratch array
 // size, the edge count it takes at most, and the devices it serves.
 constexpr size_t kNoAllocBytes = static_cast<size_t>(28) << 20;
@@ -419,39 +418,14 @@ __device__ __forceinline__ void bitonic128(uint64_t& r0, uint64_t& r1) {
   }
 }
 
-// bitonic128 for u32 keys.
-__device__ __forceinline__ void bitonic128_u32(uint32_t& r0, uint32_t& r1) {
-  const unsigned lane = __lane_id();
-#pragma unroll
-  for (int k = 2; k <= 128; k <<= 1) {
-#pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      if (j == 64) {
-        const uint32_t mn = r0 < r1 ? r0 : r1, mx = r0 < r1 ? r1 : r0;
-        r0 = mn;
-        r1 = mx;
-      } else {
-        const uint32_t o0 = lane_xor_u32(r0, j), o1 = lane_xor_u32(r1, j);
-        const bool low = (lane & j) == 0;
-        const bool up0 = (k == 128) ? true : ((lane & k) == 0);
-        const bool up1 = (k == 128) ? true : (((64u + lane) & k) == 0);
-        r0 = bitonic_ce(r0, o0, low == up0);
-        r1 = bitonic_ce(r1, o1, low == up1);
-      }
-    }
-  }
-}
-
 // ---- kernel families (launch wrappers) -----------------------------------
 // prims.hip
 int fill_i32(hdb_ctx* ctx, int32_t* p, int64_t n, int32_t v);
 int fill_u64(hdb_ctx* ctx, uint64_t* p, int64_t n, uint64_t v);
-int fill_u8(hdb_ctx* ctx, uint8_t* p, int64_t n, uint8_t v);
 // Exclusive scan of n int32 counts into n+1 int64 offsets (out[n] = total).
 int scan_i32_to_i64(hdb_ctx* ctx, const int32_t* in, int64_t n, int64_t* out);
 // Stable LSD radix sort.  Keys u32 (bits [bit0, bit1)) with u64 payload.
 int radix_sort_u32_u64(hdb_ctx* ctx, uint32_t* keys, uint64_t* vals, int64_t n, int bit0, int bit1);
-int radix_sort_u32_u32(hdb_ctx* ctx, uint32_t* keys, uint32_t* vals, int64_t n, int bit0, int bit1);
 // seg_start/seg_end[k] = [first, last+1) position of segment k = key >> shift
 // in keys sorted by that value (k < nseg); untouched segments keep 0.
 // count: a device pointer to the number of keys where the host does not know

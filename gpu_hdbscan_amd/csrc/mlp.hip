@@ -27,7 +27,6 @@ namespace hdb {
 constexpr int kHid = 128;
 constexpr int kCode = 12;
 constexpr int kOutP = 16;  // padded output width
-constexpr int kMlpWaves = 2;  // waves per forward block (LDS: 16 rows x (d_in + 2 x 128) floats each)
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));

@@ -534,7 +534,7 @@ __device__ __forceinline__ void join_quads(F f) {
 // order as the other joins, so proposals carry exactly its distances.  A
 // ranking value carries the roundings of the norms and of D products, about
 // 2^-22 (|a|^2 + |b|^2) and at most (D + 2) 2^-24 of it, and the key a relative
-// 2^-18: partners whose distances differ by less may be chosen in either
+// 2^-17: partners whose distances differ by less may be chosen in either
 // order.  Data far from the origin for its neighbour distances leaves nothing
 // but that error (unit clusters 3000 off it: recall 0.33 at 300k x 12), so a
 // wave whose last winners show it (below) ranks every partner by its
@@ -554,10 +554,13 @@ __global__ __launch_bounds__(kJoinWaves * 64, D <= 16 ? 8 : 5) void k_nnd_join2(
   constexpr int kStride = (D + 3) & ~3;
   constexpr int kSlots = KEEP == 0 ? 2 : KEEP;
   // Old x new block, rows of kBst values (odd, so the old lanes' stores and
-  // the new lanes' column reads spread over the banks).  An old-new value
-  // with the norms added in the new candidate's order comes from the block;
-  // where no * (nn + 1) passes kBlock (rarely), phase 2 takes the values with
-  // the old candidate's norm first, from the products.
+  // the new lanes' column reads spread over the banks); it holds every old-new
+  // pair.  Its values add the old candidate's norm last; where no * (nn + 1)
+  // passes kBlock, phase 2 forms them again with the new candidate's norm last.
+  // kBlock is no capacity: it decides the order of additions, and with it the
+  // choice between partners that the ranking cannot tell apart.  Taking every
+  // value from the block changes 73 of 1M lists (d = 12, join_keep 3, six
+  // iterations; the joins 8.54 -> 8.10 ms), so the limit stays.
   constexpr int kBlock = 384;
   constexpr int kBst = 33;
   // The block's space takes the candidates' rows afterwards, kCols columns
@@ -802,9 +805,11 @@ __device__ __forceinline__ uint32_t rank_key6(float acc, int j) {
 // the lane itself, which ranks at most once and is dropped here; KEEP == 0
 // has its old partners' two smallest in told.  The `keep` smallest are
 // exactly the `keep` nearest unless the last of them and the next one share
-// all their distance bits, and then (about one wave in a hundred on
-// continuous data) the wave ranks its partners again by full (distance, id)
-// keys.  dist(j): the exact distance to partner j.
+// all their distance bits, and then the wave ranks its partners again by full
+// (distance, id) keys: about one wave in a hundred on continuous data, nearly
+// every one on rounded coordinates or repeated points (kNN graph of 200k x 20,
+// join_keep 4: 7.5 and 10.3 ms; 12.0 and 11.6 with u64 keys throughout).
+// dist(j): the exact distance to partner j.
 template <bool NEWNEW, int KEEP, int SLOTS, int RANK, typename F>
 __device__ __forceinline__ void join_choose(const uint32_t (&top)[RANK], const uint32_t (&told)[2], int nn, int nc,
                                             int keep, const uint32_t* s_cand, F dist, uint64_t (&top64)[SLOTS]) {
@@ -869,11 +874,14 @@ __device__ __forceinline__ void join_choose(const uint32_t (&top)[RANK], const u
 
 // FP32 join for d <= 31 other than 12 (d = 12 and 32 have k_nnd_join2): exact
 // distances, with the candidates' padded rows in LDS and the lane's own row
-// in registers (DP: d rounded up to a multiple of 4 or so; the zeros past d
-// add nothing to a distance).  As in k_nnd_join2 each old-new pair is
-// evaluated once (a distance has the same bits both ways) and passed to the
-// new lane through an LDS block.  Ranking uses 32-bit keys (rank_key6,
-// join_choose).  KEEP is 0, or the largest join_keep the kernel serves.
+// in registers (DP: 4, 8, 12, 16, 20, 24 or 32 columns; the zeros past d add
+// nothing to a distance, but d = 25 to 28 pay for 32: six launches at 200k and
+// join_keep 4 take 4.5 ms at d = 25, 3.9 with 28 columns).  As in k_nnd_join2
+// each old-new pair is evaluated once (a distance has the same bits both ways)
+// and passed to the new lane through an LDS block.  Ranking uses 32-bit keys
+// (rank_key6, join_choose).  KEEP is 0, or the largest join_keep the kernel
+// serves: 4 or 8, as the spare slots cost little (d = 20, join_keep 1: 2.74 ms,
+// 2.56 with a kernel of its own; from 3 on nothing).
 // Bound by VALU issue (two instructions per dimension and pair): six launches
 // at 200k points and join_keep 4 take 1.76 ms at d = 8, 2.56 at 16, 3.13 at
 // 20 and 4.98 at 31, where u64 keys and the lane's own row read from LDS took
@@ -1919,13 +1927,14 @@ static int check_params(hdb_ctx* ctx, const hdb_params& prm, int64_t n, int d) {
     return ctx->fail(HDB_EINVAL, "join_keep must be in [0,4] or 8");
   if (prm.distance_mode < 0 || prm.distance_mode > 2) return ctx->fail(HDB_EINVAL, "distance_mode must be 0, 1 or 2");
   if (prm.rerank_keep != 0 && prm.rerank_keep != 16) return ctx->fail(HDB_EINVAL, "rerank_keep must be 0 or 16");
+  // the joins take any d in chunks of columns; these limits are the tested range
   if (prm.distance_mode == 1 && d > 160) return ctx->fail(HDB_EUNSUPPORTED, "BF16 join built for d <= 160");
   if (prm.distance_mode == 2 && d > 128) return ctx->fail(HDB_EUNSUPPORTED, "BF16 refinement built for d <= 128");
   if (n < 2) return ctx->fail(HDB_EINVAL, "need at least 2 points");
   // reverse-pair positions (n x 32 of them) are int32
   if (n >= kMaxPoints) return ctx->fail(HDB_EINVAL, "n must be below 2^26 (67,108,864)");
   if (d < 1) return ctx->fail(HDB_EINVAL, "d must be >= 1");
-  if (d > 255) return ctx->fail(HDB_EUNSUPPORTED, "d above 255 (one LDS row per candidate)");
+  if (d > 255) return ctx->fail(HDB_EUNSUPPORTED, "the FP32 join is built for d <= 255");
   return HDB_OK;
 }
 

@@ -25,7 +25,6 @@ static int fill_t(hdb_ctx* ctx, T* p, int64_t n, T v) {
 }
 int fill_i32(hdb_ctx* ctx, int32_t* p, int64_t n, int32_t v) { return fill_t(ctx, p, n, v); }
 int fill_u64(hdb_ctx* ctx, uint64_t* p, int64_t n, uint64_t v) { return fill_t(ctx, p, n, v); }
-int fill_u8(hdb_ctx* ctx, uint8_t* p, int64_t n, uint8_t v) { return fill_t(ctx, p, n, v); }
 
 int read_i64(hdb_ctx* ctx, const int64_t* p, int64_t* out) {
   HDB_HIP(hipMemcpyAsync(out, p, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
@@ -783,9 +782,6 @@ static int radix_sort_t(hdb_ctx* ctx, K* keys, V* vals, int64_t n, int bit0, int
 
 int radix_sort_u32_u64(hdb_ctx* ctx, uint32_t* keys, uint64_t* vals, int64_t n, int bit0, int bit1) {
   return radix_sort_t<uint32_t, uint64_t, true>(ctx, keys, vals, n, bit0, bit1, nullptr, nullptr, nullptr);
-}
-int radix_sort_u32_u32(hdb_ctx* ctx, uint32_t* keys, uint32_t* vals, int64_t n, int bit0, int bit1) {
-  return radix_sort_t<uint32_t, uint32_t, true>(ctx, keys, vals, n, bit0, bit1, nullptr, nullptr, nullptr);
 }
 int radix_sort_u64_u32(hdb_ctx* ctx, uint64_t* keys, uint32_t* vals, int64_t n, int bit0, int bit1) {
   return radix_sort_t<uint64_t, uint32_t, true>(ctx, keys, vals, n, bit0, bit1, nullptr, nullptr, nullptr);

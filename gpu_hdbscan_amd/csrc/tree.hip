@@ -62,12 +62,16 @@ constexpr int kLkBits = 10;             // segments of 1024 edges are finished i
 constexpr int kLkEdges = 1 << kLkBits;  // one per thread of k_lk_local
 constexpr int32_t kNoName = INT_MAX;
 
-// Entries of the union-find only ever fall, from an element to one of its
-// ancestors, so a stale value (another XCD's L2 may hold a newer one) is
-// still an ancestor: finds use plain cached loads, and path halving, which
-// rewrites non-roots only, may race harmlessly with other finds and hooks.
-// Only the hook itself decides what is a root, with a compare-and-swap at
-// device scope.
+// The find is ECL-CC's (Jaiganesh and Burtscher 2018) with intermediate
+// pointer jumping.  What it relies on: every value an entry ever holds is one
+// of the element's ancestors, and smaller than the element unless it is a
+// root; a root changes only by the hook's compare-and-swap at device scope;
+// and an element, once hooked, is never a root again.  An entry may rise: a
+// path-halving store of an earlier read, or the write-back of another XCD's
+// L2, can replace a lower ancestor by a higher one, and a cached load can
+// return an old value.  Both still give an ancestor, so finds end, at a root
+// or at an element that was one; the swap tells which.  So finds use plain
+// cached loads and stores (kernels that follow see every hook).
 __device__ __forceinline__ int32_t uf_load(const int32_t* uf, int32_t x) {
   return __hip_atomic_load(uf + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
