@@ -391,7 +391,8 @@ def main():
             if tj.get("join_keep") == pb["keep"]:
                 traffic = tj.get("hbm_bytes_per_launch")
         # the join kernel the library dispatches for this leg
-        jk = "k_nnd_join_mfma" if dm else ("k_nnd_join2" if d in (12, 32) else "k_nnd_join")
+        jk = ("k_nnd_join_mfma" if dm else "k_nnd_join2" if d in (12, 32) else
+              "k_nnd_join_rows" if d < 32 else "k_nnd_join_wide")
         roof = {"kernel": jk, "bound": "hbm", "achieved": round(achieved, 1), "peak": PEAK_HBM_GBS,
                 "unit": "GB/s", "frac": round(achieved / PEAK_HBM_GBS, 4), "traffic": traffic,
                 "algorithmic_bytes_per_launch": int(join_bytes), "avg_launch_ms": round(per_launch_ms, 4),

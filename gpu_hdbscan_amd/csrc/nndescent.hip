@@ -544,8 +544,9 @@ __device__ __forceinline__ void join_quads(F f) {
 // again.  At D = 32 the kernel is bound by instruction issue: at 500k points
 // and KEEP = 3 a launch takes 1.17 ms instead of 1.63 (the block and the rows
 // in one buffer: five blocks on a CU, not four).  At D = 12 it is bound by the
-// gathers of the candidates' rows: 41M L2 misses a launch of 1M points, and
-// 1.44 ms with 738 vector instructions per wave as with 1034.
+// gathers of the candidates' rows, 42M L2 misses a launch of 1M points: with 744
+// vector instructions per wave instead of 1034 a launch takes 1.44 ms at 1M (1.37
+// before) and 13.5 at 10M (13.9).
 template <int D, bool NEWNEW, int KEEP>
 __global__ __launch_bounds__(kJoinWaves * 64, D <= 16 ? 8 : 5) void k_nnd_join2(const float* __restrict__ X, int64_t n, int d, int S,
                                                                NndBufs b) {
@@ -883,9 +884,9 @@ __device__ __forceinline__ void join_choose(const uint32_t (&top)[RANK], const u
 // serves: 4 or 8, as the spare slots cost little (d = 20, join_keep 1: 2.74 ms,
 // 2.56 with a kernel of its own; from 3 on nothing).
 // Bound by VALU issue (two instructions per dimension and pair): six launches
-// at 200k points and join_keep 4 take 1.76 ms at d = 8, 2.56 at 16, 3.13 at
-// 20 and 4.98 at 31, where u64 keys and the lane's own row read from LDS took
-// 3.47, 4.57, 5.96 and 11.15.
+// at 200k points and join_keep 4 take 1.62 ms at d = 8, 2.31 at 16, 2.78 at
+// 20 and 4.49 at 31, where u64 keys and the lane's own row read from LDS took
+// 3.27, 4.19, 5.67 and 10.94.
 template <int DP, bool NEWNEW, int KEEP>
 __global__ __launch_bounds__(kJoinWaves * 64) void k_nnd_join_rows(int64_t n, int d, int S, int keep, NndBufs b) {
   constexpr int WPB = kJoinWaves;
@@ -1015,9 +1016,9 @@ __global__ __launch_bounds__(kJoinWaves * 64) void k_nnd_join_rows(int64_t n, in
 // the distances have the bits of the other forms.  The distances then go to
 // LDS in place of the rows (entry (j, lane) at 65 j + lane), where the new
 // lanes also find theirs to the old candidates.  Bound by VALU issue, two
-// instructions per dimension and pair: six launches at join_keep 4 take 5.8 ms
-// at 200k x 40, 7.0 at 200k x 64 and 6.0 at 100k x 128, where the lane's own row
-// read from LDS and u64 keys took 11.6, 19.7 and 30.4.
+// instructions per dimension and pair: six launches at join_keep 4 take 5.5 ms
+// at 200k x 40, 6.7 at 200k x 64 and 5.7 at 100k x 128, where the lane's own row
+// read from LDS and u64 keys took 11.5, 19.6 and 29.9.
 template <bool NEWNEW, int KEEP>
 __global__ __launch_bounds__(kJoinWaves * 64, 4) void k_nnd_join_wide(const float* __restrict__ X, int64_t n, int d,
                                                                    int S, int keep, NndBufs b) {
@@ -1160,8 +1161,8 @@ __global__ __launch_bounds__(kJoinWaves * 64, 4) void k_nnd_join_wide(const floa
 // chunk to the distances of its whole shortlist: reading them again (from a
 // cache, mostly) keeps the LDS of a wave at 10 KB and its chains in parallel,
 // where holding 64 whole FP32 rows left four waves to a CU, each ranking one
-// partner after the other.  A launch at 100k x 128 and join_keep 4 takes 0.85
-// ms (2.25 in that form; 0.99 with the next chunk's columns in registers of
+// partner after the other.  A launch at 100k x 128 and join_keep 4 takes 0.77
+// ms (2.19 in that form; 0.99 with the next chunk's columns in registers of
 // their own, which spill).
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
